@@ -87,9 +87,9 @@ def draw(rng):
     path = rng.choice(("step", "step", "captured", "loop", "seven", "view", "view", "bin",
                        "ssim", "adam"))
     scene = rng.choice(("box", "ball", "cluster"))
-    n = _log(rng, 5_000, 150_000 if scene == "box" else 1_500_000)
+    n = _log(rng, 5_000, 120_000 if scene == "box" else 1_000_000)
     width = _log(rng, 200, 2560)
-    height = max(150, int(width * rng.uniform(0.5, 1.0)))
+    height = min(max(150, int(width * rng.uniform(0.5, 1.0))), 4_200_000 // width)
     if path == "ssim":
         return _case(None, path, batch=rng.randint(1, 2), width=width, height=height,
                      hwc=rng.random() < 0.5, padding=rng.choice(("same", "valid")))
