@@ -29,10 +29,11 @@
 // The backward walks the list in the same front-to-back order.  With
 // S_i = sum_{k>i} w_k (g.c_k) = g.C - sum_{k<=i} w_k (g.c_k), where C is the
 // pixel's forward colour, dL/dalpha_i = T_i (g.c_i) - S_i / (1 - alpha_i + eps).
-// A lane sums its four pixels' contributions in registers, the wave reduces the
-// nine fields with DPP row butterflies plus two permlane swaps, and lane 0
-// issues one float atomic per (tile, Gaussian, field) (the reference issues one
-// per pixel: src/cuda/kernel.cu:1098-1106).
+// A lane sums its four pixels' contributions in registers and puts six sums per
+// entry aside in LDS; every four entries the wave reduces them together, a row of
+// 16 lanes each (backward_flush), and nine lanes of each row issue one float
+// atomic per (tile, Gaussian, field) (the reference issues one per pixel:
+// src/cuda/kernel.cu:1098-1106), into one row of nine floats per Gaussian.
 
 #include "wave_ops.h"
 
@@ -194,6 +195,18 @@ struct BatchLds {
     int wave_flag[W];         // W > 1: per-wave votes of the batch loops (tile_any)
     int wave_flag_once[W];    // W > 1: the backward's one vote before its loop
     uint32_t wave_work[W];    // W > 1: each wave's work so far, summed at a checkpoint
+};
+
+// Entries whose lane sums wait in LDS for one reduction (backward_flush): per
+// slot three planes of 64 float2, padded by 32 banks so that the reduction's four
+// 16-lane rows, each reading its own slot, meet different banks.
+constexpr int kPend = 4;
+constexpr int kPendStride = 3 * kWave + 16;  // float2 per slot
+
+template <int W>
+struct BackwardLds {
+    BatchLds<W> batch;
+    float2 pend[W][(kPend - 1) * kPendStride + 3 * kWave];
 };
 
 // Records whose log2 opacity is not finite -- opacity <= 0, +inf or NaN -- are
@@ -364,37 +377,24 @@ __device__ __forceinline__ Staged stage_records(BatchLds<W> &s, const Record &r,
         s.aux[slot] = make_float4(r.C, chi_eff, __uint_as_float(m), log2o);
         s.col[slot] = make_float4(r.r, r.g, r.b, __int_as_float(r.id));
         const bool special = special_opacity(log2o);
-        if (kInvO) s.inv_o[slot] = special ? 1.0f : __builtin_amdgcn_rcpf(r.o);
+        if (kInvO) s.inv_o[slot] = special ? 0.0f : __builtin_amdgcn_rcpf(r.o);
         if (special) s.o_raw[slot] = r.o;
     }
     return st;
 }
 
-// Software pipeline over a tile's list in batches of kBatch.  With kRecords,
-// the ids of batch b+2 and the records of batch b+1 are in flight while batch
-// b is processed; without, only the ids of batch b+1 (fewer registers).  The
-// backward uses kRecords (2% faster although it costs a wave per SIMD at 93
-// VGPRs); the forward does not (4% faster without).
+// Software pipeline over a tile's list in batches of kBatch: the ids of batch
+// b + 1 are in flight while batch b is processed.  Fetching its records ahead as
+// well costs registers and gains nothing: the forward is 4% slower with it, the
+// backward unchanged (178.9 against 178.2 us at 1M Gaussians, 1920x1080).
 // kInvO: also stage 1 / opacity (the backward).  W waves stage W * kBatch
 // records per batch, one per thread.
-template <bool kRecords, bool kInvO, int W = 1>
+template <bool kInvO, int W = 1>
 struct BatchPipe {
-    int32_t next_id;  // this thread's id in the batch after the next one to stage
-    Record rec;       // this thread's record of the next batch to stage (kRecords)
+    int32_t next_id;  // this thread's id in the next batch to stage
 
-    __device__ __forceinline__ void start(TileSpan span, const int32_t *__restrict__ ids,
-                                          int64_t n, const float *__restrict__ points,
-                                          const float *__restrict__ conics,
-                                          const float *__restrict__ opac,
-                                          const float *__restrict__ colors) {
-        const int32_t lane = (int32_t)threadIdx.x;
-        if (kRecords) {
-            const int32_t g0 = fetch_id(span.start + lane, span.end, ids);
-            next_id = fetch_id(span.start + kBatch * W + lane, span.end, ids);
-            rec = fetch_record(g0, n, points, conics, opac, colors);
-        } else {
-            next_id = fetch_id(span.start + lane, span.end, ids);
-        }
+    __device__ __forceinline__ void start(TileSpan span, const int32_t *__restrict__ ids) {
+        next_id = fetch_id(span.start + (int32_t)threadIdx.x, span.end, ids);
     }
 
     // Stages the batch starting at b0 (only records reaching the tile) and
@@ -406,19 +406,13 @@ struct BatchPipe {
                                            const float *__restrict__ opac,
                                            const float *__restrict__ colors, float chi,
                                            float alpha_thr, float x0, float y0) {
-        const int32_t lane = (int32_t)threadIdx.x;
-        if (!kRecords) rec = fetch_record(next_id, n, points, conics, opac, colors);
+        const Record rec = fetch_record(next_id, n, points, conics, opac, colors);
         __syncthreads();  // previous batch fully read before restaging
         const Staged st =
             stage_records<kInvO, W>(s, rec, chi, alpha_thr, __builtin_amdgcn_logf(alpha_thr), x0,
                                     y0);
         __syncthreads();
-        if (kRecords) {
-            rec = fetch_record(next_id, n, points, conics, opac, colors);
-            next_id = fetch_id(b0 + 2 * kBatch * W + lane, span.end, ids);
-        } else {
-            next_id = fetch_id(b0 + kBatch * W + lane, span.end, ids);
-        }
+        next_id = fetch_id(b0 + kBatch * W + (int32_t)threadIdx.x, span.end, ids);
         return st;
     }
 };
@@ -652,8 +646,8 @@ __device__ __forceinline__ void blend_accumulate(
     }
     if (n_ck) *n_ck = 0;
     if (span.end <= span.start) return;
-    BatchPipe<false, false, W> pipe;
-    pipe.start(span, ids, n, points, conics, opac, colors);
+    BatchPipe<false, W> pipe;
+    pipe.start(span, ids);
     const bool counter = W == 1 || tile_wave() == 0;
     int batch = 0, saved = 0;
     for (int32_t b0 = span.start; b0 < span.end; b0 += kBatch * W, ++batch) {
@@ -693,7 +687,6 @@ constexpr int kDppXor1 = 0xB1;        // quad_perm [1,0,3,2]
 constexpr int kDppXor2 = 0x4E;        // quad_perm [2,3,0,1]
 constexpr int kDppHalfMirror = 0x141; // reverse each 8-lane half row
 constexpr int kDppMirror = 0x140;     // reverse each 16-lane row
-constexpr int kDppRor8 = 0x128;       // rotate each row by 8 lanes
 
 // a + b where the two 32-lane halves are exchanged between them first:
 // lanes 0-31 get a[l] + a[l+32], lanes 32-63 get b[l-32] + b[l].
@@ -720,48 +713,41 @@ __device__ __forceinline__ float wave_sum(float x) {
     return swap32_add(x, x);
 }
 
-// Lane that holds field f's wave total after wave_sum9 (the others hold partials):
-// f0 0, f1 32, f2 16, f3 48, f4 8, f5 40, f6 24, f7 56, f8 4.
-__device__ __forceinline__ int sum9_field_of_lane(int lane) {
-    switch (lane) {
-    case 0: return 0;
-    case 32: return 1;
-    case 16: return 2;
-    case 48: return 3;
-    case 8: return 4;
-    case 40: return 5;
-    case 24: return 6;
-    case 56: return 7;
-    case 4: return 8;
-    default: return -1;
-    }
-}
-
-// Wave sums of nine per-lane values by transposition: each exchange step halves
-// the lanes a field is spread over and doubles the fields a register holds, so
-// the nine sums cost 9 swaps/selects and 14 adds instead of nine full
-// reductions.  All 64 lanes must be active.
-__device__ __forceinline__ float wave_sum9(const float (&f)[kGradFields], bool hi8,
-                                           bool f8_lane) {
-    const float p0 = swap32_add(f[0], f[1]);  // halves: f0 | f1
-    const float p1 = swap32_add(f[2], f[3]);  // f2 | f3
-    const float p2 = swap32_add(f[4], f[5]);  // f4 | f5
-    const float p3 = swap32_add(f[6], f[7]);  // f6 | f7
-    const float p4 = swap32_add(f[8], 0.0f);  // f8 | 0
-    const float q0 = swap16_add(p0, p1);      // rows: f0 f2 f1 f3
-    const float q1 = swap16_add(p2, p3);      // rows: f4 f6 f5 f7
-    float q2 = swap16_add(p4, 0.0f);          // rows: f8 0 0 0
-    // low 8 lanes of each row take q0's row field, high 8 lanes q1's
-    const float x = hi8 ? q1 : q0, y = hi8 ? q0 : q1;
-    float r = x + GS_DPP(y, kDppRor8);
-    r += GS_DPP(r, kDppXor1);
-    r += GS_DPP(r, kDppXor2);
-    r += GS_DPP(r, kDppHalfMirror);
-    q2 += GS_DPP(q2, kDppXor1);
-    q2 += GS_DPP(q2, kDppXor2);
-    q2 += GS_DPP(q2, kDppHalfMirror);
-    q2 += GS_DPP(q2, kDppMirror);
-    return f8_lane ? q2 : r;
+// Sums of nine per-lane values over each row of 16 lanes, by transposition: the
+// first two steps fold lane l with l + 8 and the halves of 8 lanes, each keeping
+// one field in the low and another in the high lanes (the masked DPP adds write
+// only their banks of 4 lanes); two butterflies within the quads finish.  22 DPP
+// adds for nine sums in four rows at once.  Bank b of q0 holds field (0, 2, 1, 3)[b],
+// of q1 field (4, 6, 5, 7)[b], every lane of q2 field 8.  All lanes must be active.
+// One asm block: every DPP source is written at least two instructions before it
+// is read (the leading s_nop covers the inputs).
+__device__ __forceinline__ void row_sum9(const float (&f)[kGradFields], float &q0, float &q1,
+                                         float &q2) {
+    float p0, p1, p2, p3;
+    asm("s_nop 1\n\t"
+        "v_add_f32_dpp %3, %7, %7 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %4, %9, %9 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %5, %11, %11 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %6, %13, %13 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %2, %15, %15 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %3, %8, %8 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %4, %10, %10 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %5, %12, %12 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %6, %14, %14 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %0, %3, %3 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %1, %5, %5 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %2, %2, %2 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %0, %4, %4 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %1, %6, %6 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %2, %2, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %1, %1, %1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %2, %2, %2 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %1, %1, %1 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf"
+        : "=&v"(q0), "=&v"(q1), "=&v"(q2), "=&v"(p0), "=&v"(p1), "=&v"(p2), "=&v"(p3)
+        : "v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(f[4]), "v"(f[5]), "v"(f[6]), "v"(f[7]),
+          "v"(f[8]));
 }
 
 // One tile per workgroup of W waves (64 W threads).  Held to 64 VGPRs (8 waves
@@ -857,8 +843,27 @@ void blend_forward_kernel(
     }
 }
 
-// Destination of the lane's field after wave_sum9:
-// out[stride * g] += value * (inv_o ? 1 / o : fa).  stride4 = 4 * stride (bytes).
+// Where the backward adds its gradients: field f of Gaussian g of each output at
+// base[stride * g + f].  Four arrays of their own (strides 2, 3, 1, 3), or one row
+// of nine floats per Gaussian (grad_rows): the nine atomics of an entry then fall
+// into one or two 64-byte lines instead of four.  They are executed at the memory
+// side, a line at a time, and their number bounded the kernel: backward at 1M
+// Gaussians, 1920x1080 244 -> 179 us, 2M at 3840x2160 735 -> 585 us, 200k at
+// 1280x720 141 -> 116 us (no atomics at all: 178, 577 and 116 us).
+struct GradOut {
+    float *points, *conics, *opac, *colors;
+    int s_points, s_conics, s_opac, s_colors;
+};
+inline GradOut grad_arrays(float *points, float *conics, float *opac, float *colors) {
+    return {points, conics, opac, colors, 2, 3, 1, 3};
+}
+inline GradOut grad_rows(float *rows) {
+    return {rows, rows + 2, rows + 5, rows + 6, kGradFields, kGradFields, kGradFields, kGradFields};
+}
+
+// Destination of the lane's field after row_sum9 (lane % 16 alone decides: the
+// four rows hold four entries): out[stride * g] += value * (inv_o ? 1 / o : fa).
+// stride4 = 4 * stride (bytes).  The lane's value is q0, q1 or q2 by lane % 4.
 struct GradTarget {
     float *base;
     uint32_t stride4;
@@ -867,26 +872,27 @@ struct GradTarget {
     bool active;
 };
 
-__device__ __forceinline__ GradTarget grad_target(int lane, float *g_points, float *g_conics,
-                                                  float *g_opac, float *g_colors) {
+__device__ __forceinline__ GradTarget grad_target(int lane, const GradOut &out) {
     GradTarget t;
-    const int f = sum9_field_of_lane(lane);
-    t.active = f >= 0;
-    t.base = g_points;
-    int stride = 2;
+    const int bank = (lane >> 2) & 3, i = lane & 3;
+    // bank b: q0 field (0, 2, 1, 3)[b], q1 field (4, 6, 5, 7)[b]
+    const int swapped = (bank & 1) * 2 + (bank >> 1);
+    const int f = i == 0 ? swapped : (i == 1 ? 4 + swapped : 8);
+    t.active = i < 2 || (i == 2 && bank == 0);
+    t.base = out.points;
+    int stride = out.s_points;
     t.fa = 1.0f;
     t.inv_o = false;
     switch (f) {
-    case 0: t.base = g_points; break;
-    case 1: t.base = g_points + 1; break;
-    case 2: t.base = g_conics; stride = 3; t.fa = -0.5f; break;
-    case 3: t.base = g_conics + 1; stride = 3; t.fa = -1.0f; break;
-    case 4: t.base = g_conics + 2; stride = 3; t.fa = -0.5f; break;
-    case 5: t.base = g_opac; stride = 1; t.inv_o = true; break;
-    case 6: t.base = g_colors; stride = 3; break;
-    case 7: t.base = g_colors + 1; stride = 3; break;
-    case 8: t.base = g_colors + 2; stride = 3; break;
-    default: break;
+    case 0: break;
+    case 1: t.base = out.points + 1; break;
+    case 2: t.base = out.conics; stride = out.s_conics; t.fa = -0.5f; break;
+    case 3: t.base = out.conics + 1; stride = out.s_conics; t.fa = -1.0f; break;
+    case 4: t.base = out.conics + 2; stride = out.s_conics; t.fa = -0.5f; break;
+    case 5: t.base = out.opac; stride = out.s_opac; t.inv_o = true; break;
+    case 6: t.base = out.colors; stride = out.s_colors; break;
+    case 7: t.base = out.colors + 1; stride = out.s_colors; break;
+    default: t.base = out.colors + 2; stride = out.s_colors; break;
     }
     t.stride4 = 4u * (uint32_t)stride;
     return t;
@@ -894,54 +900,194 @@ __device__ __forceinline__ GradTarget grad_target(int lane, float *g_points, flo
 
 // Per-lane state of the backward walk: transmittance and the running sum
 // acc = sum_{k<=i} w_k (g.c_k) - g.C of the lane's four pixels (minus the
-// remaining colour gradient S_i, starting at -g.C), their colour gradients g
-// and gC = g.C.
+// remaining colour gradient S_i, starting at -g.C) and their colour gradients g.
 template <int S>
 struct BackwardLane {
     float T[S], acc[S];
-    float gr[S], gg[S], gb[S], gC[S];
+    float gr[S], gg[S], gb[S];
 };
 
-// One staged entry j: per-strip gradient terms summed over the lane's pixels,
-// then the nine-field wave sum and one atomic per field (lanes of tgt).  With
-// W waves per tile each wave sums and adds its own S strips' share.
-template <bool kSafe, int W>
-__device__ __forceinline__ void backward_entry(const BatchLds<W> &s, int j,
-                                               const LanePixels<kStrips / W> &pix,
-                                               float alpha_thr, float T_thr, float chi,
-                                               BackwardLane<kStrips / W> &L,
-                                               const GradTarget &tgt, bool hi8, bool f8_lane) {
-    constexpr int S = kStrips / W;
-    const float4 aux = s.aux[j];
-    uint32_t smask = __builtin_amdgcn_readfirstlane(__float_as_uint(aux.z));
-    if constexpr (W > 1) {
-        smask = (smask >> (tile_wave() * S)) & ((1u << S) - 1u);
-        if (smask == 0u) return;  // uniform: none of this wave's strips
+// Entries of the batch whose lane sums wait in LDS: slot p holds staged record
+// (js >> 8 p) & 255 (uniform).
+struct Pending {
+    int n;
+    uint32_t js;
+};
+
+// The order of a wave's own LDS accesses, for the compiler (the hardware keeps it).
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Puts an entry's six lane sums aside.
+template <int W>
+__device__ __forceinline__ void backward_pend(BackwardLds<W> &s, Pending &pd, int j, float sH,
+                                              float s1, float s2, float sr, float sg, float sb) {
+    float2 *p = s.pend[W == 1 ? 0 : tile_wave()] + pd.n * kPendStride + threadIdx.x % kWave;
+    p[0] = make_float2(sH, s1);
+    p[kWave] = make_float2(s2, sr);
+    p[2 * kWave] = make_float2(sg, sb);
+    pd.js |= (uint32_t)j << (8 * pd.n);
+    ++pd.n;
+}
+
+// Sums of up to kPend pending entries over the wave and their atomics: row e of
+// 16 lanes takes slot e.  Lane x of the row adds the four 16-lane groups' sums of
+// tile column x (which share du), forms the nine fields and the row sums them
+// (row_sum9), so one pass of 60 vector instructions serves four entries; reducing
+// each entry by itself took about 50 (five permlane32 and three permlane16 swaps
+// of 8 cycles, 9 DPP adds, two 64-bit address multiply-adds).  Every lane must be
+// active; slots past pd.n hold stale sums, whose rows add nothing.
+template <int W>
+__device__ __forceinline__ void backward_flush(const BackwardLds<W> &s, Pending &pd, float fx,
+                                               const GradTarget &tgt) {
+    wave_lds_fence();
+    const int lane = threadIdx.x % kWave, e = lane >> 4;
+    const uint32_t j = (pd.js >> (8 * e)) & 255u;  // < kBatch * W, also for a stale slot
+    const float4 geo = s.batch.geo[j];
+    const float C = s.batch.aux[j].x;
+    const uint32_t g = __float_as_uint(s.batch.col[j].w);
+    const float inv_o = s.batch.inv_o[j];
+    const float2 *p = s.pend[W == 1 ? 0 : tile_wave()] + e * kPendStride + (lane & 15);
+    float2 a = p[0], b = p[kWave], c = p[2 * kWave];
+#pragma unroll
+    for (int r = 16; r < kWave; r += 16) {
+        const float2 x = p[r], y = p[kWave + r], z = p[2 * kWave + r];
+        a.x += x.x;
+        a.y += x.y;
+        b.x += y.x;
+        b.y += y.y;
+        c.x += z.x;
+        c.y += z.y;
     }
-    const float4 geo = s.geo[j];
-    // uniform: a record with a non-finite log2 opacity (only in the select-based
-    // path); its opacity gradient is summed as G dalpha (its staged 1 / o is 1)
-    const bool special =
-        kSafe && special_opacity(__uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(aux.w))));
-    const float o_sp = special ? s.o_raw[j] : 0.0f;
-    float sGd = -0.0f;
-    const float4 col = s.col[j];
+    const float sH = a.x, s1 = a.y;
+    const float du = fx - geo.x;
+    const float B = 0.5f * geo.w;
+    const float ad = du * sH;
+    float f[kGradFields];
+    f[0] = fmaf(geo.z, ad, B * s1);  // d/du
+    f[1] = fmaf(B, ad, C * s1);      // d/dv
+    f[2] = du * ad;                  // d/dA / (-1/2)
+    f[3] = du * s1;                  // d/dB / (-1)
+    f[4] = b.x;                      // d/dC / (-1/2)
+    f[5] = sH;                       // d/dopacity * o
+    f[6] = b.y;
+    f[7] = c.x;
+    f[8] = c.y;
+    float q0, q1, q2;
+    row_sum9(f, q0, q1, q2);
+    const float total = (lane & 3) == 0 ? q0 : ((lane & 3) == 1 ? q1 : q2);
+    const float scale = tgt.inv_o ? inv_o : tgt.fa;
+    // a record with a special opacity stages 0 for 1 / o: its opacity gradient was
+    // added by the entry itself (backward_entry_safe)
+    if (tgt.active && e < pd.n && scale != 0.0f) {
+        const uint64_t off = (uint64_t)g * (uint64_t)tgt.stride4;
+        unsafeAtomicAdd(reinterpret_cast<float *>(reinterpret_cast<char *>(tgt.base) + off),
+                        total * scale);
+    }
+    wave_lds_fence();
+    pd.n = 0;
+    pd.js = 0;
+}
+
+// The batch's entry j applied to the lane's pixels: their gradient terms summed
+// over the lane's strips and put aside for backward_flush.  act[q]: lanes whose
+// pixel in strip q still composites (T >= T_thr; kept in scalar registers, so
+// the test costs no vector instruction).
+//   w = alpha T, T' = T - w, acc += w (g.c)   (acc = -S_i)
+//   h = alpha dL/dalpha = w (g.c + acc / T')
+// since dL/dalpha = T (g.c) - S_i / (1 - alpha) and T' = T (1 - alpha): the
+// quotient is the mean of g.c over what lies behind, so the form needs neither
+// 1 - alpha nor its reciprocal's epsilon.  Once T' < T_thr nothing behind the
+// entry is composited and S_i is 0 exactly (acc holds only its rounding), so the
+// quotient is dropped there.  Needs T_thr >= kMinFastT (a finite 1 / T') and
+// finite gradients and records; backward_entry_safe serves the rest.
+constexpr float kMinFastT = 1e-30f;
+
+template <int W>
+__device__ __forceinline__ void backward_entry(BackwardLds<W> &s, int j,
+                                               const LanePixels<kStrips / W> &pix, float T_thr,
+                                               BackwardLane<kStrips / W> &L,
+                                               uint64_t (&act)[kStrips / W], Pending &pd) {
+    constexpr int S = kStrips / W;
+    const float4 aux = s.batch.aux[j];
+    const float4 geo = s.batch.geo[j];
+    const float4 col = s.batch.col[j];
     const float du = pix.fx - geo.x;
     const float Adudu = (geo.z * du) * du;
     const float B2du = geo.w * du;
-    // the alpha test as a cut-off on E, staged in aux.y: alpha = o exp(-E/2) >=
-    // alpha_thr iff E <= 2 ln(o / alpha_thr) (up to the rounding of the hardware
-    // exp2/log2)
-    const float chi_a = aux.y;
+    float dv[S], E[S];
+    uint64_t inc[S], any = 0;
+#pragma unroll
+    for (int q = 0; q < S; ++q) {
+        dv[q] = pix.fy[q] - geo.y;
+        E[q] = fmaf(fmaf(aux.x, dv[q], B2du), dv[q], Adudu);
+        // chi-square and alpha test as one cut-off on E (staged in aux.y)
+        inc[q] = __ballot(E[q] < aux.y) & act[q];
+        any |= inc[q];
+    }
+    if (any == 0) return;
     // -0 is the identity of float addition, so the first strip's sums need no add
     float sH = -0.0f, s1 = -0.0f, s2 = -0.0f, sr = -0.0f, sg = -0.0f, sb = -0.0f;
-    bool hit = false;  // some strip was evaluated (otherwise every field is -0)
+#pragma unroll
+    for (int q = 0; q < S; ++q) {
+        if (inc[q] == 0) continue;  // uniform
+        const float alpha = alpha_of(E[q], aux.w);
+        const float a = __builtin_amdgcn_inverse_ballot_w64(inc[q]) ? alpha : 0.0f;
+        const float w = a * L.T[q];
+        const float gcol = fmaf(L.gr[q], col.x, fmaf(L.gg[q], col.y, L.gb[q] * col.z));
+        const float acc = fmaf(w, gcol, L.acc[q]);
+        const float T = L.T[q] - w;
+        act[q] = __ballot(!(T < T_thr));
+        const float behind =
+            __builtin_amdgcn_inverse_ballot_w64(act[q]) ? __builtin_amdgcn_rcpf(T) : 0.0f;
+        const float h = w * fmaf(acc, behind, gcol);
+        sH += h;
+        const float t = h * dv[q];
+        s1 += t;
+        s2 = fmaf(t, dv[q], s2);
+        sr = fmaf(w, L.gr[q], sr);
+        sg = fmaf(w, L.gg[q], sg);
+        sb = fmaf(w, L.gb[q], sb);
+        L.acc[q] = acc;
+        L.T[q] = T;
+    }
+    backward_pend<W>(s, pd, j, sH, s1, s2, sr, sg, sb);
+}
+
+// The same for any input: a non-finite gradient, image value, colour or opacity
+// (selects in place of zero weights, where 0 * inf would not be 0) and any
+// threshold (dL/dalpha from 1 - alpha + 1e-10, as the reference).
+template <int W>
+__device__ __forceinline__ void backward_entry_safe(BackwardLds<W> &s, int j,
+                                                    const LanePixels<kStrips / W> &pix,
+                                                    float alpha_thr, float T_thr,
+                                                    BackwardLane<kStrips / W> &L, Pending &pd,
+                                                    const GradOut &out) {
+    constexpr int S = kStrips / W;
+    const float4 aux = s.batch.aux[j];
+    uint32_t smask = __builtin_amdgcn_readfirstlane(__float_as_uint(aux.z));
+    if constexpr (W > 1) smask = (smask >> (tile_wave() * S)) & ((1u << S) - 1u);
+    if (smask == 0u) return;  // uniform: none of this wave's strips
+    const float4 geo = s.batch.geo[j];
+    const float4 col = s.batch.col[j];
+    // uniform: a record with a non-finite log2 opacity; its opacity gradient is
+    // summed as G dalpha
+    const bool special = special_opacity(
+        __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(aux.w))));
+    const float o_sp = special ? s.batch.o_raw[j] : 0.0f;
+    const float du = pix.fx - geo.x;
+    const float Adudu = (geo.z * du) * du;
+    const float B2du = geo.w * du;
+    float sH = -0.0f, s1 = -0.0f, s2 = -0.0f, sr = -0.0f, sg = -0.0f, sb = -0.0f, sGd = -0.0f;
+    bool hit = false;  // some strip was evaluated
 #pragma unroll
     for (int q = 0; q < S; ++q) {
         if (!((smask >> q) & 1u)) continue;  // uniform
         const float dv = pix.fy[q] - geo.y;
         const float E = fmaf(fmaf(aux.x, dv, B2du), dv, Adudu);
-        bool inc = !(L.T[q] < T_thr) && (E < chi_a);
+        bool inc = !(L.T[q] < T_thr) && (E < aux.y);
         float alpha = 0.0f, G = 0.0f;
         if (special) {  // alpha = o G from the raw opacity, alpha test on its value
             G = __builtin_amdgcn_exp2f(E * kNegHalfLog2e);
@@ -951,15 +1097,14 @@ __device__ __forceinline__ void backward_entry(const BatchLds<W> &s, int j,
         if (!wave_any(inc)) continue;
         hit = true;
         if (!special) alpha = alpha_of(E, aux.w);
-        const float a = kSafe ? alpha : (inc ? alpha : 0.0f);
-        const float w = a * L.T[q];
+        const float w = alpha * L.T[q];
         const float gcol = fmaf(L.gr[q], col.x, fmaf(L.gg[q], col.y, L.gb[q] * col.z));
-        const float acc_new = fmaf(w, gcol, L.acc[q]);  // -S_i
-        const float one_m = (1.0f - a) + kTransmittanceEps;
+        const float acc = fmaf(w, gcol, L.acc[q]);  // -S_i
+        const float one_m = (1.0f - alpha) + kTransmittanceEps;
         // dalpha = T gcol - S_i / (1 - alpha + eps)
-        const float dalpha = fmaf(acc_new, __builtin_amdgcn_rcpf(one_m), L.T[q] * gcol);
-        const float h = kSafe ? (inc ? a * dalpha : 0.0f) : a * dalpha;
-        const float ws = kSafe ? (inc ? w : 0.0f) : w;
+        const float dalpha = fmaf(acc, __builtin_amdgcn_rcpf(one_m), L.T[q] * gcol);
+        const float h = inc ? alpha * dalpha : 0.0f;
+        const float ws = inc ? w : 0.0f;
         if (special) sGd += inc ? G * dalpha : 0.0f;
         sH += h;
         const float t = h * dv;
@@ -968,46 +1113,46 @@ __device__ __forceinline__ void backward_entry(const BatchLds<W> &s, int j,
         sr = fmaf(ws, L.gr[q], sr);
         sg = fmaf(ws, L.gg[q], sg);
         sb = fmaf(ws, L.gb[q], sb);
-        L.acc[q] = kSafe ? (inc ? acc_new : L.acc[q]) : acc_new;
-        L.T[q] = kSafe ? (inc ? L.T[q] - w : L.T[q]) : L.T[q] - w;
+        L.acc[q] = inc ? acc : L.acc[q];
+        L.T[q] = inc ? L.T[q] - w : L.T[q];
     }
-    if (hit) {
-        const float B = 0.5f * geo.w;
-        const float ad = du * sH;
-        float f[kGradFields];
-        f[0] = fmaf(geo.z, ad, B * s1);  // d/du
-        f[1] = fmaf(B, ad, aux.x * s1);  // d/dv
-        f[2] = du * ad;                  // d/dA / (-1/2)
-        f[3] = du * s1;                  // d/dB / (-1)
-        f[4] = s2;                       // d/dC / (-1/2)
-        f[5] = special ? sGd : sH;       // d/dopacity * o (special: d/dopacity)
-        f[6] = sr;
-        f[7] = sg;
-        f[8] = sb;
-        const float total = wave_sum9(f, hi8, f8_lane);
-        // the entry's Gaussian id is uniform (a non-negative int32): one unsigned
-        // 32 x 32 -> 64 multiply-add per field address
-        const uint32_t g = __builtin_amdgcn_readfirstlane(__float_as_uint(col.w));
-        if (tgt.active) {
-            const float scale = tgt.inv_o ? s.inv_o[j] : tgt.fa;
-            const uint64_t off = (uint64_t)g * (uint64_t)tgt.stride4;
-            unsafeAtomicAdd(reinterpret_cast<float *>(reinterpret_cast<char *>(tgt.base) + off),
-                            total * scale);
+    if (!hit) return;
+    if (special) {
+        const float total = wave_sum(sGd);
+        if (threadIdx.x % kWave == 0) {
+            const uint32_t g = __float_as_uint(col.w);
+            unsafeAtomicAdd(out.opac + (uint64_t)g * (uint64_t)(uint32_t)out.s_opac, total);
         }
     }
+    backward_pend<W>(s, pd, j, sH, s1, s2, sr, sg, sb);
 }
 
 template <bool kSafe, int W>
-__device__ __forceinline__ void backward_batch(const BatchLds<W> &s, int cnt,
+__device__ __forceinline__ void backward_batch(BackwardLds<W> &s, int cnt,
                                                const LanePixels<kStrips / W> &pix,
-                                               float alpha_thr, float T_thr, float chi,
+                                               float alpha_thr, float T_thr,
                                                BackwardLane<kStrips / W> &L,
-                                               const GradTarget &tgt, bool hi8, bool f8_lane) {
+                                               const GradTarget &tgt, const GradOut &out) {
+    constexpr int S = kStrips / W;
     if (W > 1 && !any_active(L.T, T_thr)) return;  // this wave's pixels are done
+    Pending pd{0, 0u};
+    uint64_t act[S];
+#pragma unroll
+    for (int q = 0; q < S; ++q) act[q] = __ballot(!(L.T[q] < T_thr));
     for (int j = 0; j < cnt; ++j) {
-        backward_entry<kSafe, W>(s, j, pix, alpha_thr, T_thr, chi, L, tgt, hi8, f8_lane);
-        if ((j & 7) == 7 && !any_active(L.T, T_thr)) break;
+        if (kSafe) {
+            backward_entry_safe<W>(s, j, pix, alpha_thr, T_thr, L, pd, out);
+            if ((j & 7) == 7 && !any_active(L.T, T_thr)) break;
+        } else {
+            backward_entry<W>(s, j, pix, T_thr, L, act, pd);
+            uint64_t left = 0;
+#pragma unroll
+            for (int q = 0; q < S; ++q) left |= act[q];
+            if (left == 0) break;
+        }
+        if (pd.n == kPend) backward_flush<W>(s, pd, pix.fx, tgt);
     }
+    if (pd.n > 0) backward_flush<W>(s, pd, pix.fx, tgt);
 }
 
 // Backward of the front-to-back blend, walking the list in the same order.
@@ -1035,16 +1180,14 @@ enum { kSeedImage = 0, kSeedDisplay = 1, kSeedL1 = 2 };
         int64_t k, int64_t n, const float *__restrict__ points,                               \
         const float *__restrict__ conics, const float *__restrict__ opac,                     \
         const float *__restrict__ colors, int tiles_x, int width, int height, float alpha_thr, \
-        float T_thr_in, float chi, float *__restrict__ g_points, float *__restrict__ g_conics, \
-        float *__restrict__ g_opac, float *__restrict__ g_colors,                             \
-        const float *__restrict__ grad_loss, float inv_count, const float *__restrict__ extra
+        float T_thr_in, float chi, GradOut out, const float *__restrict__ grad_loss, float inv_count, const float *__restrict__ extra
 
 // The backward walk of `tile`'s list, or (seg >= 0) of its segment seg: from the
 // start to checkpoint 0, between checkpoints seg - 1 and seg, or from the last
 // checkpoint to the end.  Every thread of the workgroup calls it with the same
 // tile and segment (it contains barriers).
 template <int kSeed, int W>
-__device__ __forceinline__ void backward_tile(BatchLds<W> &s, int tile, int seg,
+__device__ __forceinline__ void backward_tile(BackwardLds<W> &s, int tile, int seg,
                                               const Checkpoints &ck, GS_BACKWARD_PARAMS) {
     constexpr int S = kStrips / W;
     const float T_thr = effective_T_thr(T_thr_in);
@@ -1072,7 +1215,7 @@ __device__ __forceinline__ void backward_tile(BatchLds<W> &s, int tile, int seg,
     float cr[S], cg[S], cb[S];
     uint32_t work = 0;  // unused here
     if (!image)
-        blend_accumulate<W>(s, span, ids, n, points, conics, opac, colors, pix, alpha_thr,
+        blend_accumulate<W>(s.batch, span, ids, n, points, conics, opac, colors, pix, alpha_thr,
                             T_thr_in, chi, cr, cg, cb, work);
     bool finite = true;
 #pragma unroll
@@ -1105,9 +1248,9 @@ __device__ __forceinline__ void backward_tile(BatchLds<W> &s, int tile, int seg,
         L.gr[q] = gr;
         L.gg[q] = gg;
         L.gb[q] = gb;
-        L.gC[q] = gr * cr[q] + gg * cg[q] + gb * cb[q];
-        L.acc[q] = -L.gC[q];
-        finite = finite && isfinite(gr) && isfinite(gg) && isfinite(gb) && isfinite(L.gC[q]);
+        const float gC = gr * cr[q] + gg * cg[q] + gb * cb[q];
+        L.acc[q] = -gC;
+        finite = finite && isfinite(gr) && isfinite(gg) && isfinite(gb) && isfinite(gC);
         // active while !(T < T_thr); pixels outside the image or with a zero
         // gradient (skipped as in src/cuda/kernel.cu:1028-1030) start inactive
         const bool live = pix.inside[q] && !(gr == 0.0f && gg == 0.0f && gb == 0.0f);
@@ -1118,31 +1261,27 @@ __device__ __forceinline__ void backward_tile(BatchLds<W> &s, int tile, int seg,
                              (threadIdx.x % kWave) + kWave * (q0 + q);
             T0 = c[0];
             L.acc[q] = fmaf(gr, c[kTilePixels], fmaf(gg, c[2 * kTilePixels],
-                                                    gb * c[3 * kTilePixels])) - L.gC[q];
+                                                    gb * c[3 * kTilePixels])) - gC;
             finite = finite && isfinite(L.acc[q]);
         }
         L.T[q] = live ? T0 : kInactiveT;
     }
     // the zero-weight update needs finite gradients and image values in the tile
-    const bool tile_nonfinite = tile_any<W>(__ballot(!finite) != 0, s.wave_flag_once);
+    const bool tile_safe = tile_any<W>(__ballot(!finite) != 0, s.batch.wave_flag_once) ||
+                           !(T_thr >= kMinFastT);
 
-    const int lane = threadIdx.x % kWave;
-    const bool hi8 = (lane & 8) != 0;
-    const bool f8_lane = lane == 4;
-    const GradTarget tgt = grad_target(lane, g_points, g_conics, g_opac, g_colors);
+    const GradTarget tgt = grad_target(threadIdx.x % kWave, out);
 
-    BatchPipe<true, true, W> pipe;
-    pipe.start(span, ids, n, points, conics, opac, colors);
+    BatchPipe<true, W> pipe;
+    pipe.start(span, ids);
     for (int32_t b0 = span.start; b0 < span.end; b0 += kBatch * W) {
-        if (!tile_any<W>(any_active(L.T, T_thr), s.wave_flag)) break;
-        const Staged st = pipe.advance(s, b0, span, ids, n, points, conics, opac, colors, chi,
-                                       alpha_thr, pix.x0, pix.y0);
-        if (st.nonfinite || tile_nonfinite)
-            backward_batch<true, W>(s, st.count, pix, alpha_thr, T_thr, chi, L, tgt, hi8,
-                                    f8_lane);
+        if (!tile_any<W>(any_active(L.T, T_thr), s.batch.wave_flag)) break;
+        const Staged st = pipe.advance(s.batch, b0, span, ids, n, points, conics, opac, colors,
+                                       chi, alpha_thr, pix.x0, pix.y0);
+        if (st.nonfinite || tile_safe)
+            backward_batch<true, W>(s, st.count, pix, alpha_thr, T_thr, L, tgt, out);
         else
-            backward_batch<false, W>(s, st.count, pix, alpha_thr, T_thr, chi, L, tgt, hi8,
-                                     f8_lane);
+            backward_batch<false, W>(s, st.count, pix, alpha_thr, T_thr, L, tgt, out);
     }
 }
 
@@ -1155,7 +1294,7 @@ __device__ __forceinline__ void backward_tile(BatchLds<W> &s, int tile, int seg,
 template <int kSeed, int W>
 __global__ __launch_bounds__(kWave * W) void blend_backward_kernel(
     GS_BACKWARD_PARAMS, const int32_t *__restrict__ tile_order, Checkpoints ck) {
-    __shared__ BatchLds<W> s;
+    __shared__ BackwardLds<W> s;
     int tile, seg = -1;
     if (!ck.items) {
         const int slot = tile_of_block(blockIdx.x, n_tiles);
@@ -1172,8 +1311,30 @@ __global__ __launch_bounds__(kWave * W) void blend_backward_kernel(
     }
     backward_tile<kSeed, W>(s, tile, seg, ck, grad_image, image, offsets, ids, n_tiles, k, n,
                             points, conics, opac, colors, tiles_x, width, height, alpha_thr,
-                            T_thr_in, chi, g_points, g_conics, g_opac, g_colors, grad_loss,
-                            inv_count, extra);
+                            T_thr_in, chi, out, grad_loss, inv_count, extra);
+}
+
+// Rows of nine gradients (grad_rows) -> the four arrays.  Bound by memory: a
+// block's 9 KB are read and written in whole lines, through LDS.
+constexpr int kSplitBlock = 256;
+
+__global__ __launch_bounds__(kSplitBlock) void split_rows_kernel(
+    const float *__restrict__ rows, int64_t n, float *__restrict__ points,
+    float *__restrict__ conics, float *__restrict__ opac, float *__restrict__ colors) {
+    __shared__ float lds[kSplitBlock * kGradFields];
+    const int64_t first = (int64_t)blockIdx.x * kSplitBlock;
+    const int nb = (int)min((int64_t)kSplitBlock, n - first);
+    const int t = threadIdx.x;
+    for (int i = t; i < nb * kGradFields; i += kSplitBlock) lds[i] = rows[first * kGradFields + i];
+    __syncthreads();
+    for (int i = t; i < nb * 2; i += kSplitBlock)
+        points[first * 2 + i] = lds[(i >> 1) * kGradFields + (i & 1)];
+    for (int i = t; i < nb * 3; i += kSplitBlock) {
+        const int g = i / 3, c = i - 3 * g;
+        conics[first * 3 + i] = lds[g * kGradFields + 2 + c];
+        colors[first * 3 + i] = lds[g * kGradFields + 6 + c];
+    }
+    if (t < nb) opac[first + t] = lds[t * kGradFields + 5];
 }
 
 // ------------------------------------------------ generic tile size path
@@ -1219,8 +1380,7 @@ __global__ void blend_backward_generic_kernel(
     const int32_t *__restrict__ offsets, const int32_t *__restrict__ ids, int n_tiles,
     int64_t k, int64_t n, const float *__restrict__ points, const float *__restrict__ conics,
     const float *__restrict__ opac, const float *__restrict__ colors, int tiles_x, int width,
-    int height, int ts, float alpha_thr, float T_thr, float chi, float *__restrict__ g_points,
-    float *__restrict__ g_conics, float *__restrict__ g_opac, float *__restrict__ g_colors) {
+    int height, int ts, float alpha_thr, float T_thr, float chi, GradOut out) {
     const int tile = blockIdx.x;
     const int px = (tile % tiles_x) * ts + (int)threadIdx.x % ts;
     const int py = (tile / tiles_x) * ts + (int)threadIdx.x / ts;
@@ -1273,15 +1433,18 @@ __global__ void blend_backward_generic_kernel(
         const float one_m = (1.0f - alpha) + kTransmittanceEps;
         const float dalpha = T * gcol - (gC - acc_new) / one_m;
         const float h = alpha * dalpha;
-        unsafeAtomicAdd(g_points + 2 * g, h * fmaf(A, du, B * dv));
-        unsafeAtomicAdd(g_points + 2 * g + 1, h * fmaf(B, du, C * dv));
-        unsafeAtomicAdd(g_conics + 3 * g, -0.5f * h * du * du);
-        unsafeAtomicAdd(g_conics + 3 * g + 1, -h * du * dv);
-        unsafeAtomicAdd(g_conics + 3 * g + 2, -0.5f * h * dv * dv);
-        unsafeAtomicAdd(g_opac + g, G * dalpha);
-        unsafeAtomicAdd(g_colors + 3 * g, w * gr);
-        unsafeAtomicAdd(g_colors + 3 * g + 1, w * gg);
-        unsafeAtomicAdd(g_colors + 3 * g + 2, w * gb);
+        float *g_points = out.points + (int64_t)g * out.s_points;
+        float *g_conics = out.conics + (int64_t)g * out.s_conics;
+        float *g_colors = out.colors + (int64_t)g * out.s_colors;
+        unsafeAtomicAdd(g_points, h * fmaf(A, du, B * dv));
+        unsafeAtomicAdd(g_points + 1, h * fmaf(B, du, C * dv));
+        unsafeAtomicAdd(g_conics, -0.5f * h * du * du);
+        unsafeAtomicAdd(g_conics + 1, -h * du * dv);
+        unsafeAtomicAdd(g_conics + 2, -0.5f * h * dv * dv);
+        unsafeAtomicAdd(out.opac + (int64_t)g * out.s_opac, G * dalpha);
+        unsafeAtomicAdd(g_colors, w * gr);
+        unsafeAtomicAdd(g_colors + 1, w * gg);
+        unsafeAtomicAdd(g_colors + 2, w * gb);
         acc = acc_new;
         T = T * one_m;
         if (T < T_thr) break;
@@ -1697,34 +1860,39 @@ extern "C" int gs_l1_finish(const float *tile_loss, int32_t n_tiles, int64_t cou
                             nullptr, stream);
 }
 
+// `out`: the caller's outputs, each checked against null by the callers; zeroed
+// here unless accumulate.
 static int rasterize_backward_impl(
     const float *grad_image, const float *image, const int32_t *indexing_offset,
     const int32_t *gaussian_ids_sorted, int32_t n_tiles, int64_t k, const float *points_image,
     const float *cov_inv_image, const float *opacities, const float *colors, int64_t n,
     int32_t width, int32_t height, int32_t tile_size, float alpha_threshold,
-    float transmittance_threshold, float chi_squared_threshold, float *grad_points_image,
-    float *grad_cov_inv_image, float *grad_opacities, float *grad_colors, int32_t accumulate,
-    int seed, const float *grad_loss, float inv_count, hipStream_t stream,
-    const float *extra = nullptr, const int32_t *tile_order = nullptr,
-    Checkpoints ck = kNoCheckpoints) {
+    float transmittance_threshold, float chi_squared_threshold, const GradOut &out,
+    int32_t accumulate, int seed, const float *grad_loss, float inv_count, hipStream_t stream,
+    const float *extra = nullptr, const int32_t *tile_schedule = nullptr) {
     int st = check_blend_args(indexing_offset, gaussian_ids_sorted, n_tiles, k, n, width, height,
                               tile_size, alpha_threshold, transmittance_threshold,
                               chi_squared_threshold);
     if (st) return st;
-    if (n > 0 && (!grad_points_image || !grad_cov_inv_image || !grad_opacities || !grad_colors))
+    if (n > 0 && (!out.points || !out.conics || !out.opac || !out.colors))
         return GS_ERR_INVALID_ARGUMENT;
     if (seed != kSeedImage && (!image || tile_size != kTile)) return GS_ERR_INVALID_ARGUMENT;
     if (seed == kSeedL1 && !grad_loss) return GS_ERR_INVALID_ARGUMENT;
     if (n > 0 && !accumulate) {
-        st = zero_bytes(grad_points_image, (size_t)n * 2 * sizeof(float), stream);
-        if (!st) st = zero_bytes(grad_cov_inv_image, (size_t)n * 3 * sizeof(float), stream);
-        if (!st) st = zero_bytes(grad_opacities, (size_t)n * sizeof(float), stream);
-        if (!st) st = zero_bytes(grad_colors, (size_t)n * 3 * sizeof(float), stream);
+        if (out.s_points == kGradFields) {
+            st = zero_bytes(out.points, (size_t)n * kGradFields * sizeof(float), stream);
+        } else {
+            st = zero_bytes(out.points, (size_t)n * 2 * sizeof(float), stream);
+            if (!st) st = zero_bytes(out.conics, (size_t)n * 3 * sizeof(float), stream);
+            if (!st) st = zero_bytes(out.opac, (size_t)n * sizeof(float), stream);
+            if (!st) st = zero_bytes(out.colors, (size_t)n * 3 * sizeof(float), stream);
+        }
         if (st) return st;
     }
     if (n_tiles == 0 || k == 0) return GS_OK;
     if (!grad_image || !points_image || !cov_inv_image || !opacities || !colors)
         return GS_ERR_INVALID_ARGUMENT;
+    const int32_t *tile_order = tile_schedule ? tile_schedule + n_tiles : nullptr;
     const int tiles_x = (width + tile_size - 1) / tile_size;
     if (tile_size == kTile) {
         const int W = blend_waves(n_tiles);
@@ -1742,25 +1910,29 @@ static int rasterize_backward_impl(
                                     blend_backward_kernel<kSeedImage, 1>);
         // segments from the forward's checkpoints need the image (a recomputed
         // forward has none) and the order they came with
-        if (!image || !tile_order) ck = kNoCheckpoints;
+        const Checkpoints ck = image ? schedule_ck(tile_schedule, n_tiles) : kNoCheckpoints;
         // with lists: kSegments workgroups per slot of the largest range, on each XCD
         const int64_t grid =
             ck.items ? (int64_t)kXcds * kSegments * ((n_tiles + kXcds - 1) / kXcds) : n_tiles;
         hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kWave * W), 0, stream, grad_image,
                            image, indexing_offset, gaussian_ids_sorted, n_tiles, k, n,
                            points_image, cov_inv_image, opacities, colors, tiles_x, width, height,
-                           alpha_threshold, transmittance_threshold, chi_squared_threshold,
-                           grad_points_image, grad_cov_inv_image, grad_opacities, grad_colors,
+                           alpha_threshold, transmittance_threshold, chi_squared_threshold, out,
                            grad_loss, inv_count, extra, tile_order, ck);
     } else {
         hipLaunchKernelGGL(blend_backward_generic_kernel, dim3(n_tiles),
                            dim3(tile_size * tile_size), 0, stream, grad_image, image,
                            indexing_offset, gaussian_ids_sorted, n_tiles, k, n, points_image,
                            cov_inv_image, opacities, colors, tiles_x, width, height, tile_size,
-                           alpha_threshold, transmittance_threshold, chi_squared_threshold,
-                           grad_points_image, grad_cov_inv_image, grad_opacities, grad_colors);
+                           alpha_threshold, transmittance_threshold, chi_squared_threshold, out);
     }
     return launch_status();
+}
+
+// loss_scale / (H * W * 3): the L1 term's gradient w.r.t. display / 255 is
+// sign * *grad_loss * that.
+static float l1_inv_count(float loss_scale, int32_t width, int32_t height) {
+    return (float)((double)loss_scale / ((double)width * (double)height * 3.0));
 }
 
 extern "C" int gs_rasterize_backward(
@@ -1771,12 +1943,12 @@ extern "C" int gs_rasterize_backward(
     float transmittance_threshold, float chi_squared_threshold, float *grad_points_image,
     float *grad_cov_inv_image, float *grad_opacities, float *grad_colors, int32_t accumulate,
     hipStream_t stream) {
-    return rasterize_backward_impl(grad_image, image, indexing_offset, gaussian_ids_sorted,
-                                   n_tiles, k, points_image, cov_inv_image, opacities, colors, n,
-                                   width, height, tile_size, alpha_threshold,
-                                   transmittance_threshold, chi_squared_threshold,
-                                   grad_points_image, grad_cov_inv_image, grad_opacities,
-                                   grad_colors, accumulate, kSeedImage, nullptr, 0.0f, stream);
+    return rasterize_backward_impl(
+        grad_image, image, indexing_offset, gaussian_ids_sorted, n_tiles, k, points_image,
+        cov_inv_image, opacities, colors, n, width, height, tile_size, alpha_threshold,
+        transmittance_threshold, chi_squared_threshold,
+        grad_arrays(grad_points_image, grad_cov_inv_image, grad_opacities, grad_colors),
+        accumulate, kSeedImage, nullptr, 0.0f, stream);
 }
 
 extern "C" int gs_rasterize_display_backward(
@@ -1787,14 +1959,12 @@ extern "C" int gs_rasterize_display_backward(
     float transmittance_threshold, float chi_squared_threshold, float *grad_points_image,
     float *grad_cov_inv_image, float *grad_opacities, float *grad_colors, int32_t accumulate,
     const int32_t *tile_schedule, hipStream_t stream) {
-    return rasterize_backward_impl(grad_display, image, indexing_offset, gaussian_ids_sorted,
-                                   n_tiles, k, points_image, cov_inv_image, opacities, colors, n,
-                                   width, height, tile_size, alpha_threshold,
-                                   transmittance_threshold, chi_squared_threshold,
-                                   grad_points_image, grad_cov_inv_image, grad_opacities,
-                                   grad_colors, accumulate, kSeedDisplay, nullptr, 0.0f, stream,
-                                   nullptr, tile_schedule ? tile_schedule + n_tiles : nullptr,
-                                   schedule_ck(tile_schedule, n_tiles));
+    return rasterize_backward_impl(
+        grad_display, image, indexing_offset, gaussian_ids_sorted, n_tiles, k, points_image,
+        cov_inv_image, opacities, colors, n, width, height, tile_size, alpha_threshold,
+        transmittance_threshold, chi_squared_threshold,
+        grad_arrays(grad_points_image, grad_cov_inv_image, grad_opacities, grad_colors),
+        accumulate, kSeedDisplay, nullptr, 0.0f, stream, nullptr, tile_schedule);
 }
 
 extern "C" int gs_rasterize_l1_backward(
@@ -1808,16 +1978,48 @@ extern "C" int gs_rasterize_l1_backward(
     const int32_t *tile_schedule, hipStream_t stream) {
     if (!target || width <= 0 || height <= 0 || !(loss_scale == loss_scale))
         return GS_ERR_INVALID_ARGUMENT;
-    // d loss / d (display / 255) = sign * *grad_loss * loss_scale / (H * W * 3)
-    const float inv_count = (float)((double)loss_scale / ((double)width * (double)height * 3.0));
-    return rasterize_backward_impl(target, image, indexing_offset, gaussian_ids_sorted, n_tiles,
-                                   k, points_image, cov_inv_image, opacities, colors, n, width,
-                                   height, tile_size, alpha_threshold, transmittance_threshold,
-                                   chi_squared_threshold, grad_points_image, grad_cov_inv_image,
-                                   grad_opacities, grad_colors, accumulate, kSeedL1, grad_loss,
-                                   inv_count, stream, grad_display01,
-                                   tile_schedule ? tile_schedule + n_tiles : nullptr,
-                                   schedule_ck(tile_schedule, n_tiles));
+    return rasterize_backward_impl(
+        target, image, indexing_offset, gaussian_ids_sorted, n_tiles, k, points_image,
+        cov_inv_image, opacities, colors, n, width, height, tile_size, alpha_threshold,
+        transmittance_threshold, chi_squared_threshold,
+        grad_arrays(grad_points_image, grad_cov_inv_image, grad_opacities, grad_colors),
+        accumulate, kSeedL1, grad_loss, l1_inv_count(loss_scale, width, height), stream,
+        grad_display01, tile_schedule);
+}
+
+extern "C" int gs_rasterize_backward_rows(
+    int32_t seed, const float *grad, const float *grad_loss, const float *image,
+    const int32_t *indexing_offset, const int32_t *gaussian_ids_sorted, int32_t n_tiles,
+    int64_t k, const float *points_image, const float *cov_inv_image, const float *opacities,
+    const float *colors, int64_t n, int32_t width, int32_t height, int32_t tile_size,
+    float alpha_threshold, float transmittance_threshold, float chi_squared_threshold,
+    float *rows, int32_t accumulate, float loss_scale, const float *grad_display01,
+    const int32_t *tile_schedule, hipStream_t stream) {
+    if (seed != kSeedImage && seed != kSeedDisplay && seed != kSeedL1)
+        return GS_ERR_INVALID_ARGUMENT;
+    if (seed == kSeedL1 && (!grad || width <= 0 || height <= 0 || !(loss_scale == loss_scale)))
+        return GS_ERR_INVALID_ARGUMENT;
+    if (n > 0 && !rows) return GS_ERR_INVALID_ARGUMENT;
+    return rasterize_backward_impl(
+        grad, image, indexing_offset, gaussian_ids_sorted, n_tiles, k, points_image,
+        cov_inv_image, opacities, colors, n, width, height, tile_size, alpha_threshold,
+        transmittance_threshold, chi_squared_threshold, grad_rows(rows), accumulate, seed,
+        seed == kSeedL1 ? grad_loss : nullptr,
+        seed == kSeedL1 ? l1_inv_count(loss_scale, width, height) : 0.0f, stream,
+        seed == kSeedL1 ? grad_display01 : nullptr, tile_schedule);
+}
+
+extern "C" int gs_split_gradient_rows(const float *rows, int64_t n, float *grad_points_image,
+                                      float *grad_cov_inv_image, float *grad_opacities,
+                                      float *grad_colors, hipStream_t stream) {
+    if (n < 0) return GS_ERR_INVALID_ARGUMENT;
+    if (n == 0) return GS_OK;
+    if (!rows || !grad_points_image || !grad_cov_inv_image || !grad_opacities || !grad_colors)
+        return GS_ERR_INVALID_ARGUMENT;
+    hipLaunchKernelGGL(split_rows_kernel, dim3((unsigned)((n + kSplitBlock - 1) / kSplitBlock)),
+                       dim3(kSplitBlock), 0, stream, rows, n, grad_points_image,
+                       grad_cov_inv_image, grad_opacities, grad_colors);
+    return launch_status();
 }
 
 extern "C" int gs_rasterize_work(const int32_t *indexing_offset,

@@ -527,11 +527,16 @@ __global__ __launch_bounds__(kShBlock) void preprocess_forward_kernel(
 // 12-byte stores (10 KB of LDS per block instead of the 23 KB of staged rows).
 constexpr int kBasisStride = 16;  // LDS floats per Gaussian's basis values (15 used)
 
+// Gradients of the blend inputs: four arrays (strides 2, 3, 1, 3), or one row of
+// nine floats per Gaussian (the strides are then 9).
+struct BlendGrads {
+    const float *points, *conics, *opac, *colors;
+    int s_points, s_conics, s_opac, s_colors;
+};
+
 template <bool kRaw, bool kCached>
 __global__ __launch_bounds__(kShBlock) void preprocess_backward_kernel(
-    int64_t n, const float *__restrict__ grad_points_image,
-    const float *__restrict__ grad_cov_inv, const float *__restrict__ grad_opac,
-    const float *__restrict__ grad_colors, const float *__restrict__ means,
+    int64_t n, BlendGrads grads, const float *__restrict__ means,
     const float *__restrict__ log_scales, const float *__restrict__ quats_raw,
     const float *__restrict__ logits, const float *__restrict__ sh_dc,
     const float *__restrict__ sh_rest, const float *__restrict__ cov_image,
@@ -570,12 +575,14 @@ __global__ __launch_bounds__(kShBlock) void preprocess_backward_kernel(
         float gm[3] = {0.f, 0.f, 0.f}, gdc[3] = {0.f, 0.f, 0.f};
         if (mask[i]) {
             const Camera cam = load_camera(w2c, K, width, height);
+            const float *g_pt = grads.points + i * grads.s_points;
+            const float *g_cv = grads.conics + i * grads.s_conics;
             project_gaussian_backward(
                 cam, means[3 * i], means[3 * i + 1], means[3 * i + 2], a.s[0], a.s[1], a.s[2],
                 a.q[0], a.q[1], a.q[2], a.q[3], cov_image[3 * i], cov_image[3 * i + 1],
-                cov_image[3 * i + 2], grad_points_image[2 * i], grad_points_image[2 * i + 1],
-                grad_cov_inv[3 * i], grad_cov_inv[3 * i + 1], grad_cov_inv[3 * i + 2], gp[0],
-                gp[1], gp[2], gs[0], gs[1], gs[2], gq[0], gq[1], gq[2], gq[3]);
+                cov_image[3 * i + 2], g_pt[0], g_pt[1], g_cv[0], g_cv[1], g_cv[2], gp[0], gp[1],
+                gp[2], gs[0], gs[1], gs[2], gq[0], gq[1], gq[2], gq[3]);
+            const float *g_cl = grads.colors + i * grads.s_colors;
             float cx, cy, cz;
             camera_position(nullptr, w2c, cx, cy, cz);
             const ShView v = sh_view(means + 3 * i, cx, cy, cz);
@@ -585,7 +592,7 @@ __global__ __launch_bounds__(kShBlock) void preprocess_backward_kernel(
                 const uint32_t pass = sh_cache_load(sh_cache, i, m);
 #pragma unroll
                 for (int c = 0; c < 3; ++c) {
-                    g[c] = grad_colors[3 * i + c];
+                    g[c] = g_cl[c];
                     if (!((pass >> c) & 1u)) g[c] = 0.0f;
                 }
                 sh_mean_grad(m, g, gm);
@@ -598,7 +605,7 @@ __global__ __launch_bounds__(kShBlock) void preprocess_backward_kernel(
             } else {
 #pragma unroll
                 for (int c = 0; c < 3; ++c) {
-                    g[c] = grad_colors[3 * i + c];
+                    g[c] = g_cl[c];
                     const float raw = sh_raw_channel(v, sh_dc + 3 * i, lrest, c);
                     if (!(raw + 0.5f >= 0.0f)) g[c] = 0.0f;
                 }
@@ -616,8 +623,8 @@ __global__ __launch_bounds__(kShBlock) void preprocess_backward_kernel(
         float g_ls[3], g_logit = 0.0f;
         float4 g_qr;
         if constexpr (kRaw) {
-            activate_backward_one(a, gs, make_float4(gq[0], gq[1], gq[2], gq[3]), grad_opac[i],
-                                  g_ls, g_qr, g_logit);
+            activate_backward_one(a, gs, make_float4(gq[0], gq[1], gq[2], gq[3]),
+                                  grads.opac[i * grads.s_opac], g_ls, g_qr, g_logit);
         } else {
 #pragma unroll
             for (int c = 0; c < 3; ++c) g_ls[c] = gs[c];
@@ -885,18 +892,16 @@ extern "C" int gs_preprocess_forward(const float *means, const float *log_scales
     return launch_status();
 }
 
-extern "C" int gs_preprocess_backward(
-    const float *grad_points_image, const float *grad_cov_inv_image,
-    const float *grad_opacities, const float *grad_colors, const float *means,
-    const float *log_scales, const float *quats_raw, const float *opacity_logits,
-    const float *sh_dc, const float *sh_rest, const float *cov_image, const uint8_t *mask,
-    const float *world_to_camera, const float *intrinsic, int64_t n, int32_t width,
-    int32_t height, float *grad_means, float *grad_log_scales, float *grad_quats_raw,
-    float *grad_opacity_logits, float *grad_sh_dc, float *grad_sh_rest, const float *sh_cache,
-    hipStream_t stream) {
+static int preprocess_backward_impl(
+    const BlendGrads &grads, const float *means, const float *log_scales, const float *quats_raw,
+    const float *opacity_logits, const float *sh_dc, const float *sh_rest, const float *cov_image,
+    const uint8_t *mask, const float *world_to_camera, const float *intrinsic, int64_t n,
+    int32_t width, int32_t height, float *grad_means, float *grad_log_scales,
+    float *grad_quats_raw, float *grad_opacity_logits, float *grad_sh_dc, float *grad_sh_rest,
+    const float *sh_cache, hipStream_t stream) {
     if (n < 0 || width <= 0 || height <= 0) return GS_ERR_INVALID_ARGUMENT;
     if (n == 0) return GS_OK;
-    if (!grad_points_image || !grad_cov_inv_image || !grad_opacities || !grad_colors || !means ||
+    if (!grads.points || !grads.conics || !grads.opac || !grads.colors || !means ||
         !log_scales || !quats_raw || !opacity_logits || (!sh_cache && (!sh_dc || !sh_rest)) ||
         !cov_image || !mask || !world_to_camera || !intrinsic || !grad_means ||
         !grad_log_scales || !grad_quats_raw || !grad_opacity_logits || !grad_sh_dc ||
@@ -906,12 +911,46 @@ extern "C" int gs_preprocess_backward(
         return GS_ERR_INVALID_ARGUMENT;
     auto kern = sh_cache ? preprocess_backward_kernel<true, true>
                          : preprocess_backward_kernel<true, false>;
-    hipLaunchKernelGGL(kern, dim3(ceil_div(n, kShBlock)), dim3(kShBlock), 0, stream, n,
-                       grad_points_image, grad_cov_inv_image, grad_opacities, grad_colors, means,
-                       log_scales, quats_raw, opacity_logits, sh_dc, sh_rest, cov_image, mask,
-                       world_to_camera, intrinsic, width, height, grad_means, grad_log_scales,
-                       grad_quats_raw, grad_opacity_logits, grad_sh_dc, grad_sh_rest, sh_cache);
+    hipLaunchKernelGGL(kern, dim3(ceil_div(n, kShBlock)), dim3(kShBlock), 0, stream, n, grads,
+                       means, log_scales, quats_raw, opacity_logits, sh_dc, sh_rest, cov_image,
+                       mask, world_to_camera, intrinsic, width, height, grad_means,
+                       grad_log_scales, grad_quats_raw, grad_opacity_logits, grad_sh_dc,
+                       grad_sh_rest, sh_cache);
     return launch_status();
+}
+
+extern "C" int gs_preprocess_backward(
+    const float *grad_points_image, const float *grad_cov_inv_image, const float *grad_opacities,
+    const float *grad_colors, const float *means, const float *log_scales,
+    const float *quats_raw, const float *opacity_logits, const float *sh_dc,
+    const float *sh_rest, const float *cov_image, const uint8_t *mask,
+    const float *world_to_camera, const float *intrinsic, int64_t n, int32_t width,
+    int32_t height, float *grad_means, float *grad_log_scales, float *grad_quats_raw,
+    float *grad_opacity_logits, float *grad_sh_dc, float *grad_sh_rest, const float *sh_cache,
+    hipStream_t stream) {
+    const BlendGrads grads{grad_points_image, grad_cov_inv_image, grad_opacities, grad_colors,
+                           2, 3, 1, 3};
+    return preprocess_backward_impl(grads, means, log_scales, quats_raw, opacity_logits, sh_dc,
+                                    sh_rest, cov_image, mask, world_to_camera, intrinsic, n,
+                                    width, height, grad_means, grad_log_scales, grad_quats_raw,
+                                    grad_opacity_logits, grad_sh_dc, grad_sh_rest, sh_cache,
+                                    stream);
+}
+
+extern "C" int gs_preprocess_backward_rows(
+    const float *rows, const float *means, const float *log_scales, const float *quats_raw,
+    const float *opacity_logits, const float *sh_dc, const float *sh_rest, const float *cov_image,
+    const uint8_t *mask, const float *world_to_camera, const float *intrinsic, int64_t n,
+    int32_t width, int32_t height, float *grad_means, float *grad_log_scales,
+    float *grad_quats_raw, float *grad_opacity_logits, float *grad_sh_dc, float *grad_sh_rest,
+    const float *sh_cache, hipStream_t stream) {
+    if (n > 0 && !rows) return GS_ERR_INVALID_ARGUMENT;
+    const BlendGrads grads{rows, rows + 2, rows + 5, rows + 6, 9, 9, 9, 9};
+    return preprocess_backward_impl(grads, means, log_scales, quats_raw, opacity_logits, sh_dc,
+                                    sh_rest, cov_image, mask, world_to_camera, intrinsic, n,
+                                    width, height, grad_means, grad_log_scales, grad_quats_raw,
+                                    grad_opacity_logits, grad_sh_dc, grad_sh_rest, sh_cache,
+                                    stream);
 }
 
 extern "C" int gs_render_preprocess_backward(
@@ -928,12 +967,13 @@ extern "C" int gs_render_preprocess_backward(
         !world_to_camera || !intrinsic || !grad_means || !grad_scales || !grad_quaternions ||
         !grad_sh_dc || !grad_sh_rest || (reinterpret_cast<uintptr_t>(sh_cache) & 7))
         return GS_ERR_INVALID_ARGUMENT;
+    const BlendGrads grads{grad_points_image, grad_cov_inv_image, nullptr, grad_colors,
+                           2, 3, 0, 3};
     auto kern = sh_cache ? preprocess_backward_kernel<false, true>
                          : preprocess_backward_kernel<false, false>;
     hipLaunchKernelGGL(kern, dim3(ceil_div(n, kShBlock)), dim3(kShBlock), 0, stream, n,
-                       grad_points_image, grad_cov_inv_image, nullptr, grad_colors, means, scales,
-                       quaternions, nullptr, sh_dc, sh_rest, cov_image, mask, world_to_camera,
-                       intrinsic, width, height, grad_means, grad_scales, grad_quaternions,
-                       nullptr, grad_sh_dc, grad_sh_rest, sh_cache);
+                       grads, means, scales, quaternions, nullptr, sh_dc, sh_rest, cov_image,
+                       mask, world_to_camera, intrinsic, width, height, grad_means, grad_scales,
+                       grad_quaternions, nullptr, grad_sh_dc, grad_sh_rest, sh_cache);
     return launch_status();
 }

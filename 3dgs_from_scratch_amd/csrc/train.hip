@@ -50,12 +50,13 @@ __global__ __launch_bounds__(kTrainBlock) void adam_kernel(AdamBatch batch, floa
 // src/strategy.py:47-68: for Gaussians with both radii > 0,
 //   grads += |(du * W/2, dv * H/2)|, count += 1.
 __global__ __launch_bounds__(kTrainBlock) void accumulate_grad2d_kernel(
-    int64_t n, const float *__restrict__ grad_points, const float *__restrict__ radii,
-    float half_w, float half_h, float *__restrict__ grads, float *__restrict__ count) {
+    int64_t n, const float *__restrict__ grad_points, int stride,
+    const float *__restrict__ radii, float half_w, float half_h, float *__restrict__ grads, float *__restrict__ count) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     if (!(radii[2 * i] > 0.0f && radii[2 * i + 1] > 0.0f)) return;
-    const float gx = grad_points[2 * i] * half_w, gy = grad_points[2 * i + 1] * half_h;
+    const float *g = grad_points + i * stride;
+    const float gx = g[0] * half_w, gy = g[1] * half_h;
     grads[i] += sqrtf(gx * gx + gy * gy);
     count[i] += 1.0f;
 }
@@ -123,16 +124,24 @@ extern "C" int gs_adam_step(const GsAdamTensor *tensors, int32_t n_tensors, doub
     return GS_OK;
 }
 
-extern "C" int gs_accumulate_grad2d(const float *grad_points_image, const float *radii, int64_t n,
-                                    int32_t width, int32_t height, float *grads, float *count,
-                                    hipStream_t stream) {
-    if (n < 0 || width <= 0 || height <= 0) return GS_ERR_INVALID_ARGUMENT;
+extern "C" int gs_accumulate_grad2d_strided(const float *grad_points_image, int32_t row_stride,
+                                            const float *radii, int64_t n, int32_t width,
+                                            int32_t height, float *grads, float *count,
+                                            hipStream_t stream) {
+    if (n < 0 || width <= 0 || height <= 0 || row_stride < 2) return GS_ERR_INVALID_ARGUMENT;
     if (n == 0) return GS_OK;
     if (!grad_points_image || !radii || !grads || !count) return GS_ERR_INVALID_ARGUMENT;
     hipLaunchKernelGGL(accumulate_grad2d_kernel, dim3(ceil_div(n, kTrainBlock)), dim3(kTrainBlock),
-                       0, stream, n, grad_points_image, radii, (float)width / 2.0f,
+                       0, stream, n, grad_points_image, row_stride, radii, (float)width / 2.0f,
                        (float)height / 2.0f, grads, count);
     return launch_status();
+}
+
+extern "C" int gs_accumulate_grad2d(const float *grad_points_image, const float *radii, int64_t n,
+                                    int32_t width, int32_t height, float *grads, float *count,
+                                    hipStream_t stream) {
+    return gs_accumulate_grad2d_strided(grad_points_image, 2, radii, n, width, height, grads,
+                                        count, stream);
 }
 
 extern "C" int gs_gather_rows(int64_t n_out, const int32_t *src_rows, const uint8_t *fresh_rows,

@@ -56,9 +56,11 @@ __all__ = [
     "activate_backward",
     "preprocess_forward",
     "preprocess_backward",
+    "preprocess_backward_rows",
     "render_preprocess_backward",
     "rasterize_display_l1",
     "rasterize_l1_backward",
+    "rasterize_l1_backward_rows",
     "blend_grad_accumulators",
     "tile_schedule",
     "schedule_size",
@@ -687,14 +689,45 @@ def _blend_grad_views(buf, n):
             buf[6 * n :].view(n, 3))
 
 
-def _zeroed_blend_grads(n, dev):
-    """Four zeroed gradient outputs (N,2), (N,3), (N,), (N,3) carved from one buffer."""
-    return _blend_grad_views(torch.zeros((9 * n,), dtype=torch.float32, device=dev), n)
+_SEED_IMAGE, _SEED_DISPLAY, _SEED_L1 = 0, 1, 2
+
+
+def _backward_rows(stage, seed, grad, blend, width, height, tile_size, alpha_threshold,
+                   transmittance_threshold, chi_squared_threshold, image, rows, grad_loss=None,
+                   loss_scale=0.0, extra=None, schedule=None):
+    """gs_rasterize_backward_rows: adds the blend gradients into `rows`, 9N floats, one
+    row of nine per Gaussian.  `blend`: _blend_inputs' result.  `stage` names the
+    timed library call (the blend kernel alone)."""
+    dev, n, off, ids, pts, conic, opac, col = blend
+    ev = _lib.timer.record(stage, dev)
+    _lib.check(_lib.load().gs_rasterize_backward_rows(
+        seed, _ptr(grad), _ptr(grad_loss), _ptr(image), _ptr(off), _ptr(ids), off.shape[0],
+        ids.shape[0], _ptr(pts), _ptr(conic), _ptr(opac), _ptr(col), n, width, height,
+        int(tile_size), float(alpha_threshold), float(transmittance_threshold),
+        float(chi_squared_threshold), _ptr(rows), 1, float(loss_scale), _ptr(extra),
+        _ptr(schedule), _stream(dev)), stage)
+    _lib.timer.stop(ev, dev)
+
+
+def _backward_split(*args, **kw):
+    """_backward_rows into zeroed rows, then the four gradients (N,2), (N,3), (N,), (N,3),
+    carved from one buffer.  The rows' atomics are much cheaper than the four arrays'
+    and their copy costs a few microseconds: 72 MB moved at 1M Gaussians."""
+    blend = args[3]
+    dev, n = blend[0], blend[1]
+    with torch.cuda.device(dev):
+        rows = torch.zeros((9 * n,), dtype=torch.float32, device=dev)
+        _backward_rows(*args, rows=rows, **kw)
+        out = _blend_grad_views(torch.empty_like(rows), n)
+        _lib.check(_lib.load().gs_split_gradient_rows(_ptr(rows), n, *(_ptr(t) for t in out),
+                                                      _stream(dev)), args[0])
+    return out
 
 
 def blend_grad_accumulators(n, device):
     """An uninitialised 9N fp32 buffer for the blend gradients: pass it as
     rasterize_display_l1(clear=...) (which zeroes it) and then as
+    rasterize_l1_backward_rows(accumulators=...) or, for the four arrays,
     rasterize_l1_backward(accumulators=...)."""
     return torch.empty((9 * int(n),), dtype=torch.float32, device=device)
 
@@ -805,31 +838,18 @@ def rasterize_backward(
     grad_colors[N,3]).  `rendered_image`, if given, must be rasterize()'s
     output for the same inputs.
     """
-    dev, n, off, ids, pts, conic, opac, col = _blend_inputs(
+    blend = _blend_inputs(
         indexing_offset, gaussian_ids_sorted, points_image, cov_inv_image, opacities, colors)
+    dev = blend[0]
     width, height = int(width), int(height)
     f32 = torch.float32
     grad = _prep(grad_rendered_image, "grad_rendered_image", f32, (height, width, 3), dev)
     img = None
     if rendered_image is not None:
         img = _prep(rendered_image, "rendered_image", f32, (height, width, 3), dev)
-    # zeroed here (one fill) so that the library call and its timing events are the
-    # blend kernel alone
-    g_pts, g_conic, g_opac, g_col = _zeroed_blend_grads(n, dev)
-    with torch.cuda.device(dev):
-        ev = _lib.timer.record("rasterize_backward", dev)
-        _lib.check(
-            _lib.load().gs_rasterize_backward(
-                _ptr(grad), _ptr(img), _ptr(off), _ptr(ids), off.shape[0], ids.shape[0],
-                _ptr(pts), _ptr(conic), _ptr(opac), _ptr(col), n, width, height, int(tile_size),
-                float(alpha_threshold), float(transmittance_threshold),
-                float(chi_squared_threshold), _ptr(g_pts), _ptr(g_conic), _ptr(g_opac),
-                _ptr(g_col), 1, _stream(dev),
-            ),
-            "rasterize_backward",
-        )
-        _lib.timer.stop(ev, dev)
-    return g_pts, g_conic, g_opac, g_col
+    return _backward_split("rasterize_backward", _SEED_IMAGE, grad, blend, width, height,
+                           tile_size, alpha_threshold, transmittance_threshold,
+                           chi_squared_threshold, img)
 
 
 def rasterize_work(indexing_offset, gaussian_ids_sorted, points_image, cov_inv_image, opacities,
@@ -1024,29 +1044,18 @@ def rasterize_display_backward(grad_display, indexing_offset, gaussian_ids_sorte
     """Gradient of rasterize_display's display output; `rendered_image` (its
     un-clamped image) is required.  Returns the four gradients of rasterize_backward.
     `schedule`: the tensor rasterize_display filled for the same layout."""
-    dev, n, off, ids, pts, conic, opac, col = _blend_inputs(
+    blend = _blend_inputs(
         indexing_offset, gaussian_ids_sorted, points_image, cov_inv_image, opacities, colors)
+    dev, off = blend[0], blend[2]
     width, height = int(width), int(height)
     if schedule is not None:
         _check_schedule(schedule, off.shape[0], dev, "rasterize_display_backward")
     f32 = torch.float32
     grad = _prep(grad_display, "grad_display", f32, (height, width, 3), dev)
     img = _prep(rendered_image, "rendered_image", f32, (height, width, 3), dev)
-    g_pts, g_conic, g_opac, g_col = _zeroed_blend_grads(n, dev)
-    with torch.cuda.device(dev):
-        ev = _lib.timer.record("rasterize_display_backward", dev)
-        _lib.check(
-            _lib.load().gs_rasterize_display_backward(
-                _ptr(grad), _ptr(img), _ptr(off), _ptr(ids), off.shape[0], ids.shape[0],
-                _ptr(pts), _ptr(conic), _ptr(opac), _ptr(col), n, width, height, int(tile_size),
-                float(alpha_threshold), float(transmittance_threshold),
-                float(chi_squared_threshold), _ptr(g_pts), _ptr(g_conic), _ptr(g_opac),
-                _ptr(g_col), 1, _ptr(schedule), _stream(dev),
-            ),
-            "rasterize_display_backward",
-        )
-        _lib.timer.stop(ev, dev)
-    return g_pts, g_conic, g_opac, g_col
+    return _backward_split("rasterize_display_backward", _SEED_DISPLAY, grad, blend, width,
+                           height, tile_size, alpha_threshold, transmittance_threshold,
+                           chi_squared_threshold, img, schedule=schedule)
 
 
 # ------------------------------------------------------ fused training step
@@ -1163,10 +1172,35 @@ def preprocess_backward(grad_points_image, grad_cov_inv_image, grad_opacities, g
     dev = _device_of(means)
     n = means.shape[0]
     f32 = torch.float32
-    g_pts = _prep(grad_points_image, "grad_points_image", f32, (n, 2), dev)
-    g_conic = _prep(grad_cov_inv_image, "grad_cov_inv_image", f32, (n, 3), dev)
-    g_opac = _prep(grad_opacities, "grad_opacities", f32, (n,), dev)
-    g_col = _prep(grad_colors, "grad_colors", f32, (n, 3), dev)
+    grads = (_prep(grad_points_image, "grad_points_image", f32, (n, 2), dev),
+             _prep(grad_cov_inv_image, "grad_cov_inv_image", f32, (n, 3), dev),
+             _prep(grad_opacities, "grad_opacities", f32, (n,), dev),
+             _prep(grad_colors, "grad_colors", f32, (n, 3), dev))
+    return _preprocess_backward("gs_preprocess_backward", grads, means, log_scales, quats_raw,
+                                opacity_logits, sh_coeffs_dc, sh_coeffs_rest, cov_image, mask,
+                                world_to_camera, intrinsic, width, height, sh_cache)
+
+
+def preprocess_backward_rows(grad_rows, means, log_scales, quats_raw, opacity_logits,
+                             sh_coeffs_dc, sh_coeffs_rest, cov_image, mask, world_to_camera,
+                             intrinsic, width, height, sh_cache=None):
+    """preprocess_backward from (N, 9) rows of blend gradients
+    (rasterize_l1_backward_rows), read in place."""
+    dev = _device_of(means)
+    n = means.shape[0]
+    grads = (_prep(grad_rows, "grad_rows", torch.float32, (n, 9), dev),)
+    return _preprocess_backward("gs_preprocess_backward_rows", grads, means, log_scales,
+                                quats_raw, opacity_logits, sh_coeffs_dc, sh_coeffs_rest,
+                                cov_image, mask, world_to_camera, intrinsic, width, height,
+                                sh_cache)
+
+
+def _preprocess_backward(entry, grads, means, log_scales, quats_raw, opacity_logits,
+                         sh_coeffs_dc, sh_coeffs_rest, cov_image, mask, world_to_camera,
+                         intrinsic, width, height, sh_cache):
+    dev = means.device
+    n = means.shape[0]
+    f32 = torch.float32
     means = _prep(means, "means", f32, (n, 3), dev)
     log_scales = _prep(log_scales, "log_scales", f32, (n, 3), dev)
     quats_raw = _prep(quats_raw, "quats_raw", f32, (n, 4), dev)
@@ -1181,10 +1215,10 @@ def preprocess_backward(grad_points_image, grad_cov_inv_image, grad_opacities, g
             for shape in ((n, 3), (n, 3), (n, 4), (n,), (n, 3), (n, 15, 3))]
     with torch.cuda.device(dev):
         ev = _lib.timer.record("preprocess_backward", dev)
-        _lib.check(_lib.load().gs_preprocess_backward(
-            _ptr(g_pts), _ptr(g_conic), _ptr(g_opac), _ptr(g_col), _ptr(means), _ptr(log_scales),
-            _ptr(quats_raw), _ptr(opacity_logits), _ptr(dc), _ptr(rest), _ptr(cov_image),
-            _ptr(mask), _ptr(world_to_camera), _ptr(intrinsic), n, int(width), int(height),
+        _lib.check(getattr(_lib.load(), entry)(
+            *(_ptr(g) for g in grads), _ptr(means), _ptr(log_scales), _ptr(quats_raw),
+            _ptr(opacity_logits), _ptr(dc), _ptr(rest), _ptr(cov_image), _ptr(mask),
+            _ptr(world_to_camera), _ptr(intrinsic), n, int(width), int(height),
             *[_ptr(t) for t in outs], _ptr(sh_cache), _stream(dev)), "preprocess_backward")
         _lib.timer.stop(ev, dev)
     return tuple(outs)
@@ -1284,6 +1318,31 @@ def rasterize_display_l1(indexing_offset, gaussian_ids_sorted, points_image, cov
     return image, display, loss
 
 
+def _check_accumulators(accumulators, n, dev, who):
+    if (accumulators.dtype != torch.float32 or accumulators.device != dev
+            or accumulators.numel() != 9 * n or not accumulators.is_contiguous()):
+        raise RuntimeError(f"{who}: accumulators must be a contiguous fp32 "
+                           f"tensor of {9 * n} elements on {dev}")
+
+
+def _l1_backward_inputs(target, grad_loss, indexing_offset, gaussian_ids_sorted, points_image,
+                        cov_inv_image, opacities, colors, width, height, rendered_image,
+                        grad_display01, schedule):
+    blend = _blend_inputs(
+        indexing_offset, gaussian_ids_sorted, points_image, cov_inv_image, opacities, colors)
+    dev = blend[0]
+    width, height = int(width), int(height)
+    f32 = torch.float32
+    target = _prep(target, "target", f32, (height, width, 3), dev)
+    img = _prep(rendered_image, "rendered_image", f32, (height, width, 3), dev)
+    gl = _prep(grad_loss.reshape(1), "grad_loss", f32, (1,), dev)
+    extra = (None if grad_display01 is None
+             else _prep(grad_display01, "grad_display01", f32, (height, width, 3), dev))
+    if schedule is not None:
+        _check_schedule(schedule, blend[2].shape[0], dev, "rasterize_l1_backward")
+    return blend, target, img, gl, extra
+
+
 def rasterize_l1_backward(target, grad_loss, indexing_offset, gaussian_ids_sorted, points_image,
                           cov_inv_image, opacities, colors, width, height, rendered_image,
                           alpha_threshold=1e-4, transmittance_threshold=1e-4,
@@ -1297,25 +1356,18 @@ def rasterize_l1_backward(target, grad_loss, indexing_offset, gaussian_ids_sorte
     `loss_scale` weights the L1 term (1 - lambda in an L1 + SSIM loss).
     `schedule`: the tensor rasterize_display_l1 filled for the same layout (the
     tiles then start heaviest first; the gradients do not depend on it)."""
-    dev, n, off, ids, pts, conic, opac, col = _blend_inputs(
-        indexing_offset, gaussian_ids_sorted, points_image, cov_inv_image, opacities, colors)
+    blend, target, img, gl, extra = _l1_backward_inputs(
+        target, grad_loss, indexing_offset, gaussian_ids_sorted, points_image, cov_inv_image,
+        opacities, colors, width, height, rendered_image, grad_display01, schedule)
+    dev, n, off, ids, pts, conic, opac, col = blend
     width, height = int(width), int(height)
-    f32 = torch.float32
-    target = _prep(target, "target", f32, (height, width, 3), dev)
-    img = _prep(rendered_image, "rendered_image", f32, (height, width, 3), dev)
-    gl = _prep(grad_loss.reshape(1), "grad_loss", f32, (1,), dev)
-    extra = (None if grad_display01 is None
-             else _prep(grad_display01, "grad_display01", f32, (height, width, 3), dev))
     if accumulators is None:
-        g_pts, g_conic, g_opac, g_col = _zeroed_blend_grads(n, dev)
-    else:
-        if (accumulators.dtype != f32 or accumulators.device != dev
-                or accumulators.numel() != 9 * n or not accumulators.is_contiguous()):
-            raise RuntimeError("rasterize_l1_backward: accumulators must be a contiguous fp32 "
-                               f"tensor of {9 * n} elements on {dev}")
-        g_pts, g_conic, g_opac, g_col = _blend_grad_views(accumulators, n)
-    if schedule is not None:
-        _check_schedule(schedule, off.shape[0], dev, "rasterize_l1_backward")
+        return _backward_split("rasterize_l1_backward", _SEED_L1, target, blend, width, height,
+                               16, alpha_threshold, transmittance_threshold,
+                               chi_squared_threshold, img, grad_loss=gl, loss_scale=loss_scale,
+                               extra=extra, schedule=schedule)
+    _check_accumulators(accumulators, n, dev, "rasterize_l1_backward")
+    g_pts, g_conic, g_opac, g_col = _blend_grad_views(accumulators, n)
     with torch.cuda.device(dev):
         ev = _lib.timer.record("rasterize_l1_backward", dev)
         _lib.check(_lib.load().gs_rasterize_l1_backward(
@@ -1327,3 +1379,26 @@ def rasterize_l1_backward(target, grad_loss, indexing_offset, gaussian_ids_sorte
             "rasterize_l1_backward")
         _lib.timer.stop(ev, dev)
     return g_pts, g_conic, g_opac, g_col
+
+
+def rasterize_l1_backward_rows(target, grad_loss, indexing_offset, gaussian_ids_sorted,
+                               points_image, cov_inv_image, opacities, colors, width, height,
+                               rendered_image, alpha_threshold=1e-4, transmittance_threshold=1e-4,
+                               chi_squared_threshold=9.21, accumulators=None, grad_display01=None,
+                               loss_scale=1.0, schedule=None):
+    """rasterize_l1_backward with the gradients as one (N, 9) tensor of rows (du, dv, dA,
+    dB, dC, dopacity, dr, dg, db) for preprocess_backward_rows: a view of
+    `accumulators` (9N zeroed floats, added into) or of a new buffer."""
+    blend, target, img, gl, extra = _l1_backward_inputs(
+        target, grad_loss, indexing_offset, gaussian_ids_sorted, points_image, cov_inv_image,
+        opacities, colors, width, height, rendered_image, grad_display01, schedule)
+    dev, n = blend[0], blend[1]
+    if accumulators is None:
+        accumulators = torch.zeros((9 * n,), dtype=torch.float32, device=dev)
+    _check_accumulators(accumulators, n, dev, "rasterize_l1_backward_rows")
+    with torch.cuda.device(dev):
+        _backward_rows("rasterize_l1_backward", _SEED_L1, target, blend, int(width), int(height),
+                       16, alpha_threshold, transmittance_threshold, chi_squared_threshold, img,
+                       rows=accumulators, grad_loss=gl, loss_scale=loss_scale, extra=extra,
+                       schedule=schedule)
+    return accumulators.view(n, 9)

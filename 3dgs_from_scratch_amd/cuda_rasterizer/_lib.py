@@ -47,6 +47,10 @@ SIGNATURES = {
     "gs_preprocess_forward": [_P] * 8 + [_I64, _F, _F, _F, _F, _F, _I32, _I32] + [_P] * 9 + [_P],
     "gs_preprocess_backward": [_P] * 14 + [_I64, _I32, _I32] + [_P] * 7 + [_P],
     "gs_render_preprocess_backward": [_P] * 12 + [_I64, _I32, _I32] + [_P] * 6 + [_P],
+    "gs_preprocess_backward_rows": [_P] * 11 + [_I64, _I32, _I32] + [_P] * 7 + [_P],
+    "gs_rasterize_backward_rows": [_I32] + [_P] * 5 + [_I32, _I64] + [_P] * 4
+    + [_I64, _I32, _I32, _I32, _F, _F, _F, _P, _I32, _F, _P, _P, _P],
+    "gs_split_gradient_rows": [_P, _I64] + [_P] * 4 + [_P],
     "gs_activate_backward": [_P] * 6 + [_I64] + [_P] * 3 + [_P],
     "gs_rasterize_display_l1": [_P, _P, _I32, _I64] + [_P] * 4
     + [_I64, _I32, _I32, _I32, _F, _F, _F] + [_P] * 7 + [_I64, _P, _P],
@@ -83,6 +87,7 @@ SIGNATURES.update({
     "gs_adam_step": [ctypes.POINTER(GsAdamTensor), _I32, ctypes.c_double, ctypes.c_double,
                      ctypes.c_double, _P],
     "gs_accumulate_grad2d": [_P, _P, _I64, _I32, _I32, _P, _P, _P],
+    "gs_accumulate_grad2d_strided": [_P, _I32, _P, _I64, _I32, _I32, _P, _P, _P],
     "gs_gather_rows": [_I64, _P, _P, ctypes.POINTER(GsGatherTensor), _I32, _P],
     "gs_ssim_workspace_size": [_I32, _I32, _I32, _I32, _PSZ],
     "gs_ssim_forward": [_P] * 4 + [_I32] * 5 + [_F] + [_P] * 5 + [_F, _P, _P, _SZ, _P],

@@ -217,15 +217,15 @@ class RenderL1Function(torch.autograd.Function):
         # buffers, so it neither adds onto nor overwrites the first one's results
         accumulators = acc if ctx.acc_fresh else None
         ctx.acc_fresh = False
-        g_pts, g_conic, g_opac, g_col = _cr.rasterize_l1_backward(
+        rows = _cr.rasterize_l1_backward_rows(
             target, g, off, ids, pts, conic, opac, colors, width, height, image, a_thr, t_thr,
             chi, accumulators=accumulators, grad_display01=extra, loss_scale=1.0 - lam,
             schedule=sched)
         if ctx.densifier is not None:
-            ctx.densifier.update(g_pts, ctx.radii, width, height)
-        g_means, g_ls, g_qr, g_logit, g_dc, g_rest = _cr.preprocess_backward(
-            g_pts, g_conic, g_opac, g_col, means, log_scales, quats_raw, logits, dc, rest, cov,
-            mask, w2c, K, width, height, sh_cache=ctx.sh_cache)
+            ctx.densifier.update(rows[:, :2], ctx.radii, width, height)
+        g_means, g_ls, g_qr, g_logit, g_dc, g_rest = _cr.preprocess_backward_rows(
+            rows, means, log_scales, quats_raw, logits, dc, rest, cov, mask, w2c, K, width,
+            height, sh_cache=ctx.sh_cache)
         return (g_means, g_ls, g_qr, g_logit, g_dc, g_rest) + (None,) * 18
 
 

@@ -107,15 +107,18 @@ class Densifier:
         self.count = torch.zeros(n, device=device)
 
     def update(self, grad_points_image: torch.Tensor, radii: torch.Tensor, width: int, height: int):
-        """src/strategy.py:47-68 (gs_accumulate_grad2d)."""
+        """src/strategy.py:47-68 (gs_accumulate_grad2d_strided: rows of a wider tensor,
+        as the fused step's, are read in place)."""
         n = self.grads.shape[0]
-        g = grad_points_image.detach().contiguous()
+        g = grad_points_image.detach()
+        if g.dim() != 2 or g.stride(1) != 1 or not 2 <= g.stride(0) < 2**31:
+            g = g.contiguous()
+        stride = g.stride(0) if g.dim() == 2 else 2
         r = radii.detach().contiguous()
         with torch.cuda.device(g.device):
-            _lib.check(_lib.load().gs_accumulate_grad2d(_ptr(g), _ptr(r), n, int(width),
-                                                        int(height), _ptr(self.grads),
-                                                        _ptr(self.count), _stream(g)),
-                       "accumulate_grad2d")
+            _lib.check(_lib.load().gs_accumulate_grad2d_strided(
+                _ptr(g), stride, _ptr(r), n, int(width), int(height), _ptr(self.grads),
+                _ptr(self.count), _stream(g)), "accumulate_grad2d")
 
     # --------------------------------------------------------------- rebuild
     def _rebuild(self, params: dict, opt: FusedAdam | None, src_rows: torch.Tensor,

@@ -280,6 +280,32 @@ int gs_rasterize_backward(const float *grad_image, const float *image,
                           float *grad_opacities, float *grad_colors, int32_t accumulate,
                           hipStream_t stream);
 
+/*
+ * The backward of gs_rasterize (seed 0: grad is the gradient of image),
+ * gs_rasterize_display (1: of display; image required) or gs_rasterize_display_l1
+ * (2: grad is the target; grad_loss, loss_scale, grad_display01 and image as in
+ * gs_rasterize_l1_backward, ignored for the other seeds) with the gradients in one
+ * row of nine floats per Gaussian, (du, dv, dA, dB, dC, dopacity, dr, dg, db): an
+ * entry's nine atomics then share a memory line or two, which makes the kernel a
+ * quarter faster on large images than the four arrays of the entries above.
+ * accumulate and tile_schedule as there.  gs_split_gradient_rows copies the rows
+ * into the four arrays; gs_preprocess_backward_rows and
+ * gs_accumulate_grad2d_strided read them in place.
+ */
+int gs_rasterize_backward_rows(int32_t seed, const float *grad, const float *grad_loss,
+                               const float *image, const int32_t *indexing_offset,
+                               const int32_t *gaussian_ids_sorted, int32_t n_tiles, int64_t k,
+                               const float *points_image, const float *cov_inv_image,
+                               const float *opacities, const float *colors, int64_t n,
+                               int32_t width, int32_t height, int32_t tile_size,
+                               float alpha_threshold, float transmittance_threshold,
+                               float chi_squared_threshold, float *rows, int32_t accumulate,
+                               float loss_scale, const float *grad_display01,
+                               const int32_t *tile_schedule, hipStream_t stream);
+int gs_split_gradient_rows(const float *rows, int64_t n, float *grad_points_image,
+                           float *grad_cov_inv_image, float *grad_opacities, float *grad_colors,
+                           hipStream_t stream);
+
 /* ------------------------------------------------------- render() fusions */
 
 /*
@@ -393,6 +419,16 @@ int gs_preprocess_backward(const float *grad_points_image, const float *grad_cov
                            float *grad_log_scales, float *grad_quats_raw,
                            float *grad_opacity_logits, float *grad_sh_dc, float *grad_sh_rest,
                            const float *sh_cache, hipStream_t stream);
+
+/* gs_preprocess_backward reading rows of nine gradients (gs_rasterize_backward_rows). */
+int gs_preprocess_backward_rows(const float *rows, const float *means, const float *log_scales,
+                                const float *quats_raw, const float *opacity_logits,
+                                const float *sh_dc, const float *sh_rest, const float *cov_image,
+                                const uint8_t *mask, const float *world_to_camera,
+                                const float *intrinsic, int64_t n, int32_t width, int32_t height,
+                                float *grad_means, float *grad_log_scales, float *grad_quats_raw,
+                                float *grad_opacity_logits, float *grad_sh_dc,
+                                float *grad_sh_rest, const float *sh_cache, hipStream_t stream);
 
 /*
  * The drop-in render()'s backward of projection and colours in one pass:
@@ -526,6 +562,8 @@ int gs_tile_schedule_size(int32_t n_tiles, size_t *elements);
  *   formed in double and rounded once to float, as PyTorch does.
  * gs_accumulate_grad2d: src/strategy.py:47-68 -- for Gaussians whose two radii
  *   are > 0, grads += |(du * W/2, dv * H/2)| and count += 1.
+ *   gs_accumulate_grad2d_strided: du, dv of Gaussian i at grad_points_image[
+ *   row_stride * i] and the next (9: rows of gs_rasterize_backward_rows).
  * gs_gather_rows: dst row r = src row src_rows[r] (+ delta row r when delta is
  *   set) for every tensor of the list, or zeros where fresh_rows[r] != 0 and
  *   the tensor has zero_fresh (optimizer state of new Gaussians).  Rebuilds
@@ -554,6 +592,9 @@ int gs_adam_step(const GsAdamTensor *tensors, int32_t n_tensors, double beta1, d
 int gs_accumulate_grad2d(const float *grad_points_image, const float *radii, int64_t n,
                          int32_t width, int32_t height, float *grads, float *count,
                          hipStream_t stream);
+int gs_accumulate_grad2d_strided(const float *grad_points_image, int32_t row_stride,
+                                 const float *radii, int64_t n, int32_t width, int32_t height,
+                                 float *grads, float *count, hipStream_t stream);
 int gs_gather_rows(int64_t n_out, const int32_t *src_rows, const uint8_t *fresh_rows,
                    const GsGatherTensor *tensors, int32_t n_tensors, hipStream_t stream);
 

@@ -258,3 +258,45 @@ def test_rasterize_work_counts(gpu):
     assert v_ref > 0 and c_ref > 0
     # exp implementations differ in the last bits: an entry at the alpha threshold may flip
     assert abs(v - v_ref) <= 1e-4 * v_ref and abs(c - c_ref) <= 1e-4 * c_ref
+
+
+@pytest.mark.parametrize("opaque,t_thr", [(False, 1e-4), (True, 1e-4), (False, 0.0)])
+@pytest.mark.parametrize("count", [1, 3, 4, 5, 8, 63, 65, 130])
+def test_backward_pending_entries(gpu, waves, count, opaque, t_thr):
+    """The backward reduces four entries at a time: list lengths around multiples of
+    four and of a batch, also with pixels that an opacity of exactly 1 saturates
+    (alpha 1 at the splat's centre) and with no transmittance threshold.  The sums run
+    in float32 in another order than the oracle's: about sqrt(256) roundings of 6e-8
+    on terms of either sign, 1e-5 of the result here."""
+    W, H = 19, 17  # 2 x 2 tiles, three of them partial
+    g = torch.Generator().manual_seed(count)
+    pts = torch.rand(count, 2, generator=g) * torch.tensor([W - 1.0, H - 1.0])
+    if opaque:
+        pts = pts.round()
+    scale = torch.rand(count, generator=g) * 0.2 + 0.02
+    conic = torch.stack([scale, 0.3 * scale, 1.5 * scale], dim=1)
+    opac = torch.rand(count, generator=g) * 0.8 + 0.1
+    if opaque:
+        opac[count // 2] = 1.0
+    col = torch.rand(count, 3, generator=g)
+    ids = torch.arange(count, dtype=torch.int32).repeat(4)
+    off = torch.arange(4, dtype=torch.int32) * count
+    args = (W, H, 16, 1e-4, t_thr, 9.21)
+    ins = [t.clone().requires_grad_(True) for t in (pts, conic, opac, col)]
+    image = blend.rasterize(off, ids, *ins, *args)
+    up = torch.randn(H, W, 3, generator=g)
+    (image * up).sum().backward()
+    d = [t.to(gpu) for t in (pts, conic, opac, col)]
+    img = cr.rasterize(off.to(gpu), ids.to(gpu), *d, *args)
+    assert helpers.max_abs(img, image) <= 1e-5
+    got = cr.rasterize_backward(up.to(gpu), off.to(gpu), ids.to(gpu), *d, *args,
+                                rendered_image=img)
+    for nm, a, t in zip(INPUTS, got, ins):
+        assert a.is_contiguous() and helpers.rel_l2(a, t.grad) <= 1e-4, nm
+    # the rows and the four arrays of the L1 seed hold the same sums (atomics in any order)
+    target, one = torch.rand(H, W, 3, generator=g).to(gpu), torch.ones(1, device=gpu)
+    l1 = (target, one, off.to(gpu), ids.to(gpu), *d, W, H, img, 1e-4, t_thr, 9.21)
+    want = cr.rasterize_l1_backward(*l1, accumulators=torch.zeros(9 * count, device=gpu))
+    rows = cr.rasterize_l1_backward_rows(*l1)
+    for nm, a, b in zip(INPUTS, want, (rows[:, :2], rows[:, 2:5], rows[:, 5], rows[:, 6:])):
+        assert helpers.rel_l2(b, a) <= 1e-5, nm
