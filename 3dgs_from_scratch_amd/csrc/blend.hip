@@ -1,17 +1,17 @@
 // Tile blending: front-to-back alpha compositing and its gradient.
 //
-// One wave64 per 16x16 tile (on grids of at most 1024 tiles, 4 waves per tile:
-// see blend_waves).  Lane l owns the four pixels (x0 + l%16, y0 + l/16 + 4s),
-// s = 0..3, i.e. one pixel in each 16x4 strip of the tile (with W waves per
-// tile, wave w's lanes own strips w*4/W .. and the waves share the staging).  The tile's depth-sorted Gaussian list is walked in batches of 64
-// Gaussians (one per lane); at staging each lane computes which strips the
-// Gaussian's chi-square / alpha ellipse reaches, and only Gaussians reaching
-// the tile are written to LDS (ballot compaction, list order kept) with that
-// strip mask and log2 of the opacity (alpha = exp2(E * -log2(e)/2 + log2 o)).
-// The wave evaluates only those strips, and it stops once the
-// transmittance of all 256 pixels fell below the threshold.  Tiles are assigned to workgroups XCD by XCD (the dispatcher
-// places workgroup b on XCD b % 8) so that neighbouring tiles, which share
-// Gaussians, run on the same XCD and share its L2.
+// One, two or four wave64 per 16x16 tile (see blend_waves).  With one, lane l owns
+// the four pixels (x0 + l%16, y0 + l/16 + 4s), s = 0..3, i.e. one pixel in each 16x4
+// strip of the tile; with W, wave w's lanes own strips w*4/W .. and the waves share
+// the staging.  The tile's depth-sorted Gaussian list is walked in batches of 64 W
+// (one per thread); at staging each lane computes which strips the Gaussian's
+// chi-square / alpha ellipse reaches, writes the records that reach the tile to its
+// LDS slot with log2 of the opacity (alpha = exp2(E * -log2(e)/2 + log2 o)), and the
+// strips' ballots tell the waves which slots to visit, in list order.  A wave stops
+// once the transmittance of its pixels fell below the threshold, the tile once all
+// have.  Tiles are assigned to workgroups XCD by XCD (the dispatcher places workgroup
+// b on XCD b % 8) so that neighbouring tiles, which share Gaussians, run on the same
+// XCD and share its L2.
 //
 // In the forward, the exponent E and the transmittance T are computed with
 // separately rounded ops in the Torch rasterizer's order
@@ -46,11 +46,14 @@ constexpr int kGradFields = 9;   // du, dv, dA, dB, dC, dopacity, dr, dg, db
 constexpr int kXcds = 8;
 
 // Work units of a tile's walk, counted by the forward and used to launch the
-// backward's tiles heaviest first: per staged batch, per staged record (its
-// staging and, for nearly all of them, the backward's wave sum and atomics) and
-// per evaluated strip, in proportion to the backward's instructions for each.
+// backward's tiles heaviest first: per staged batch, per staged record and per strip
+// of an entry that it evaluates.  A strip takes the backward about 85 cycles and its
+// share of the entry's sums 20, staging a batch 400; a staged record costs only where
+// the walk still reaches it, so it counts little: with 11, 5 and 2 units per record
+// the backward took 126, 126 and 111 us at 200k Gaussians, 1280x720, and 127, 119 and
+// 112 us at 100k, 800x800 (other sizes the same within 3%).
 constexpr uint32_t kCostBatch = 33;
-constexpr uint32_t kCostStaged = 11;
+constexpr uint32_t kCostStaged = 2;
 constexpr uint32_t kCostStrip = 6;
 
 struct TileSpan {
@@ -72,7 +75,7 @@ __device__ __forceinline__ TileSpan tile_span(const int32_t *__restrict__ offset
 
 // Checkpoints of the forward walk, which let the backward walk a long tile list
 // in up to kCheckpoints + 1 segments on as many workgroups.  Every
-// checkpoint_spacing<W>() batches (at most kCheckpoints times) the forward
+// kCheckpointSpacing list entries (at most kCheckpoints times) the forward
 // saves each pixel's transmittance and accumulated colour before the batch at
 // list position pos, where the next segment starts.  A segment's backward walk
 // starts from that state: T from the checkpoint and the running colour-gradient
@@ -93,10 +96,9 @@ constexpr int kSegments = kCheckpoints + 1;
 constexpr int kCheckpointMaxTiles = 6144;
 constexpr int kTilePixels = 256;  // 16 x 16
 
-template <int W>
-__device__ __forceinline__ constexpr int checkpoint_spacing() {
-    return W == 1 ? 2 : 1;  // batches of W * kBatch records: 128 records with one wave
-}
+// Records between checkpoints: two batches with one wave, a batch with two, half a
+// batch with four.
+constexpr int kCheckpointSpacing = 128;
 
 struct Checkpoints {
     float *data;      // [n_tiles * kCheckpoints][4][kTilePixels]: T, r, g, b planes
@@ -182,19 +184,22 @@ __device__ __forceinline__ float conic_exponent(float A, float B2, float C, floa
 // alpha = o exp(-E/2) = exp2(E * kNegHalfLog2e + log2(o)): one fma and one
 // v_exp_f32 per (entry, pixel).
 constexpr float kNegHalfLog2e = -0.72134752044448170f;
-// One batch of staged records of a tile worked by W waves (W * kBatch records).
+// One batch of staged records of a tile worked by W waves: W * kBatch slots, one
+// per thread of the workgroup, and a last one that composites nothing.  mask[q][g]
+// has a bit for each slot of group g (the 64 that wave g stages) whose record
+// reaches strip q: the walks iterate those bits in scalar registers, in list order,
+// so that no record is compacted and no strip mask is read back from LDS.
 template <int W>
 struct BatchLds {
-    float4 geo[kBatch * W];  // u, v, A, 2B
-    float4 aux[kBatch * W];  // C, E cut-off (chi_eff), strip mask, log2(opacity)
-    float4 col[kBatch * W];  // r, g, b, (gaussian id bits)
-    float inv_o[kBatch * W];  // 1 / opacity (staged by the backward for its opacity gradient)
-    float o_raw[kBatch * W];  // the opacity of a record whose log2 is not finite (see below)
-    int wave_count[W];        // W > 1: records each wave stages, and whether one is
-    int wave_bad[W];          //   non-finite (the batch then takes the select-based path)
+    float4 geo[kBatch * W + 1];  // u, v, A, 2B
+    float4 aux[kBatch * W + 1];  // C, E cut-off (chi_eff), log2(opacity), r
+    float4 col[kBatch * W + 1];  // g, b, gaussian id bits, 1 / opacity (see staged_opacity)
+    uint64_t mask[kStrips][W];   // W > 1: the waves' strip ballots
+    int wave_bad[W];          // W > 1: whether a wave stages a non-finite record (the batch
+                              //   then takes the select-based path)
     int wave_flag[W];         // W > 1: per-wave votes of the batch loops (tile_any)
     int wave_flag_once[W];    // W > 1: the backward's one vote before its loop
-    uint32_t wave_work[W];    // W > 1: each wave's work so far, summed at a checkpoint
+    uint32_t wave_work[W];    // each wave's work before a checkpoint, to be summed
 };
 
 // Entries whose lane sums wait in LDS for one reduction (backward_flush): per
@@ -216,7 +221,7 @@ struct BackwardLds {
 // staged only when the alpha test can pass them: with alpha_thr > 0 an opacity
 // <= 0 has the cut-off -inf.  Their opacity gradient is sum G dalpha
 // (G = exp(-E/2)); the h / o form of the other records would give 0 * inf at
-// o = 0, so the backward stages 1 for their 1 / o.
+// o = 0, so theirs is added apart (backward_entry_safe).
 __device__ __forceinline__ bool special_opacity(float log2o) { return !isfinite(log2o); }
 
 // log2(o) for the exponent form of alpha; -inf when o <= 0 and NaN for a NaN
@@ -318,22 +323,45 @@ __device__ __forceinline__ uint32_t exact_strip_mask(uint32_t box, float u, floa
     return m;
 }
 
-// Result of staging one batch: the number of staged records, and whether one
-// of them has a non-finite colour (the batch then takes the select-based path).
+// The staged batch as one wave sees it: for each strip of the wave and each group
+// of 64 slots, the slots whose record reaches the strip; how many records the wave
+// itself staged; and whether some record of the batch needs the select-based path.
+template <int W>
 struct Staged {
+    uint64_t mask[kStrips / W][W];
     int count;
     bool nonfinite;
 };
 
-// Stages the thread's record into the next free LDS slot if its ellipse (with
-// the chi-square and alpha cut-offs) reaches the tile, keeping thread (= list)
-// order, with its E cut-off (effective_chi) in aux.y, its strip mask (all four
-// strips of the tile) in aux.z and log2 of its opacity in aux.w.  With W > 1
-// waves, wave w's records follow those of waves 0..w-1 (one more barrier).
+// The wave's index within its tile's workgroup, as a wave-uniform value.
+__device__ __forceinline__ int tile_wave() {
+    return __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+}
+
+__device__ __forceinline__ uint64_t uniform64(uint64_t x) {
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)x);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));
+    return ((uint64_t)hi << 32) | lo;
+}
+
+// Fills the slot past the batch: a record that no pixel composites.
+template <int W>
+__device__ __forceinline__ void stage_none(BatchLds<W> &s) {
+    if (threadIdx.x == 0) {
+        s.geo[kBatch * W] = make_float4(0.f, 0.f, 0.f, 0.f);
+        s.aux[kBatch * W] = make_float4(0.f, -1.0f, 0.f, 0.f);
+        s.col[kBatch * W] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+}
+
+// Stages the thread's record into its LDS slot if its ellipse (with the chi-square
+// and alpha cut-offs) reaches the tile, with its E cut-off (effective_chi) in aux.y
+// and log2 of its opacity in aux.z; the strips it reaches go to the ballots.  col.w
+// holds 1 / opacity (kInvO, the backward) or, for a special opacity, the opacity.
 template <bool kInvO, int W>
-__device__ __forceinline__ Staged stage_records(BatchLds<W> &s, const Record &r, float chi,
-                                                float alpha_thr, float log2_alpha_thr, float x0,
-                                                float y0) {
+__device__ __forceinline__ Staged<W> stage_records(BatchLds<W> &s, const Record &r, float chi,
+                                                   float alpha_thr, float log2_alpha_thr,
+                                                   float x0, float y0) {
     uint32_t m = 0u;
     const float log2o = log2_opacity(r.o);
     const float chi_eff = effective_chi(log2o, chi, alpha_thr, log2_alpha_thr);
@@ -343,42 +371,43 @@ __device__ __forceinline__ Staged stage_records(BatchLds<W> &s, const Record &r,
         m = exact_strip_mask(strip_mask(r.u, r.v, ex, ey, x0, y0), r.u, r.v, r.A, r.B, r.C,
                              chi_eff, x0, y0);
     }
-    const uint64_t keep = __ballot(m != 0u);
     // a non-finite colour or log2 opacity (o <= 0, +inf or NaN): the batch takes
     // the select-based path (the only one that handles such opacities)
     const bool bad = m != 0u && !(isfinite(r.r) && isfinite(r.g) && isfinite(r.b) &&
                                   isfinite(log2o));
-    Staged st;
-    int first = 0;  // this wave's first slot
+    if (m != 0u) {
+        const int slot = (int)threadIdx.x;
+        s.geo[slot] = make_float4(r.u, r.v, r.A, r.B + r.B);
+        s.aux[slot] = make_float4(r.C, chi_eff, log2o, r.r);
+        const float o = kInvO && !special_opacity(log2o) ? __builtin_amdgcn_rcpf(r.o) : r.o;
+        s.col[slot] = make_float4(r.g, r.b, __int_as_float(r.id), o);
+    }
+    Staged<W> st;
+    st.count = __popcll(__ballot(m != 0u));
     if constexpr (W == 1) {
-        st.count = __popcll(keep);
+#pragma unroll
+        for (int q = 0; q < kStrips; ++q) st.mask[q][0] = __ballot(((m >> q) & 1u) != 0u);
         st.nonfinite = __ballot(bad) != 0;
-    } else {
-        const int wave = threadIdx.x / kWave;
-        const bool wave_bad = __ballot(bad) != 0;
-        if (threadIdx.x % kWave == 0) {
-            s.wave_count[wave] = __popcll(keep);
-            s.wave_bad[wave] = wave_bad ? 1 : 0;
-        }
         __syncthreads();
-        st.count = 0;
+    } else {
+        constexpr int S = kStrips / W;
+        const int wave = tile_wave();
+        const bool wave_bad = __ballot(bad) != 0;
+#pragma unroll
+        for (int q = 0; q < kStrips; ++q) {
+            const uint64_t b = __ballot(((m >> q) & 1u) != 0u);
+            if (threadIdx.x % kWave == 0) s.mask[q][wave] = b;
+        }
+        if (threadIdx.x % kWave == 0) s.wave_bad[wave] = wave_bad ? 1 : 0;
+        __syncthreads();
         st.nonfinite = false;
 #pragma unroll
-        for (int w = 0; w < W; ++w) {
-            const int c = s.wave_count[w];
-            first += w < wave ? c : 0;
-            st.count += c;
-            st.nonfinite = st.nonfinite || s.wave_bad[w] != 0;
+        for (int g = 0; g < W; ++g) {
+            st.nonfinite = st.nonfinite || s.wave_bad[g] != 0;
+#pragma unroll
+            for (int q = 0; q < S; ++q) st.mask[q][g] = uniform64(s.mask[wave * S + q][g]);
         }
-    }
-    if (m != 0u) {
-        const int slot = first + __popcll(keep & lanemask_lt());
-        s.geo[slot] = make_float4(r.u, r.v, r.A, r.B + r.B);
-        s.aux[slot] = make_float4(r.C, chi_eff, __uint_as_float(m), log2o);
-        s.col[slot] = make_float4(r.r, r.g, r.b, __int_as_float(r.id));
-        const bool special = special_opacity(log2o);
-        if (kInvO) s.inv_o[slot] = special ? 0.0f : __builtin_amdgcn_rcpf(r.o);
-        if (special) s.o_raw[slot] = r.o;
+        st.nonfinite = __builtin_amdgcn_readfirstlane((int)st.nonfinite) != 0;
     }
     return st;
 }
@@ -393,25 +422,26 @@ template <bool kInvO, int W = 1>
 struct BatchPipe {
     int32_t next_id;  // this thread's id in the next batch to stage
 
-    __device__ __forceinline__ void start(TileSpan span, const int32_t *__restrict__ ids) {
+    __device__ __forceinline__ void start(BatchLds<W> &s, TileSpan span,
+                                          const int32_t *__restrict__ ids) {
+        stage_none<W>(s);
         next_id = fetch_id(span.start + (int32_t)threadIdx.x, span.end, ids);
     }
 
     // Stages the batch starting at b0 (only records reaching the tile) and
     // fetches ahead.
-    __device__ __forceinline__ Staged advance(BatchLds<W> &s, int32_t b0, TileSpan span,
-                                           const int32_t *__restrict__ ids, int64_t n,
-                                           const float *__restrict__ points,
-                                           const float *__restrict__ conics,
-                                           const float *__restrict__ opac,
-                                           const float *__restrict__ colors, float chi,
-                                           float alpha_thr, float x0, float y0) {
+    __device__ __forceinline__ Staged<W> advance(BatchLds<W> &s, int32_t b0, TileSpan span,
+                                              const int32_t *__restrict__ ids, int64_t n,
+                                              const float *__restrict__ points,
+                                              const float *__restrict__ conics,
+                                              const float *__restrict__ opac,
+                                              const float *__restrict__ colors, float chi,
+                                              float alpha_thr, float x0, float y0) {
         const Record rec = fetch_record(next_id, n, points, conics, opac, colors);
         __syncthreads();  // previous batch fully read before restaging
-        const Staged st =
+        const Staged<W> st =
             stage_records<kInvO, W>(s, rec, chi, alpha_thr, __builtin_amdgcn_logf(alpha_thr), x0,
                                     y0);
-        __syncthreads();
         next_id = fetch_id(b0 + kBatch * W + (int32_t)threadIdx.x, span.end, ids);
         return st;
     }
@@ -426,11 +456,6 @@ struct LanePixels {
     float x0, y0;   // tile origin
     bool inside[S];
 };
-
-// The wave's index within its tile's workgroup, as a wave-uniform value.
-__device__ __forceinline__ int tile_wave() {
-    return __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
-}
 
 template <int W>
 __device__ __forceinline__ LanePixels<kStrips / W> lane_pixels(int tile, int tiles_x, int width,
@@ -508,79 +533,224 @@ __device__ __forceinline__ bool tile_any(bool v, int *flag) {
     }
 }
 
-// One staged entry j applied to the lane's four pixels.  Branch-free per
-// strip: an entry that fails the chi-square or alpha test gets weight 0, so
-// C += 0 * c and T -= 0 leave the pixel unchanged; kSafe (a non-finite colour
-// in the batch, where 0 * inf would not be 0) uses selects instead.
-// T_{i+1} = T_i - alpha T_i, i.e. T_i (1 - alpha): the 1e-10 of the
-// reference's 1 - alpha + 1e-10 is below the float resolution of that factor
-// unless alpha is within 1e-7 of 1, where T drops below any threshold either way.
-// With W waves per tile, the entry is applied to the wave's own S strips only
-// (and skipped when its strip mask misses them).
-template <bool kSafe, int W>
-__device__ __forceinline__ void blend_entry(const BatchLds<W> &s, int j,
-                                            const LanePixels<kStrips / W> &pix, float alpha_thr,
-                                            float T_thr, float chi, float (&T)[kStrips / W],
-                                            float (&cr)[kStrips / W], float (&cg)[kStrips / W],
-                                            float (&cb)[kStrips / W], uint32_t &work) {
-    constexpr int S = kStrips / W;
-    const float4 aux = s.aux[j];
-    uint32_t smask = __builtin_amdgcn_readfirstlane(__float_as_uint(aux.z));
-    if constexpr (W > 1) {
-        smask = (smask >> (tile_wave() * S)) & ((1u << S) - 1u);
-        if (smask == 0u) return;  // uniform: none of this wave's strips
+// Active pixels of the wave's strips, a lane mask per strip: !(T < T_thr), so a NaN
+// T stays active.
+template <int S>
+__device__ __forceinline__ uint64_t active_masks(const float (&T)[S], float T_thr,
+                                                 uint64_t (&act)[S]) {
+    uint64_t any = 0;
+#pragma unroll
+    for (int q = 0; q < S; ++q) {
+        act[q] = __ballot(!(T[q] < T_thr));
+        any |= act[q];
     }
-    const float4 geo = s.geo[j];
-    const float4 col = s.col[j];
-    // uniform: a record with a non-finite log2 opacity (only in the select-based path)
-    const bool special =
-        kSafe && special_opacity(__uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(aux.w))));
-    const float o_sp = special ? s.o_raw[j] : 0.0f;
+    return any;
+}
+
+// The forward's state of a lane's pixels.
+template <int S>
+struct ForwardLane {
+    float T[S], cr[S], cg[S], cb[S];
+};
+
+// The staged entry in `slot` applied to the lane's pixels, the strips where no pixel
+// takes it skipped.  Without branches per pixel: an entry that fails the chi-square or
+// alpha test gets weight 0, so C += 0 * c and T -= 0 leave the pixel unchanged.
+// T_{i+1} = T_i - alpha T_i, i.e. T_i (1 - alpha): the 1e-10 of the reference's
+// 1 - alpha + 1e-10 is below the float resolution of that factor unless alpha is
+// within 1e-7 of 1, where T drops below any threshold either way.
+template <int W>
+__device__ __forceinline__ void blend_entry(const BatchLds<W> &s, int slot,
+                                            const LanePixels<kStrips / W> &pix, float T_thr,
+                                            ForwardLane<kStrips / W> &L,
+                                            uint64_t (&act)[kStrips / W], uint32_t &work) {
+    constexpr int S = kStrips / W;
+    const float4 aux = s.aux[slot];
+    const float4 geo = s.geo[slot];
+    const float2 gb = *reinterpret_cast<const float2 *>(&s.col[slot]);
     const float du = pix.fx - geo.x;
     const float Adudu = (geo.z * du) * du;  // (A du) du, as in the oracle's A*du*du
     const float B2du = geo.w * du;
+    float E[S];
+    uint64_t inc[S], any = 0;
 #pragma unroll
     for (int q = 0; q < S; ++q) {
-        if (!((smask >> q) & 1u)) continue;  // uniform
+        const float dv = pix.fy[q] - geo.y;
+        E[q] = (Adudu + B2du * dv) + (aux.x * dv) * dv;
+        inc[q] = __ballot(E[q] < aux.y) & act[q];
+        any |= inc[q];
+    }
+    if (any == 0) return;
+#pragma unroll
+    for (int q = 0; q < S; ++q) {
+        if (inc[q] == 0) continue;
+        work += kCostStrip;
+        const float alpha = alpha_of(E[q], aux.z);
+        const float w = (__builtin_amdgcn_inverse_ballot_w64(inc[q]) ? alpha : 0.0f) * L.T[q];
+        L.cr[q] = fmaf(w, aux.w, L.cr[q]);
+        L.cg[q] = fmaf(w, gb.x, L.cg[q]);
+        L.cb[q] = fmaf(w, gb.y, L.cb[q]);
+        L.T[q] = L.T[q] - w;
+        act[q] = __ballot(!(L.T[q] < T_thr));
+    }
+}
+
+// blend_entry for any input, with selects in place of zero weights: a non-finite
+// colour (0 * inf would not be 0) or a special opacity, whose alpha = o exp(-E/2)
+// comes from the raw opacity with the alpha test on its value.
+template <int W>
+__device__ __forceinline__ void blend_entry_safe(const BatchLds<W> &s, int slot, uint32_t bits,
+                                                 const LanePixels<kStrips / W> &pix,
+                                                 float alpha_thr, float T_thr,
+                                                 ForwardLane<kStrips / W> &L, uint32_t &work) {
+    constexpr int S = kStrips / W;
+    const float4 aux = s.aux[slot];
+    const float4 geo = s.geo[slot];
+    const float4 col = s.col[slot];
+    const bool special = special_opacity(
+        __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(aux.z))));
+    const float du = pix.fx - geo.x;
+    const float Adudu = (geo.z * du) * du;
+    const float B2du = geo.w * du;
+#pragma unroll
+    for (int q = 0; q < S; ++q) {
+        if (!((bits >> q) & 1u)) continue;  // uniform
         const float dv = pix.fy[q] - geo.y;
         const float E = (Adudu + B2du * dv) + (aux.x * dv) * dv;
-        // the chi-square and alpha tests as one cut-off on E (staged in aux.y)
-        bool inc = !(T[q] < T_thr) && (E < aux.y);
+        bool inc = !(L.T[q] < T_thr) && (E < aux.y);
         float alpha = 0.0f;
-        if (special) {  // alpha = o exp(-E/2) from the raw opacity, alpha test on its value
-            alpha = o_sp * __builtin_amdgcn_exp2f(E * kNegHalfLog2e);
+        if (special) {
+            alpha = col.w * __builtin_amdgcn_exp2f(E * kNegHalfLog2e);
             inc = inc && !(alpha < alpha_thr);
         }
         if (!wave_any(inc)) continue;
         work += kCostStrip;
-        if (!special) alpha = alpha_of(E, aux.w);
-        if (kSafe) {
-            const float w = alpha * T[q];
-            cr[q] = inc ? fmaf(w, col.x, cr[q]) : cr[q];
-            cg[q] = inc ? fmaf(w, col.y, cg[q]) : cg[q];
-            cb[q] = inc ? fmaf(w, col.z, cb[q]) : cb[q];
-            T[q] = inc ? T[q] - w : T[q];
-        } else {
-            const float w = (inc ? alpha : 0.0f) * T[q];
-            cr[q] = fmaf(w, col.x, cr[q]);
-            cg[q] = fmaf(w, col.y, cg[q]);
-            cb[q] = fmaf(w, col.z, cb[q]);
-            T[q] = T[q] - w;
+        if (!special) alpha = alpha_of(E, aux.z);
+        const float w = alpha * L.T[q];
+        L.cr[q] = inc ? fmaf(w, aux.w, L.cr[q]) : L.cr[q];
+        L.cg[q] = inc ? fmaf(w, col.x, L.cg[q]) : L.cg[q];
+        L.cb[q] = inc ? fmaf(w, col.y, L.cb[q]) : L.cb[q];
+        L.T[q] = inc ? L.T[q] - w : L.T[q];
+    }
+}
+
+constexpr int kGroup = 4;
+
+// The next entries of a wave's list that reach its strips (bits of `m`, past its end
+// the slot that composites nothing), kGroup at a time.  Their records are loaded and
+// their alphas formed together, without branches, over all the wave's strips: only T
+// runs from entry to entry (a product, a difference and a select, which keeps a
+// finished pixel's T at 0).  A walk's length is its instructions' latencies where few
+// waves share a SIMD: entry by entry, 20k Gaussians at 251x183 (192 tiles) spent about
+// 380 cycles on each, 118 us in all, in groups 45 us.
+template <int W>
+__device__ __forceinline__ void blend_group(const BatchLds<W> &s, int base, uint64_t &m,
+                                            const LanePixels<kStrips / W> &pix, float T_thr,
+                                            ForwardLane<kStrips / W> &L,
+                                            uint64_t (&act)[kStrips / W]) {
+    constexpr int S = kStrips / W;
+    float4 aux[kGroup], geo[kGroup];
+    float2 gb[kGroup];
+#pragma unroll
+    for (int i = 0; i < kGroup; ++i) {
+        const int slot = (i == 0 || m != 0) ? base + __builtin_ctzll(m) : kBatch * W;
+        m &= m - 1;  // 0 stays 0
+        aux[i] = s.aux[slot];
+        geo[i] = s.geo[slot];
+        gb[i] = *reinterpret_cast<const float2 *>(&s.col[slot]);
+    }
+    float alpha[kGroup][S];
+#pragma unroll
+    for (int i = 0; i < kGroup; ++i) {
+        const float du = pix.fx - geo[i].x;
+        const float Adudu = (geo[i].z * du) * du;  // (A du) du, as in the oracle's A*du*du
+        const float B2du = geo[i].w * du;
+#pragma unroll
+        for (int q = 0; q < S; ++q) {
+            const float dv = pix.fy[q] - geo[i].y;
+            const float E = (Adudu + B2du * dv) + (aux[i].x * dv) * dv;
+            const float a = alpha_of(E, aux[i].z);
+            alpha[i][q] = E < aux[i].y ? a : 0.0f;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < kGroup; ++i) {
+#pragma unroll
+        for (int q = 0; q < S; ++q) {
+            const float w = alpha[i][q] * L.T[q];
+            L.cr[q] = fmaf(w, aux[i].w, L.cr[q]);
+            L.cg[q] = fmaf(w, gb[i].x, L.cg[q]);
+            L.cb[q] = fmaf(w, gb[i].y, L.cb[q]);
+            const float T = L.T[q] - w;
+            act[q] = __ballot(!(T < T_thr));
+            L.T[q] = __builtin_amdgcn_inverse_ballot_w64(act[q]) ? T : 0.0f;
         }
     }
 }
 
-template <bool kSafe, int W>
-__device__ __forceinline__ void blend_batch(const BatchLds<W> &s, int cnt,
+// Passes the pixels' state through an opaque operation, so that the compiler keeps
+// one copy of it in registers: with W = 1 it kept two of the colours, 80 registers and
+// a spill (160 against 138 us at 1M Gaussians, 1920x1080).
+template <int S>
+__device__ __forceinline__ void pin_state(ForwardLane<S> &L) {
+#pragma unroll
+    for (int q = 0; q < S; ++q)
+        asm volatile("" : "+v"(L.T[q]), "+v"(L.cr[q]), "+v"(L.cg[q]), "+v"(L.cb[q]));
+}
+
+// One exit per loop (the bits left are cleared when the wave's pixels are done):
+// returns from inside would keep two copies of the pixels' state in registers.
+// Applies the batch's groups G0 .. G1 - 1.
+template <bool kSafe, int W, int G0, int G1>
+__device__ __forceinline__ void blend_batch(const BatchLds<W> &s, const Staged<W> &st,
                                             const LanePixels<kStrips / W> &pix, float alpha_thr,
-                                            float T_thr, float chi, float (&T)[kStrips / W],
-                                            float (&cr)[kStrips / W], float (&cg)[kStrips / W],
-                                            float (&cb)[kStrips / W], uint32_t &work) {
-    if (W > 1 && !any_active(T, T_thr)) return;  // this wave's pixels are done
-    for (int j = 0; j < cnt; ++j) {
-        blend_entry<kSafe, W>(s, j, pix, alpha_thr, T_thr, chi, T, cr, cg, cb, work);
-        if ((j & 7) == 7 && !any_active(T, T_thr)) break;
+                                            float T_thr, ForwardLane<kStrips / W> &L,
+                                            uint32_t &work) {
+    constexpr int S = kStrips / W;
+    uint64_t act[S];
+    uint64_t left = active_masks(L.T, T_thr, act);
+    pin_state(L);
+#pragma unroll
+    for (int g = G0; g < G1; ++g) {
+        uint64_t any = 0;
+#pragma unroll
+        for (int q = 0; q < S; ++q) any |= st.mask[q][g];
+        if (left == 0) any = 0;
+        if constexpr (!kSafe && W > 1) {
+            while (any != 0) {
+                const uint32_t before = (uint32_t)__popcll(any);
+                blend_group<W>(s, g * kBatch, any, pix, T_thr, L, act);
+                const uint32_t cost = kCostStrip * (before - (uint32_t)__popcll(any));
+                left = 0;
+#pragma unroll
+                for (int q = 0; q < S; ++q) {
+                    work += act[q] != 0 ? cost : 0;
+                    left |= act[q];
+                }
+                if (left == 0) any = 0;
+            }
+        } else {
+            while (any != 0) {
+                const int j = __builtin_ctzll(any);
+                any &= any - 1;
+                if constexpr (kSafe) {
+                    uint32_t bits = 0;
+#pragma unroll
+                    for (int q = 0; q < S; ++q)
+                        bits |= (uint32_t)((st.mask[q][g] >> j) & 1u) << q;
+                    blend_entry_safe<W>(s, g * kBatch + j, bits, pix, alpha_thr, T_thr, L, work);
+                    left = active_masks(L.T, T_thr, act);
+                } else {
+                    blend_entry<W>(s, g * kBatch + j, pix, T_thr, L, act, work);
+                    left = 0;
+#pragma unroll
+                    for (int q = 0; q < S; ++q) left |= act[q];
+                }
+                if (left == 0) any = 0;
+            }
+        }
     }
+    pin_state(L);
 }
 
 // Transmittance of a pixel that takes no part (outside the image, or a zero
@@ -594,16 +764,14 @@ __device__ __forceinline__ float effective_T_thr(float T_thr) { return fmaxf(T_t
 // Front-to-back accumulation of the lane's pixels over the tile's list, the
 // tile's W waves sharing each staged batch of W * kBatch records.  Every thread
 // of the workgroup must call it (it contains barriers).  `work` counts the
-// wave's own strips and, in wave 0 only, the batches and staged records.
+// wave's own strips and staged records and, in wave 0 only, the batches.
 // The lane's pixels of checkpoint i of `tile` (local pixel lane + 64 * strip):
 // each strip's 64 lanes store 1 KB contiguously.
 template <int W>
-__device__ __forceinline__ void save_checkpoint(const Checkpoints &ck, int tile, int i,
+__device__ __forceinline__ void save_checkpoint(BatchLds<W> &s, const Checkpoints &ck, int tile,
+                                                int i,
                                                 int32_t pos, uint32_t work,
-                                                const float (&T)[kStrips / W],
-                                                const float (&cr)[kStrips / W],
-                                                const float (&cg)[kStrips / W],
-                                                const float (&cb)[kStrips / W]) {
+                                                const ForwardLane<kStrips / W> &L) {
     constexpr int S = kStrips / W;
     // the slot is uniform: a scalar base plus the lane's 32-bit offset
     const int slot = __builtin_amdgcn_readfirstlane(tile * kCheckpoints + i);
@@ -613,15 +781,25 @@ __device__ __forceinline__ void save_checkpoint(const Checkpoints &ck, int tile,
 #pragma unroll
     for (int q = 0; q < S; ++q) {  // four planes: no packing of the values into quads
         const uint32_t p = lane + (uint32_t)(kWave * (q0 + q));
-        dst[p] = T[q];
-        dst[kTilePixels + p] = cr[q];
-        dst[2 * kTilePixels + p] = cg[q];
-        dst[3 * kTilePixels + p] = cb[q];
+        dst[p] = L.T[q];
+        dst[kTilePixels + p] = L.cr[q];
+        dst[2 * kTilePixels + p] = L.cg[q];
+        dst[3 * kTilePixels + p] = L.cb[q];
     }
-    if (threadIdx.x == 0) {  // thread 0 holds the batch and record work (wave 0)
-        ck.pos[slot] = pos;
-        ck.work[slot] = work;
-    }
+    if (threadIdx.x == 0) ck.pos[slot] = pos;
+    if (threadIdx.x % kWave == 0) s.wave_work[W == 1 ? 0 : tile_wave()] = work;
+}
+
+// The tile's work before the checkpoint saved last, its waves' work summed.  After a
+// barrier that follows save_checkpoint.
+template <int W>
+__device__ __forceinline__ void save_checkpoint_work(const BatchLds<W> &s, const Checkpoints &ck,
+                                                     int tile, int i) {
+    if (threadIdx.x != 0) return;
+    uint32_t sum = 0;
+#pragma unroll
+    for (int w = 0; w < W; ++w) sum += s.wave_work[w];
+    ck.work[tile * kCheckpoints + i] = sum;
 }
 
 // With ck.data (the forward of a tile in [0, n_tiles)), saves up to kCheckpoints
@@ -632,48 +810,58 @@ __device__ __forceinline__ void blend_accumulate(
     const float *__restrict__ points, const float *__restrict__ conics,
     const float *__restrict__ opac, const float *__restrict__ colors,
     const LanePixels<kStrips / W> &pix, float alpha_thr, float T_thr_in, float chi,
-    float (&cr)[kStrips / W], float (&cg)[kStrips / W], float (&cb)[kStrips / W],
-    uint32_t &work, const Checkpoints &ck = kNoCheckpoints,
+    ForwardLane<kStrips / W> &L, uint32_t &work, const Checkpoints &ck = kNoCheckpoints,
     int tile = 0, int *n_ck = nullptr) {
     constexpr int S = kStrips / W;
     // a pixel is active while !(T < T_thr)
     const float T_thr = effective_T_thr(T_thr_in);
-    float T[S];
 #pragma unroll
     for (int q = 0; q < S; ++q) {
-        T[q] = pix.inside[q] ? 1.0f : kInactiveT;
-        cr[q] = cg[q] = cb[q] = 0.0f;
+        // outside the image: 0 where blend_group multiplies it by alpha
+        L.T[q] = pix.inside[q] ? 1.0f : 0.0f;
+        L.cr[q] = L.cg[q] = L.cb[q] = 0.0f;
     }
     if (n_ck) *n_ck = 0;
     if (span.end <= span.start) return;
     BatchPipe<false, W> pipe;
-    pipe.start(span, ids);
+    pipe.start(s, span, ids);
     const bool counter = W == 1 || tile_wave() == 0;
-    int batch = 0, saved = 0;
+    constexpr int kEvery = W == 1 ? kCheckpointSpacing / kBatch : 1;  // batches
+    constexpr bool kMid = kBatch * W > kCheckpointSpacing;  // also within a batch
+    int batch = 0, saved = 0, summed = 0;
     for (int32_t b0 = span.start; b0 < span.end; b0 += kBatch * W, ++batch) {
-        // with W > 1 waves, each one's work joins the vote's barrier, so that a
-        // checkpoint records the tile's work so far, not wave 0's
-        const bool ck_now = ck.data && batch > 0 && batch % checkpoint_spacing<W>() == 0 &&
-                            saved < kCheckpoints;
-        if (W > 1 && ck_now && threadIdx.x % kWave == 0) s.wave_work[tile_wave()] = work;
-        if (!tile_any<W>(any_active(T, T_thr), s.wave_flag)) break;
-        if (ck_now) {
-            uint32_t tile_work = work;
-            if constexpr (W > 1) {
-                tile_work = 0;
-#pragma unroll
-                for (int w = 0; w < W; ++w) tile_work += s.wave_work[w];
-            }
-            save_checkpoint<W>(ck, tile, saved, b0, tile_work, T, cr, cg, cb);
-            ++saved;
+        const bool more = tile_any<W>(any_active(L.T, T_thr), s.wave_flag);
+        if (W > 1 && summed < saved) save_checkpoint_work<W>(s, ck, tile, summed++);
+        if (!more) break;
+        if (ck.data && batch > 0 && batch % kEvery == 0 && saved < kCheckpoints) {
+            if (W > 1) __syncthreads();  // the work of the checkpoint before is summed
+            save_checkpoint<W>(s, ck, tile, saved++, b0, work, L);
         }
-        const Staged st = pipe.advance(s, b0, span, ids, n, points, conics, opac, colors, chi,
-                                       alpha_thr, pix.x0, pix.y0);
-        if (counter) work += kCostBatch + kCostStaged * (uint32_t)st.count;
+        const Staged<W> st = pipe.advance(s, b0, span, ids, n, points, conics, opac, colors, chi,
+                                          alpha_thr, pix.x0, pix.y0);
+        // the barriers of the staging lie between save_checkpoint and this
+        if (summed < saved) save_checkpoint_work<W>(s, ck, tile, summed++);
+        work += (counter ? kCostBatch : 0) + kCostStaged * (uint32_t)st.count;
+        constexpr int kHalf = kMid ? kCheckpointSpacing / kBatch : W;
         if (st.nonfinite)
-            blend_batch<true, W>(s, st.count, pix, alpha_thr, T_thr, chi, T, cr, cg, cb, work);
+            blend_batch<true, W, 0, kHalf>(s, st, pix, alpha_thr, T_thr, L, work);
         else
-            blend_batch<false, W>(s, st.count, pix, alpha_thr, T_thr, chi, T, cr, cg, cb, work);
+            blend_batch<false, W, 0, kHalf>(s, st, pix, alpha_thr, T_thr, L, work);
+        if constexpr (kMid) {
+            const int32_t mid = b0 + kCheckpointSpacing;
+            if (ck.data && saved < kCheckpoints && mid < span.end) {
+                __syncthreads();  // the work of the checkpoint before is summed
+                save_checkpoint<W>(s, ck, tile, saved++, mid, work, L);
+            }
+            if (st.nonfinite)
+                blend_batch<true, W, kHalf, W>(s, st, pix, alpha_thr, T_thr, L, work);
+            else
+                blend_batch<false, W, kHalf, W>(s, st, pix, alpha_thr, T_thr, L, work);
+        }
+    }
+    if (summed < saved) {  // uniform: the last batch's
+        __syncthreads();
+        save_checkpoint_work<W>(s, ck, tile, summed);
     }
     if (n_ck) *n_ck = saved;
 }
@@ -750,11 +938,9 @@ __device__ __forceinline__ void row_sum9(const float (&f)[kGradFields], float &q
           "v"(f[8]));
 }
 
-// One tile per workgroup of W waves (64 W threads).  Held to 64 VGPRs (8 waves
-// per SIMD), which the compiler meets without spilling; the checkpoint stores
-// would otherwise take it to 72 (7 waves).
+// One tile per workgroup of W waves (64 W threads).
 template <int W>
-__global__ __launch_bounds__(kWave * W) __attribute__((amdgpu_waves_per_eu(8, 8)))
+__global__ __launch_bounds__(kWave * W) __attribute__((amdgpu_waves_per_eu(W == 1 ? 6 : 5)))
 void blend_forward_kernel(
     const int32_t *__restrict__ offsets, const int32_t *__restrict__ ids, int n_tiles,
     int64_t k, int64_t n, const float *__restrict__ points, const float *__restrict__ conics,
@@ -781,37 +967,23 @@ void blend_forward_kernel(
     if ((unsigned)tile >= (unsigned)n_tiles) return;  // uniform across the workgroup
     const LanePixels<S> pix = lane_pixels<W>(tile, tiles_x, width, height);
     const TileSpan span = tile_span(offsets, n_tiles, k, tile);
-    if (n_tiles <= kCheckpointMaxTiles) {
-        // Grids whose tiles all start at once end with their longest walks: give
-        // the tiles with long lists (their walks' upper bound) more of the SIMDs'
-        // issue slots while they share them.  On larger grids the raised
-        // priority delays the tiles that start later and the kernel ends later.
-        const int64_t mean = (k - (int64_t)offsets[0]) / n_tiles;  // offsets[0]: the capped shift
-        const int64_t len = span.end - span.start;
-        if (len >= 3 * mean / 2)
-            __builtin_amdgcn_s_setprio(3);
-        else if (len >= 6 * mean / 5)
-            __builtin_amdgcn_s_setprio(2);
-        else if (len >= 9 * mean / 10)
-            __builtin_amdgcn_s_setprio(1);
-    }
-    float cr[S], cg[S], cb[S];
+    ForwardLane<S> L;
     uint32_t work = 0;
     int n_ck = 0;
     blend_accumulate<W>(s, span, ids, n, points, conics, opac, colors, pix, alpha_thr, T_thr, chi,
-                        cr, cg, cb, work, ck, tile, &n_ck);
+                        L, work, ck, tile, &n_ck);
     if (ck.count && threadIdx.x == 0) ck.count[tile] = n_ck;
     float l1 = 0.0f;
 #pragma unroll
     for (int q = 0; q < S; ++q) {
         if (!pix.inside[q]) continue;
         const int64_t o = ((int64_t)pix.fy[q] * width + (int64_t)pix.fx) * 3;
-        image[o] = cr[q];
-        image[o + 1] = cg[q];
-        image[o + 2] = cb[q];
+        image[o] = L.cr[q];
+        image[o + 1] = L.cg[q];
+        image[o + 2] = L.cb[q];
         if (display) {  // image.clamp(0, 1) * 255 (src/cuda/wrapper.py:294)
-            const float d[3] = {clamp01(cr[q]) * 255.0f, clamp01(cg[q]) * 255.0f,
-                                clamp01(cb[q]) * 255.0f};
+            const float d[3] = {clamp01(L.cr[q]) * 255.0f, clamp01(L.cg[q]) * 255.0f,
+                                clamp01(L.cb[q]) * 255.0f};
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
                 display[o + c] = d[c];
@@ -946,9 +1118,9 @@ __device__ __forceinline__ void backward_flush(const BackwardLds<W> &s, Pending 
     const int lane = threadIdx.x % kWave, e = lane >> 4;
     const uint32_t j = (pd.js >> (8 * e)) & 255u;  // < kBatch * W, also for a stale slot
     const float4 geo = s.batch.geo[j];
-    const float C = s.batch.aux[j].x;
-    const uint32_t g = __float_as_uint(s.batch.col[j].w);
-    const float inv_o = s.batch.inv_o[j];
+    const float C = s.batch.aux[j].x, log2o = s.batch.aux[j].z;
+    const uint32_t g = __float_as_uint(s.batch.col[j].z);
+    const float inv_o = s.batch.col[j].w;
     const float2 *p = s.pend[W == 1 ? 0 : tile_wave()] + e * kPendStride + (lane & 15);
     float2 a = p[0], b = p[kWave], c = p[2 * kWave];
 #pragma unroll
@@ -979,9 +1151,8 @@ __device__ __forceinline__ void backward_flush(const BackwardLds<W> &s, Pending 
     row_sum9(f, q0, q1, q2);
     const float total = (lane & 3) == 0 ? q0 : ((lane & 3) == 1 ? q1 : q2);
     const float scale = tgt.inv_o ? inv_o : tgt.fa;
-    // a record with a special opacity stages 0 for 1 / o: its opacity gradient was
-    // added by the entry itself (backward_entry_safe)
-    if (tgt.active && e < pd.n && scale != 0.0f) {
+    // the opacity gradient of a special opacity was added by backward_entry_safe
+    if (tgt.active && e < pd.n && !(tgt.inv_o && special_opacity(log2o))) {
         const uint64_t off = (uint64_t)g * (uint64_t)tgt.stride4;
         unsafeAtomicAdd(reinterpret_cast<float *>(reinterpret_cast<char *>(tgt.base) + off),
                         total * scale);
@@ -1013,7 +1184,7 @@ __device__ __forceinline__ void backward_entry(BackwardLds<W> &s, int j,
     constexpr int S = kStrips / W;
     const float4 aux = s.batch.aux[j];
     const float4 geo = s.batch.geo[j];
-    const float4 col = s.batch.col[j];
+    const float2 gb = *reinterpret_cast<const float2 *>(&s.batch.col[j]);
     const float du = pix.fx - geo.x;
     const float Adudu = (geo.z * du) * du;
     const float B2du = geo.w * du;
@@ -1033,10 +1204,10 @@ __device__ __forceinline__ void backward_entry(BackwardLds<W> &s, int j,
 #pragma unroll
     for (int q = 0; q < S; ++q) {
         if (inc[q] == 0) continue;  // uniform
-        const float alpha = alpha_of(E[q], aux.w);
+        const float alpha = alpha_of(E[q], aux.z);
         const float a = __builtin_amdgcn_inverse_ballot_w64(inc[q]) ? alpha : 0.0f;
         const float w = a * L.T[q];
-        const float gcol = fmaf(L.gr[q], col.x, fmaf(L.gg[q], col.y, L.gb[q] * col.z));
+        const float gcol = fmaf(L.gr[q], aux.w, fmaf(L.gg[q], gb.x, L.gb[q] * gb.y));
         const float acc = fmaf(w, gcol, L.acc[q]);
         const float T = L.T[q] - w;
         act[q] = __ballot(!(T < T_thr));
@@ -1061,22 +1232,19 @@ __device__ __forceinline__ void backward_entry(BackwardLds<W> &s, int j,
 // threshold (dL/dalpha from 1 - alpha + 1e-10, as the reference).
 template <int W>
 __device__ __forceinline__ void backward_entry_safe(BackwardLds<W> &s, int j,
+                                                    uint32_t bits,
                                                     const LanePixels<kStrips / W> &pix,
                                                     float alpha_thr, float T_thr,
                                                     BackwardLane<kStrips / W> &L, Pending &pd,
                                                     const GradOut &out) {
     constexpr int S = kStrips / W;
     const float4 aux = s.batch.aux[j];
-    uint32_t smask = __builtin_amdgcn_readfirstlane(__float_as_uint(aux.z));
-    if constexpr (W > 1) smask = (smask >> (tile_wave() * S)) & ((1u << S) - 1u);
-    if (smask == 0u) return;  // uniform: none of this wave's strips
     const float4 geo = s.batch.geo[j];
     const float4 col = s.batch.col[j];
     // uniform: a record with a non-finite log2 opacity; its opacity gradient is
     // summed as G dalpha
     const bool special = special_opacity(
-        __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(aux.w))));
-    const float o_sp = special ? s.batch.o_raw[j] : 0.0f;
+        __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(aux.z))));
     const float du = pix.fx - geo.x;
     const float Adudu = (geo.z * du) * du;
     const float B2du = geo.w * du;
@@ -1084,21 +1252,21 @@ __device__ __forceinline__ void backward_entry_safe(BackwardLds<W> &s, int j,
     bool hit = false;  // some strip was evaluated
 #pragma unroll
     for (int q = 0; q < S; ++q) {
-        if (!((smask >> q) & 1u)) continue;  // uniform
+        if (!((bits >> q) & 1u)) continue;  // uniform
         const float dv = pix.fy[q] - geo.y;
         const float E = fmaf(fmaf(aux.x, dv, B2du), dv, Adudu);
         bool inc = !(L.T[q] < T_thr) && (E < aux.y);
         float alpha = 0.0f, G = 0.0f;
         if (special) {  // alpha = o G from the raw opacity, alpha test on its value
             G = __builtin_amdgcn_exp2f(E * kNegHalfLog2e);
-            alpha = o_sp * G;
+            alpha = col.w * G;
             inc = inc && !(alpha < alpha_thr);
         }
         if (!wave_any(inc)) continue;
         hit = true;
-        if (!special) alpha = alpha_of(E, aux.w);
+        if (!special) alpha = alpha_of(E, aux.z);
         const float w = alpha * L.T[q];
-        const float gcol = fmaf(L.gr[q], col.x, fmaf(L.gg[q], col.y, L.gb[q] * col.z));
+        const float gcol = fmaf(L.gr[q], aux.w, fmaf(L.gg[q], col.x, L.gb[q] * col.y));
         const float acc = fmaf(w, gcol, L.acc[q]);  // -S_i
         const float one_m = (1.0f - alpha) + kTransmittanceEps;
         // dalpha = T gcol - S_i / (1 - alpha + eps)
@@ -1120,7 +1288,7 @@ __device__ __forceinline__ void backward_entry_safe(BackwardLds<W> &s, int j,
     if (special) {
         const float total = wave_sum(sGd);
         if (threadIdx.x % kWave == 0) {
-            const uint32_t g = __float_as_uint(col.w);
+            const uint32_t g = __float_as_uint(col.z);
             unsafeAtomicAdd(out.opac + (uint64_t)g * (uint64_t)(uint32_t)out.s_opac, total);
         }
     }
@@ -1128,29 +1296,37 @@ __device__ __forceinline__ void backward_entry_safe(BackwardLds<W> &s, int j,
 }
 
 template <bool kSafe, int W>
-__device__ __forceinline__ void backward_batch(BackwardLds<W> &s, int cnt,
+__device__ __forceinline__ void backward_batch(BackwardLds<W> &s, const Staged<W> &st,
                                                const LanePixels<kStrips / W> &pix,
                                                float alpha_thr, float T_thr,
                                                BackwardLane<kStrips / W> &L,
                                                const GradTarget &tgt, const GradOut &out) {
     constexpr int S = kStrips / W;
-    if (W > 1 && !any_active(L.T, T_thr)) return;  // this wave's pixels are done
-    Pending pd{0, 0u};
     uint64_t act[S];
+    uint64_t left = active_masks(L.T, T_thr, act);
+    Pending pd{0, 0u};
 #pragma unroll
-    for (int q = 0; q < S; ++q) act[q] = __ballot(!(L.T[q] < T_thr));
-    for (int j = 0; j < cnt; ++j) {
-        if (kSafe) {
-            backward_entry_safe<W>(s, j, pix, alpha_thr, T_thr, L, pd, out);
-            if ((j & 7) == 7 && !any_active(L.T, T_thr)) break;
-        } else {
-            backward_entry<W>(s, j, pix, T_thr, L, act, pd);
-            uint64_t left = 0;
+    for (int g = 0; g < W; ++g) {
+        uint64_t any = 0;
 #pragma unroll
-            for (int q = 0; q < S; ++q) left |= act[q];
-            if (left == 0) break;
+        for (int q = 0; q < S; ++q) any |= st.mask[q][g];
+        while (any != 0 && left != 0) {
+            const int j = __builtin_ctzll(any), slot = g * kBatch + j;
+            any &= any - 1;
+            if constexpr (kSafe) {
+                uint32_t bits = 0;
+#pragma unroll
+                for (int q = 0; q < S; ++q) bits |= (uint32_t)((st.mask[q][g] >> j) & 1u) << q;
+                backward_entry_safe<W>(s, slot, bits, pix, alpha_thr, T_thr, L, pd, out);
+                left = active_masks(L.T, T_thr, act);
+            } else {
+                backward_entry<W>(s, slot, pix, T_thr, L, act, pd);
+                left = 0;
+#pragma unroll
+                for (int q = 0; q < S; ++q) left |= act[q];
+            }
+            if (pd.n == kPend) backward_flush<W>(s, pd, pix.fx, tgt);
         }
-        if (pd.n == kPend) backward_flush<W>(s, pd, pix.fx, tgt);
     }
     if (pd.n > 0) backward_flush<W>(s, pd, pix.fx, tgt);
 }
@@ -1212,11 +1388,12 @@ __device__ __forceinline__ void backward_tile(BackwardLds<W> &s, int tile, int s
     const float l1_scale = kSeed == kSeedL1 ? *grad_loss * inv_count : 0.0f;
 
     BackwardLane<S> L;
-    float cr[S], cg[S], cb[S];
+    ForwardLane<S> F;   // the pixels' colours
     uint32_t work = 0;  // unused here
     if (!image)
         blend_accumulate<W>(s.batch, span, ids, n, points, conics, opac, colors, pix, alpha_thr,
-                            T_thr_in, chi, cr, cg, cb, work);
+                            T_thr_in, chi, F, work);
+    float(&cr)[S] = F.cr, (&cg)[S] = F.cg, (&cb)[S] = F.cb;
     bool finite = true;
 #pragma unroll
     for (int q = 0; q < S; ++q) {
@@ -1273,15 +1450,15 @@ __device__ __forceinline__ void backward_tile(BackwardLds<W> &s, int tile, int s
     const GradTarget tgt = grad_target(threadIdx.x % kWave, out);
 
     BatchPipe<true, W> pipe;
-    pipe.start(span, ids);
+    pipe.start(s.batch, span, ids);
     for (int32_t b0 = span.start; b0 < span.end; b0 += kBatch * W) {
         if (!tile_any<W>(any_active(L.T, T_thr), s.batch.wave_flag)) break;
-        const Staged st = pipe.advance(s.batch, b0, span, ids, n, points, conics, opac, colors,
+        const Staged<W> st = pipe.advance(s.batch, b0, span, ids, n, points, conics, opac, colors,
                                        chi, alpha_thr, pix.x0, pix.y0);
         if (st.nonfinite || tile_safe)
-            backward_batch<true, W>(s, st.count, pix, alpha_thr, T_thr, L, tgt, out);
+            backward_batch<true, W>(s, st, pix, alpha_thr, T_thr, L, tgt, out);
         else
-            backward_batch<false, W>(s, st.count, pix, alpha_thr, T_thr, L, tgt, out);
+            backward_batch<false, W>(s, st, pix, alpha_thr, T_thr, L, tgt, out);
     }
 }
 
@@ -1512,22 +1689,22 @@ static int check_blend_args(const int32_t *indexing_offset, const int32_t *ids, 
     return GS_OK;
 }
 
-// Waves per tile of the 16x16 blend kernels.  A grid with few tiles leaves most
-// SIMDs idle, and a kernel then lasts as long as its slowest tile takes on its
-// waves: splitting each tile's strips over 2 or 4 waves (which share the staged
-// batches) shortens that, at the price of each wave reading the entries that
-// reach its strips, and in the backward of a wave sum and atomics per wave and
-// entry.  Measured (blend forward / backward, us, 1 -> 2 -> 4 waves):
-// 256 tiles 101/155 -> 86/118 -> 73/88; 2500 tiles 140/193 -> 138/247 ->
-// 149/352; 3600 tiles 160/210 -> 146/229 -> 152/329; 8160 tiles 159/238 ->
-// 173/396 -> 202/712.
-// Two waves gain in the forward on mid-size grids and lose in every backward, so
-// the backward takes 4 waves up to kFourWaveTiles tiles and 1 above, the forward
-// also 2 up to kCheckpointMaxTiles tiles (the forward's checkpoints and the
-// backward's segments do not depend on either's wave count).  Per-tile timing of
-// the forward with checkpoints (kernel span, us, 1 -> 2 waves): 3600 tiles
-// 161.9 -> 140.9, 2500 tiles 129.7 -> 125.6.
+// Waves per tile of the 16x16 blend kernels.  Splitting a tile's strips over 2 or 4
+// waves (which share the staged batches) shortens its walk, at the price of each wave
+// reading the entries that reach its strips, and in the backward of a wave sum and
+// atomics per wave and entry.
+// Forward, us, 1 / 2 / 4 waves (entry by entry with one wave, in groups with more):
+//   192 tiles (20k Gaussians) 176 / 70 / 45, 256 tiles 99 / 43 / 29, 2170 tiles
+//   155 / 96 / 77, 3600 tiles 147 / 102 / 87, 6700 tiles 120 / 107 / 109, 8160 tiles
+//   138 / 122 / 127 (3M Gaussians 149 / 121 / 126), 32400 tiles 355 / 380 / 440.
+// So 4 up to kCheckpointMaxTiles tiles, 2 up to kTwoWaveTiles and 1 above, where the
+// chip is full and only the instructions count.  Backward, us, 1 / 2 / 4 waves, from
+// the same checkpoints: 192 tiles 109 / 67 / 46, 256 tiles 54 / 39 / 30, 2170 tiles
+// 97 / 103 / 133, 3600 tiles 115 / 132 / 174, 8160 tiles 175 / 231 / 345: 4 up to
+// kFourWaveTiles and 1 above.  The forward's checkpoints and the backward's segments
+// do not depend on either's wave count.
 constexpr int kFourWaveTiles = 1024;
+constexpr int kTwoWaveTiles = 16384;
 static int g_blend_waves = 0;  // gs_set_blend_waves: 0 = by tile count
 
 static int blend_waves(int32_t n_tiles) {
@@ -1537,7 +1714,7 @@ static int blend_waves(int32_t n_tiles) {
 
 static int blend_waves_forward(int32_t n_tiles) {
     if (g_blend_waves) return g_blend_waves;
-    return n_tiles <= kFourWaveTiles ? 4 : (n_tiles <= kCheckpointMaxTiles ? 2 : 1);
+    return n_tiles <= kCheckpointMaxTiles ? 4 : (n_tiles <= kTwoWaveTiles ? 2 : 1);
 }
 
 static int rasterize_impl(const int32_t *indexing_offset, const int32_t *gaussian_ids_sorted,
