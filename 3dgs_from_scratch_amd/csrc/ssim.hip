@@ -9,13 +9,13 @@
 // with zero padding, C1 = 0.01^2, C2 = 0.03^2, averaged over all pixels or
 // over the pixels at least 5 from the border.
 //
-// Layout.  Work is cut into units of 64 columns x 34 rows of outputs of one
-// plane, one per wave (lane = output column); a fixed number of workgroups of
-// 4 waves (set by the image geometry alone) walk them, each XCD a contiguous
-// range.  A wave streams its unit's input rows (10 more than its
-// output rows) top to bottom: each row's 74 staged values (and the products
-// x^2 + y^2, xy) go to a wave-private LDS line, each lane filters its 11
-// neighbours, and the column filter accumulates into an 11-row ring of
+// Layout.  Work is cut into units of 64 columns x `rows` rows of outputs of one
+// plane, one per wave (lane = output column); workgroups of 4 waves, their
+// number and the units' height set by the image geometry alone (unit_rows),
+// each XCD a contiguous range.  A wave streams its unit's input rows (10 more
+// than its output rows) top to bottom: each row's 74 staged values (and the
+// products x^2 + y^2, xy) go to a wave-private LDS line, each lane filters its
+// 11 neighbours, and the column filter accumulates into an 11-row ring of
 // registers, so an output row is complete 10 rows after its first
 // contribution; its SSIM and derivatives are formed during the next row's LDS
 // reads.  No workgroup barrier inside the walk; input rows are loaded a few
@@ -25,6 +25,15 @@
 // The forward writes per-pixel derivative maps (planar, coalesced) for the
 // backward, which filters them back the same way.  The mean is reduced
 // deterministically: per-workgroup double partials, then one workgroup.
+//
+// What bounds it: the issue of vector instructions (the forward 120 a row and
+// wave, 88 of them FMAs by a tap) together with the LDS (11 reads of 16 bytes),
+// at 3 waves a SIMD; the backward of a large image the memory (2 x 3 x 1063 x
+// 1599: 246 MB in 65 us, 3.8 TB/s).  Measured in us, forward / backward, with
+// units of 34 rows everywhere, the taps in scalar registers and row addresses
+// formed anew each row -> as it is: 2 x 3 x 1063 x 1599 116 / 111 -> 58 / 65,
+// 3 x 1080 x 1920 48 / 37 -> 38 / 32, 3 x 720 x 1280 36 / 28 -> 24 / 19,
+// 3 x 547 x 979 28 / 22 -> 20 / 16, 3 x 2160 x 3840 209 / 202 -> 137 / 169.
 #include <cmath>
 #include <mutex>
 
@@ -46,22 +55,14 @@ constexpr float kC2 = 0.03f * 0.03f;
 
 static_assert(kTileX == kWave, "one lane per output column");
 
-// Unit shape of a pass: kRows output rows per unit (kRows + 2 kRadius input
-// rows, walked in whole ring turns: the rows past them complete output rows
-// past the unit, which are not written), input rows loaded kAheadRows ahead of
-// the filtered one.  kRows + 2 kRadius a multiple of kRing walks no rows past
-// the unit; taller units re-read fewer halo rows (from L2) but leave fewer
-// waves to fill the GPU.
-template <int kRows, int kAheadRows>
-struct Shape {
-    static constexpr int rows = kRows;
-    static constexpr int ahead = kAheadRows;
-    static constexpr int in_rows = kRows + 2 * kRadius;
-    static constexpr int walk = (in_rows + kRing - 1) / kRing * kRing;
-    static_assert(kAheadRows > 0 && kAheadRows < kRing, "prefetch within the ring");
-};
-using FwdShape = Shape<34, 5>;
-using BwdShape = Shape<34, 4>;
+// Input rows loaded ahead of the filtered one.
+constexpr int kFwdAhead = 5;
+constexpr int kBwdAhead = 4;
+static_assert(kFwdAhead < kRing && kBwdAhead < kRing, "prefetch within the ring");
+
+constexpr int kMaxBlocks = 1024;                 // workgroups of a pass
+constexpr int kTargetUnits = 3072;               // units of a pass, where the image allows it
+constexpr int kMaxTurns = 1 << 20;               // (the height of a unit stays in 32 bits)
 
 struct Window {
     float w[kTaps];
@@ -87,6 +88,7 @@ struct Planes {
     int r1, c1, r2, c2;    // element strides of row and column (in-plane offsets fit 31 bits)
     int channels, height, width;
     int tiles_x, tiles_y, tiles;
+    int rows, walk;        // output rows of a unit; its input rows, whole ring turns
     int valid;             // mean over pixels at least kRadius from the border
     float inv_count;       // 1 / pixels in the mean (all planes)
     float inv1;            // img1 values are its elements * inv1 (1: as stored)
@@ -95,14 +97,7 @@ struct Planes {
 // Element of img1 as the SSIM sees it: times inv1 = 1 / divisor rounded to
 // float, which is how PyTorch's GPU kernels compute image / divisor for a
 // scalar divisor (so the values equal the reference's rendered_image / 255).
-__device__ __forceinline__ float img1_value(const Planes &p, float v) {
-    return p.inv1 == 1.0f ? v : v * p.inv1;
-}
-
-__device__ __forceinline__ bool in_region(const Planes &p, int y, int x) {
-    if (!p.valid) return true;
-    return y >= kRadius && y < p.height - kRadius && x >= kRadius && x < p.width - kRadius;
-}
+__device__ __forceinline__ float img1_value(const Planes &p, float v) { return v * p.inv1; }
 
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
@@ -145,7 +140,6 @@ struct Tile {
     int ox, oy;  // first output column / row
 };
 
-template <int kRows>
 __device__ __forceinline__ Tile tile_of(const Planes &p, int t) {
     Tile r;
     r.c = t % p.channels;
@@ -155,19 +149,20 @@ __device__ __forceinline__ Tile tile_of(const Planes &p, int t) {
     r.b = rest2 / p.tiles_y;
     r.plane = r.b * p.channels + r.c;
     r.ox = tx * kTileX;
-    r.oy = (rest2 % p.tiles_y) * kRows;
+    r.oy = (rest2 % p.tiles_y) * p.rows;
     return r;
 }
 
 // This lane's staged columns of a unit: ox - kRadius + lane and, for the first
-// 2 kRadius lanes, ox - kRadius + kWave + lane (the right halo); with their
-// byte offsets, clamped into the image, in a row of img1, of img2 and of a
-// planar map, and the byte offsets of the lane's output column (clamped) in a
-// row of img1 and img2.  Row starts are wave-uniform pointers (scalar
-// registers), so a load adds only these per-lane offsets.
+// 2 kRadius lanes, ox - kRadius + kWave + lane (the right halo; the other lanes
+// repeat its last column, so that their loads touch no further memory line);
+// whether they lie in the image; and their byte offsets, clamped into the
+// image, in a row of img1, of img2 and of a planar map, and those of the lane's
+// output column (clamped) in a row of img1 and img2.  Row starts are
+// wave-uniform pointers (scalar registers), so a load adds only these per-lane
+// offsets.
 struct Cols {
-    int a, b;
-    bool has_b;
+    bool has_b, ina, inb;
     uint32_t a1, b1, a2, b2, am, bm;
     uint32_t o1, o2;
 };
@@ -175,11 +170,13 @@ struct Cols {
 __device__ __forceinline__ Cols cols_of(const Planes &p, const Tile &t) {
     const int lane = threadIdx.x % kWave;
     Cols c;
-    c.a = t.ox - kRadius + lane;
-    c.b = t.ox - kRadius + kWave + lane;
+    const int a = t.ox - kRadius + lane;
+    const int b = t.ox - kRadius + kWave + min(lane, 2 * kRadius - 1);
     c.has_b = lane < 2 * kRadius;
-    const uint32_t ca = (uint32_t)min(max(c.a, 0), p.width - 1);
-    const uint32_t cb = (uint32_t)min(c.b, p.width - 1);
+    c.ina = a >= 0 && a < p.width;
+    c.inb = b < p.width;
+    const uint32_t ca = (uint32_t)min(max(a, 0), p.width - 1);
+    const uint32_t cb = (uint32_t)min(b, p.width - 1);
     const uint32_t co = (uint32_t)min(t.ox + lane, p.width - 1);
     c.a1 = ca * (uint32_t)p.c1 * 4u;
     c.b1 = cb * (uint32_t)p.c1 * 4u;
@@ -192,73 +189,82 @@ __device__ __forceinline__ Cols cols_of(const Planes &p, const Tile &t) {
     return c;
 }
 
+// A wave-uniform row pointer that moves down one row at a time.
+struct Row {
+    const float *at;
+    __device__ __forceinline__ void next(int stride) {
+        at += (uint32_t)stride;
+        asm volatile("" : "+s"(at));  // one add a row, not a product per unrolled row
+    }
+};
+
 // The float `byte_offset` bytes past `row`, a wave-uniform pointer: a raw
-// buffer access over the bytes from `row` on, whose base and row offset live in
-// scalar registers and whose per-lane offset is the 32-bit value itself (a
-// plain access would add a 64-bit vector address per load or store).
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t span_of(const float *row) {
-    // stride 0, 2^32 - 1 bytes (no range check in practice), gfx9 data format
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(row), (short)0, -1, 0x00020000);
+// buffer access whose base lives in scalar registers and whose per-lane offset
+// is the 32-bit value itself (a plain access would add a 64-bit vector address
+// per load or store).  `bytes` is the buffer's length: ~0u (no range check in
+// practice) for a row of the image, 0 for a row outside it, where the load
+// returns 0 without an access.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t span_of(const float *row, uint32_t bytes) {
+    // stride 0, gfx9 data format
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(row), (short)0, (int)bytes,
+                                             0x00020000);
 }
 
-__device__ __forceinline__ float load_at(const float *row, uint32_t byte_offset) {
+__device__ __forceinline__ float load_at(const float *row, uint32_t bytes,
+                                         uint32_t byte_offset) {
     return __uint_as_float(
-        __builtin_amdgcn_raw_buffer_load_b32(span_of(row), (int)byte_offset, 0, 0));
+        __builtin_amdgcn_raw_buffer_load_b32(span_of(row, bytes), (int)byte_offset, 0, 0));
 }
 
-__device__ __forceinline__ void store_at(float *row, uint32_t byte_offset, float v) {
-    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), span_of(row), (int)byte_offset, 0,
-                                          0);
+__device__ __forceinline__ void store_at(const float *row, uint32_t byte_offset, float v) {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), span_of(row, ~0u),
+                                          (int)byte_offset, 0, 0);
 }
 
-// Image row gy of both images at the lane's staged columns, as stored (loads
-// at clamped, in-image positions; the positions outside the image are zeroed
-// and the divisor applied when the values are used, some rows later, so that
-// no load has to complete before then).
-__device__ __forceinline__ void load_image_row(const Planes &p, const float *b1, const float *b2,
-                                               int gy, const Cols &c, float &xa, float &ya,
-                                               float &xb, float &yb) {
-    int y = min(max(gy, 0), p.height - 1);
-    asm volatile("" : "+s"(y));  // the loads stay at their row (not hoisted ahead)
-    const float *r1 = b1 + y * p.r1, *r2 = b2 + y * p.r2;
-    xa = load_at(r1, c.a1);
-    ya = load_at(r2, c.a2);
-    xb = load_at(r1, c.b1);
-    yb = load_at(r2, c.b2);
+// Length of row y for span_of.
+__device__ __forceinline__ uint32_t row_bytes(const Planes &p, int y) {
+    // (in scalar arithmetic: as a selection the compiler makes it a vector value)
+    int n = ~((y | (p.height - 1 - y)) >> 31);
+    asm volatile("" : "+s"(n));
+    return (uint32_t)n;
 }
 
-// Whether image row gy's staged columns a and b lie in the image.
-__device__ __forceinline__ void row_inside(const Planes &p, int gy, const Cols &c, bool &ina,
-                                           bool &inb) {
-    const bool row_in = gy >= 0 && gy < p.height;
-    ina = row_in && c.a >= 0 && c.a < p.width;
-    inb = row_in && c.has_b && c.b < p.width;
+// Image row y of both images at the lane's staged columns, as stored (0 for
+// rows outside the image; columns outside it are loaded clamped, and zeroed and
+// the divisor applied when the values are used, some rows later, so that no
+// load has to complete before then).
+__device__ __forceinline__ void load_image_row(const Planes &p, Row &r1, Row &r2, int y,
+                                               const Cols &c, float &xa, float &ya, float &xb,
+                                               float &yb) {
+    const uint32_t n = row_bytes(p, y);
+    xa = load_at(r1.at, n, c.a1);
+    ya = load_at(r2.at, n, c.a2);
+    xb = load_at(r1.at, n, c.b1);
+    yb = load_at(r2.at, n, c.b2);
+    r1.next(p.r1);
+    r2.next(p.r2);
 }
 
-// Row gy of the three planar maps at the lane's staged columns, as stored
-// (clamped loads; zeroed outside the image when used).
-__device__ __forceinline__ void load_map_row(const Planes &p, const float *m0, const float *m1,
-                                             const float *m2, int64_t base, int gy, const Cols &c,
+// Row y of the three planar maps at the lane's staged columns, likewise.
+__device__ __forceinline__ void load_map_row(const Planes &p, Row (&m)[3], int y, const Cols &c,
                                              float (&va)[3], float (&vb)[3]) {
-    int y = min(max(gy, 0), p.height - 1);
-    asm volatile("" : "+s"(y));  // the loads stay at their row (not hoisted ahead)
-    const int64_t o = base + (int64_t)y * p.width;
-    va[0] = load_at(m0 + o, c.am);
-    va[1] = load_at(m1 + o, c.am);
-    va[2] = load_at(m2 + o, c.am);
-    vb[0] = load_at(m0 + o, c.bm);
-    vb[1] = load_at(m1 + o, c.bm);
-    vb[2] = load_at(m2 + o, c.bm);
+    const uint32_t n = row_bytes(p, y);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        va[q] = load_at(m[q].at, n, c.am);
+        vb[q] = load_at(m[q].at, n, c.bm);
+        m[q].next(p.width);
+    }
 }
 
-// img1 / img2 at row gy of the lane's output column as stored (clamped load;
-// zeroed and divided when used).
-__device__ __forceinline__ void load_pixel(const Planes &p, const float *b1, const float *b2,
-                                           int gy, const Cols &c, float &x, float &y) {
-    int yy = min(max(gy, 0), p.height - 1);
-    asm volatile("" : "+s"(yy));  // the loads stay at their row
-    x = load_at(b1 + yy * p.r1, c.o1);
-    y = load_at(b2 + yy * p.r2, c.o2);
+// img1 / img2 at row y of the lane's output column as stored.
+__device__ __forceinline__ void load_pixel(const Planes &p, Row &r1, Row &r2, int y,
+                                           const Cols &c, float &x, float &yv) {
+    const uint32_t n = row_bytes(p, y);
+    x = load_at(r1.at, n, c.o1);
+    yv = load_at(r2.at, n, c.o2);
+    r1.next(p.r1);
+    r2.next(p.r2);
 }
 
 typedef float f4v __attribute__((ext_vector_type(4)));
@@ -281,6 +287,18 @@ __device__ __forceinline__ void taps_ready(f4v (&v)[kTaps]) {
                  "+v"(v[6]), "+v"(v[7]), "+v"(v[8]), "+v"(v[9]), "+v"(v[10]));
 }
 
+// The window's taps in vector registers (they are symmetric: 6 of them).  An
+// FMA that reads a scalar register takes 4.3 cycles of a SIMD on gfx950, one
+// that reads only vector registers 2.5; of the forward's 130 vector
+// instructions a row 88 multiply by a tap.
+__device__ __forceinline__ void taps_to_vector(Window &win) {
+#pragma unroll
+    for (int k = 0; k <= kRadius; ++k) {
+        asm volatile("" : "+v"(win.w[k]));
+        win.w[kTaps - 1 - k] = win.w[k];
+    }
+}
+
 // Horizontal filter at this lane's output column: h[q] = sum_k w[k] v[k].q,
 // k ascending.
 template <int NQ>
@@ -292,6 +310,13 @@ __device__ __forceinline__ void filter_taps(const Window &win, const f4v (&v)[kT
     for (int k = 0; k < kTaps; ++k)
 #pragma unroll
         for (int q = 0; q < NQ; ++q) h[q] = fmaf(win.w[k], v[k][q], h[q]);
+}
+
+// Row y of the unit's plane (y may lie outside the image: the pointer is then
+// only moved on from).
+__device__ __forceinline__ const float *row_of(const float *img, const int64_t (&s)[2],
+                                               int row_stride, const Tile &t, int y) {
+    return img + ((int64_t)t.b * s[0] + (int64_t)t.c * s[1] + (int64_t)y * row_stride);
 }
 
 // Makes the wave's LDS line stores visible to the wave's loads that follow
@@ -352,35 +377,59 @@ __device__ __forceinline__ SsimOut ssim_point(const float (&a)[4]) {
     return o;
 }
 
+// The output rows of a unit and the region of the mean: rows j in [0, end) are
+// written, those in [first, last) count if the lane's column does.
+struct Out {
+    int end, first, last;
+    bool col_in, col_counts;  // the lane's output column lies in the image / in the region
+    float g;                  // 1 / pixels in the mean for a column that counts, else 0
+    uint32_t col;             // byte offset of the column in a row of a map
+};
+
+__device__ __forceinline__ Out out_of(const Planes &p, const Tile &t) {
+    const int gx = t.ox + (int)(threadIdx.x % kWave);
+    const int m = p.valid ? kRadius : 0;
+    Out o;
+    o.end = min(p.rows, p.height - t.oy);
+    o.first = max(m - t.oy, 0);
+    o.last = max(min(o.end, p.height - m - t.oy), o.first);
+    o.col_in = gx < p.width;
+    o.col_counts = gx >= m && gx < p.width - m;
+    o.g = o.col_counts ? p.inv_count : 0.0f;
+    o.col = (uint32_t)gx * 4u;
+    return o;
+}
+
 // Output row j of a forward unit, complete in ring slot kSlot: its SSIM
-// (summed into `local` over the region) and, with d_mu, the derivative maps;
-// the slot is then cleared for the output row that starts in it.
+// (summed into `local` over the region) and, with the maps, their row; the slot
+// is then cleared for the output row that starts in it.
 template <int kSlot>
-__device__ __forceinline__ void forward_out(const Planes &p, const Tile &tl, int j,
-                                            float (&acc)[kRing][4], double &local, float *d_mu,
-                                            float *d_xx, float *d_xy) {
-    const int lane = threadIdx.x % kWave;
+__device__ __forceinline__ void forward_out(const Planes &p, const Out &out, int j,
+                                            float (&acc)[kRing][4], double &local,
+                                            bool with_maps, Row (&m)[3]) {
     float(&a)[4] = acc[kSlot];
-    const int gy = tl.oy + j;
-    const int gx = tl.ox + lane;
-    if (j < FwdShape::rows && gy < p.height && gx < p.width) {
+    if (j < out.end) {
         const SsimOut o = ssim_point(a);
-        const bool in = in_region(p, gy, gx);
-        if (in) local += (double)o.S;
-        if (d_mu) {
-            const float g = in ? p.inv_count : 0.0f;
-            int row = gy;
-            asm volatile("" : "+s"(row));  // the addresses are formed here, not ahead
-            const int64_t at = (int64_t)tl.plane * p.height * p.width + (int64_t)row * p.width;
-            const uint32_t col = (uint32_t)gx * 4u;
-            store_at(d_mu + at, col, g * o.dm);
-            store_at(d_xx + at, col, g * o.dxx);
-            store_at(d_xy + at, col, g * o.dxy);
+        const bool counts = (uint32_t)(j - out.first) < (uint32_t)(out.last - out.first);
+        local += (double)(counts && out.col_counts ? o.S : 0.0f);
+        if (with_maps) {
+            const float g = counts ? out.g : 0.0f;
+            const float v[3] = {g * o.dm, g * o.dxx, g * o.dxy};
+            if (out.col_in)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) store_at(m[q].at, out.col, v[q]);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) m[q].next(p.width);
         }
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) a[q] = 0.0f;
 }
+
+struct FwdRows {
+    float xa[kRing], ya[kRing], xb[kRing], yb[kRing];  // image rows in flight
+    Row r1, r2;                                        // the next rows to load
+};
 
 // Forward of one unit: per input row ri, x, y, x^2 + y^2 and xy into the LDS
 // line, the horizontal filter, the ring.  Input row ri - 1 completed output row
@@ -388,30 +437,25 @@ __device__ __forceinline__ void forward_out(const Planes &p, const Tile &tl, int
 // taps are read, before tap 0 of this row starts the slot again.
 template <bool kFirst, int S>
 __device__ __forceinline__ void forward_row(const Planes &p, const Window &win, const Tile &tl,
-                                            const Cols &c, const float *b1, const float *b2,
-                                            float4 *line, int ri, float (&xa)[kRing],
-                                            float (&ya)[kRing], float (&xb)[kRing],
-                                            float (&yb)[kRing], float (&acc)[kRing][4],
-                                            double &local, float *d_mu, float *d_xx,
-                                            float *d_xy) {
+                                            const Cols &c, const Out &out, float4 *line, int ri,
+                                            FwdRows &r, float (&acc)[kRing][4], double &local,
+                                            bool with_maps, Row (&m)[3]) {
     const int lane = threadIdx.x % kWave;
-    constexpr int kNext = (S + FwdShape::ahead) % kRing;
-    // (rows past the walk load in-image values that are never used)
-    load_image_row(p, b1, b2, tl.oy - kRadius + ri + FwdShape::ahead, c, xa[kNext], ya[kNext],
-                   xb[kNext], yb[kNext]);
-    bool ina, inb;
-    row_inside(p, tl.oy - kRadius + ri, c, ina, inb);
-    const float x = ina ? img1_value(p, xa[S]) : 0.0f, y = ina ? ya[S] : 0.0f;
+    constexpr int kNext = (S + kFwdAhead) % kRing;
+    // (rows past the walk are loaded and never used)
+    load_image_row(p, r.r1, r.r2, tl.oy - kRadius + ri + kFwdAhead, c, r.xa[kNext], r.ya[kNext],
+                   r.xb[kNext], r.yb[kNext]);
+    const float x = c.ina ? img1_value(p, r.xa[S]) : 0.0f, y = c.ina ? r.ya[S] : 0.0f;
     line[lane] = make_float4(x, y, x * x + y * y, x * y);
     if (c.has_b) {
-        const float x2 = inb ? img1_value(p, xb[S]) : 0.0f, y2 = inb ? yb[S] : 0.0f;
+        const float x2 = c.inb ? img1_value(p, r.xb[S]) : 0.0f, y2 = c.inb ? r.yb[S] : 0.0f;
         line[kWave + lane] = make_float4(x2, y2, x2 * x2 + y2 * y2, x2 * y2);
     }
     line_sync();
     f4v v[kTaps];
     read_taps(line, v);
     // (the first kRing input rows complete no output row before this one)
-    if constexpr (!kFirst) forward_out<S>(p, tl, ri - kRing, acc, local, d_mu, d_xx, d_xy);
+    if constexpr (!kFirst) forward_out<S>(p, out, ri - kRing, acc, local, with_maps, m);
     taps_ready(v);
     float h[4];
     filter_taps<4>(win, v, h);
@@ -421,17 +465,12 @@ __device__ __forceinline__ void forward_row(const Planes &p, const Window &win, 
 
 template <bool kFirst, int S = 0>
 __device__ __forceinline__ void forward_rows(const Planes &p, const Window &win, const Tile &tl,
-                                             const Cols &c, const float *b1, const float *b2,
-                                             float4 *line, int base, float (&xa)[kRing],
-                                             float (&ya)[kRing], float (&xb)[kRing],
-                                             float (&yb)[kRing], float (&acc)[kRing][4],
-                                             double &local, float *d_mu, float *d_xx,
-                                             float *d_xy) {
+                                             const Cols &c, const Out &out, float4 *line,
+                                             int base, FwdRows &r, float (&acc)[kRing][4],
+                                             double &local, bool with_maps, Row (&m)[3]) {
     if constexpr (S < kRing) {
-        forward_row<kFirst, S>(p, win, tl, c, b1, b2, line, base + S, xa, ya, xb, yb, acc, local,
-                               d_mu, d_xx, d_xy);
-        forward_rows<kFirst, S + 1>(p, win, tl, c, b1, b2, line, base, xa, ya, xb, yb, acc,
-                                    local, d_mu, d_xx, d_xy);
+        forward_row<kFirst, S>(p, win, tl, c, out, line, base + S, r, acc, local, with_maps, m);
+        forward_rows<kFirst, S + 1>(p, win, tl, c, out, line, base, r, acc, local, with_maps, m);
     }
 }
 
@@ -445,33 +484,36 @@ __global__ __launch_bounds__(kThreads) void ssim_forward_kernel(Planes p, Window
                                                                  double *__restrict__ partials) {
     __shared__ float4 lines[kUnitWaves][kInX];
     __shared__ double red[kWaves];
+        taps_to_vector(win);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     float4 *line = lines[wave];
     const int blk = xcd_block((int)blockIdx.x, (int)gridDim.x);
     double local = 0.0;
     for (int t = blk * kUnitWaves + wave; t < p.tiles;
          t += (int)gridDim.x * kUnitWaves) {
-        const Tile tl = tile_of<FwdShape::rows>(p, t);
+        const Tile tl = tile_of(p, t);
         const Cols c = cols_of(p, tl);
-        const float *b1 = p.img1 + ((int64_t)tl.b * p.s1[0] + (int64_t)tl.c * p.s1[1]);
-        const float *b2 = p.img2 + ((int64_t)tl.b * p.s2[0] + (int64_t)tl.c * p.s2[1]);
-        float xa[kRing], ya[kRing], xb[kRing], yb[kRing];
+        const Out out = out_of(p, tl);
+        FwdRows r;
+        r.r1.at = row_of(p.img1, p.s1, p.r1, tl, tl.oy - kRadius);
+        r.r2.at = row_of(p.img2, p.s2, p.r2, tl, tl.oy - kRadius);
+        const int64_t at = ((int64_t)tl.plane * p.height + tl.oy) * p.width;
+        Row m[3] = {{d_mu + at}, {d_xx + at}, {d_xy + at}};
         float acc[kRing][4];
 #pragma unroll
-        for (int r = 0; r < kRing; ++r)
+        for (int k = 0; k < kRing; ++k)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) acc[r][q] = 0.0f;
+            for (int q = 0; q < 4; ++q) acc[k][q] = 0.0f;
 #pragma unroll
-        for (int d = 0; d < FwdShape::ahead; ++d)
-            load_image_row(p, b1, b2, tl.oy - kRadius + d, c, xa[d], ya[d], xb[d], yb[d]);
-        forward_rows<true>(p, win, tl, c, b1, b2, line, 0, xa, ya, xb, yb, acc, local, d_mu,
-                           d_xx, d_xy);
-        for (int base = kRing; base < FwdShape::walk; base += kRing)
-            forward_rows<false>(p, win, tl, c, b1, b2, line, base, xa, ya, xb, yb, acc, local,
-                                d_mu, d_xx, d_xy);
+        for (int d = 0; d < kFwdAhead; ++d)
+            load_image_row(p, r.r1, r.r2, tl.oy - kRadius + d, c, r.xa[d], r.ya[d], r.xb[d],
+                           r.yb[d]);
+        forward_rows<true>(p, win, tl, c, out, line, 0, r, acc, local, d_mu != nullptr, m);
+        for (int base = kRing; base < p.walk; base += kRing)
+            forward_rows<false>(p, win, tl, c, out, line, base, r, acc, local, d_mu != nullptr,
+                                m);
         // the output row the last input row completed
-        forward_out<FwdShape::walk % kRing>(p, tl, FwdShape::walk - kRing, acc, local, d_mu,
-                                            d_xx, d_xy);
+        forward_out<0>(p, out, p.walk - kRing, acc, local, d_mu != nullptr, m);
     }
     const double s = block_sum(local, red);
     if (threadIdx.x == 0) partials[blk] = s;
@@ -481,14 +523,18 @@ __global__ __launch_bounds__(kThreads) void ssim_forward_kernel(Planes p, Window
 // With loss, also *loss = (1 - lambda) * *other + lambda * (1 - *mean), in
 // float as a PyTorch expression of those scalars would round it.
 __global__ __launch_bounds__(kThreads) void ssim_mean_kernel(const double *__restrict__ partials,
-                                                              int64_t n, double count,
+                                                              int n, double count,
                                                               float *__restrict__ mean,
                                                               const float *__restrict__ other,
                                                               float lambda,
                                                               float *__restrict__ loss) {
     __shared__ double red[kWaves];
     double v = 0.0;
-    for (int64_t i = threadIdx.x; i < n; i += kThreads) v += partials[i];
+#pragma unroll
+    for (int k = 0; k < kMaxBlocks / kThreads; ++k) {
+        const int i = (int)threadIdx.x + k * kThreads;
+        v += i < n ? partials[i] : 0.0;
+    }
     const double s = block_sum(v, red);
     if (threadIdx.x == 0) {
         const float m = (float)(count > 0.0 ? s / count : __builtin_nan(""));
@@ -499,27 +545,26 @@ __global__ __launch_bounds__(kThreads) void ssim_mean_kernel(const double *__res
 
 // Backward of one unit: the three maps filtered back the same way; output row
 // j's gradient is up * (F[d_mu] + 2 x F[d_xx] + y F[d_xy]) with x, y its pixel
-// (loaded BwdShape::ahead rows ahead as well).
+// (loaded kBwdAhead rows ahead as well).
 struct BwdRows {
     float ma[kRing][3], mb[kRing][3];  // map rows in flight
     float xo[kRing], yo[kRing];        // img1 / img2 at the output row completed `ahead` rows on
+    Row m[3], r1, r2;                  // the next rows to load
+    Row g;                             // the next gradient row
 };
 
 // Output row j of a backward unit, complete in ring slot kSlot, with its pixel
 // in xo / yo slot kPix: its gradient; the slot is then cleared.
 template <int kSlot, int kPix>
-__device__ __forceinline__ void backward_out(const Planes &p, const Tile &tl, int j,
-                                             const BwdRows &r, float (&acc)[kRing][3], float up,
-                                             float *bg, int gs2, int gs3) {
-    const int gx = tl.ox + (int)(threadIdx.x % kWave);
+__device__ __forceinline__ void backward_out(const Planes &p, const Out &out, int j, BwdRows &r,
+                                             float (&acc)[kRing][3], float up, uint32_t col,
+                                             int row_stride) {
     float(&a)[3] = acc[kSlot];
-    const int gy = tl.oy + j;
-    if (j < BwdShape::rows && gy < p.height && gx < p.width) {
-        int row = gy;
-        asm volatile("" : "+s"(row));  // the address is formed here, not ahead
+    if (j < out.end) {
         const float x = img1_value(p, r.xo[kPix]), y = r.yo[kPix];  // an in-image pixel
-        store_at(bg + row * gs2, (uint32_t)gx * (uint32_t)gs3 * 4u,
-                 up * (a[0] + 2.0f * x * a[1] + y * a[2]));
+        const float v = up * (a[0] + 2.0f * x * a[1] + y * a[2]);
+        if (out.col_in) store_at(r.g.at, col, v);
+        r.g.next(row_stride);
     }
 #pragma unroll
     for (int q = 0; q < 3; ++q) a[q] = 0.0f;
@@ -530,33 +575,27 @@ __device__ __forceinline__ void backward_out(const Planes &p, const Tile &tl, in
 // emitted while this row's taps are read.
 template <bool kFirst, int S>
 __device__ __forceinline__ void backward_row(const Planes &p, const Window &win, const Tile &tl,
-                                             const Cols &c, const float *m0, const float *m1,
-                                             const float *m2, const float *b1, const float *b2,
-                                             float4 *line, int ri, BwdRows &r,
-                                             float (&acc)[kRing][3], float up, float *bg,
-                                             int gs2, int gs3) {
+                                             const Cols &c, const Out &out, float4 *line, int ri,
+                                             BwdRows &r, float (&acc)[kRing][3], float up,
+                                             uint32_t col, int row_stride) {
     const int lane = threadIdx.x % kWave;
-    const int64_t base = (int64_t)tl.plane * p.height * p.width;
-    constexpr int kNext = (S + BwdShape::ahead) % kRing;
-    {  // (rows past the walk load in-image values that are never used)
-        load_map_row(p, m0, m1, m2, base, tl.oy - kRadius + ri + BwdShape::ahead, c,
-                     r.ma[kNext], r.mb[kNext]);
-        // the pixel of the output row that row ri + ahead completes
-        load_pixel(p, b1, b2, tl.oy + ri + BwdShape::ahead - 2 * kRadius, c, r.xo[kNext],
-                   r.yo[kNext]);
-    }
-    bool ina, inb;
-    row_inside(p, tl.oy - kRadius + ri, c, ina, inb);
-    line[lane] = ina ? make_float4(r.ma[S][0], r.ma[S][1], r.ma[S][2], 0.0f)
-                     : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    constexpr int kNext = (S + kBwdAhead) % kRing;
+    // (rows past the walk are loaded and never used)
+    load_map_row(p, r.m, tl.oy - kRadius + ri + kBwdAhead, c, r.ma[kNext], r.mb[kNext]);
+    // the pixel of the output row that row ri + ahead completes
+    load_pixel(p, r.r1, r.r2, tl.oy + ri + kBwdAhead - 2 * kRadius, c, r.xo[kNext],
+               r.yo[kNext]);
+    line[lane] = make_float4(c.ina ? r.ma[S][0] : 0.0f, c.ina ? r.ma[S][1] : 0.0f,
+                             c.ina ? r.ma[S][2] : 0.0f, 0.0f);
     if (c.has_b)
-        line[kWave + lane] = inb ? make_float4(r.mb[S][0], r.mb[S][1], r.mb[S][2], 0.0f)
-                                 : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        line[kWave + lane] = make_float4(c.inb ? r.mb[S][0] : 0.0f, c.inb ? r.mb[S][1] : 0.0f,
+                                         c.inb ? r.mb[S][2] : 0.0f, 0.0f);
     line_sync();
     f4v v[kTaps];
     read_taps(line, v);
     if constexpr (!kFirst)
-        backward_out<S, (S + kRing - 1) % kRing>(p, tl, ri - kRing, r, acc, up, bg, gs2, gs3);
+        backward_out<S, (S + kRing - 1) % kRing>(p, out, ri - kRing, r, acc, up, col,
+                                                 row_stride);
     taps_ready(v);
     float h[3];
     filter_taps<3>(win, v, h);
@@ -566,16 +605,13 @@ __device__ __forceinline__ void backward_row(const Planes &p, const Window &win,
 
 template <bool kFirst, int S = 0>
 __device__ __forceinline__ void backward_rows(const Planes &p, const Window &win, const Tile &tl,
-                                              const Cols &c, const float *m0, const float *m1,
-                                              const float *m2, const float *b1, const float *b2,
-                                              float4 *line, int base, BwdRows &r,
-                                              float (&acc)[kRing][3], float up, float *bg,
-                                              int gs2, int gs3) {
+                                              const Cols &c, const Out &out, float4 *line,
+                                              int base, BwdRows &r, float (&acc)[kRing][3],
+                                              float up, uint32_t col, int row_stride) {
     if constexpr (S < kRing) {
-        backward_row<kFirst, S>(p, win, tl, c, m0, m1, m2, b1, b2, line, base + S, r, acc, up,
-                                bg, gs2, gs3);
-        backward_rows<kFirst, S + 1>(p, win, tl, c, m0, m1, m2, b1, b2, line, base, r, acc, up,
-                                     bg, gs2, gs3);
+        backward_row<kFirst, S>(p, win, tl, c, out, line, base + S, r, acc, up, col, row_stride);
+        backward_rows<kFirst, S + 1>(p, win, tl, c, out, line, base, r, acc, up, col,
+                                     row_stride);
     }
 }
 
@@ -584,60 +620,78 @@ __global__ __launch_bounds__(kThreads) void ssim_backward_kernel(
     const float *__restrict__ d_xx, const float *__restrict__ d_xy, float *__restrict__ grad,
     int64_t gs0, int64_t gs1, int gs2, int gs3, float grad_scale) {
     __shared__ float4 lines[kUnitWaves][kInX];
+        taps_to_vector(win);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     float4 *line = lines[wave];
     const float up = grad_scale * *grad_mean;
     const int blk = xcd_block((int)blockIdx.x, (int)gridDim.x);
     for (int t = blk * kUnitWaves + wave; t < p.tiles;
          t += (int)gridDim.x * kUnitWaves) {
-        const Tile tl = tile_of<BwdShape::rows>(p, t);
+        const Tile tl = tile_of(p, t);
         const Cols c = cols_of(p, tl);
-        const float *b1 = p.img1 + ((int64_t)tl.b * p.s1[0] + (int64_t)tl.c * p.s1[1]);
-        const float *b2 = p.img2 + ((int64_t)tl.b * p.s2[0] + (int64_t)tl.c * p.s2[1]);
-        float *bg = grad + ((int64_t)tl.b * gs0 + (int64_t)tl.c * gs1);
-        const int64_t base = (int64_t)tl.plane * p.height * p.width;
+        const Out out = out_of(p, tl);
+        const uint32_t col = (uint32_t)(tl.ox + (int)(threadIdx.x % kWave)) * (uint32_t)gs3 * 4u;
+        const int64_t at = ((int64_t)tl.plane * p.height + tl.oy - kRadius) * p.width;
         BwdRows r;
+        r.m[0].at = d_mu + at;
+        r.m[1].at = d_xx + at;
+        r.m[2].at = d_xy + at;
+        r.r1.at = row_of(p.img1, p.s1, p.r1, tl, tl.oy - 2 * kRadius);
+        r.r2.at = row_of(p.img2, p.s2, p.r2, tl, tl.oy - 2 * kRadius);
+        r.g.at = grad + ((int64_t)tl.b * gs0 + (int64_t)tl.c * gs1 + (int64_t)tl.oy * gs2);
         float acc[kRing][3];
 #pragma unroll
         for (int k = 0; k < kRing; ++k)
 #pragma unroll
             for (int q = 0; q < 3; ++q) acc[k][q] = 0.0f;
 #pragma unroll
-        for (int d = 0; d < BwdShape::ahead; ++d) {
-            load_map_row(p, d_mu, d_xx, d_xy, base, tl.oy - kRadius + d, c, r.ma[d], r.mb[d]);
+        for (int d = 0; d < kBwdAhead; ++d) {
+            load_map_row(p, r.m, tl.oy - kRadius + d, c, r.ma[d], r.mb[d]);
             // (row d completes no output row: d < 2 kRadius)
-            load_pixel(p, b1, b2, tl.oy + d - 2 * kRadius, c, r.xo[d], r.yo[d]);
+            load_pixel(p, r.r1, r.r2, tl.oy + d - 2 * kRadius, c, r.xo[d], r.yo[d]);
         }
-        backward_rows<true>(p, win, tl, c, d_mu, d_xx, d_xy, b1, b2, line, 0, r, acc, up, bg,
-                            gs2, gs3);
-        for (int rb = kRing; rb < BwdShape::walk; rb += kRing)
-            backward_rows<false>(p, win, tl, c, d_mu, d_xx, d_xy, b1, b2, line, rb, r, acc, up,
-                                 bg, gs2, gs3);
-        constexpr int kLast = BwdShape::walk % kRing;  // the last input row's output
-        backward_out<kLast, (kLast + kRing - 1) % kRing>(p, tl, BwdShape::walk - kRing, r, acc,
-                                                         up, bg, gs2, gs3);
+        backward_rows<true>(p, win, tl, c, out, line, 0, r, acc, up, col, gs2);
+        for (int rb = kRing; rb < p.walk; rb += kRing)
+            backward_rows<false>(p, win, tl, c, out, line, rb, r, acc, up, col, gs2);
+        // the output row the last input row completed
+        backward_out<0, kRing - 1>(p, out, p.walk - kRing, r, acc, up, col, gs2);
     }
+}
+
+struct Geometry {
+    int tiles_x, tiles_y, tiles;
+    int rows;
+    int blocks;
+};
+
+// Output rows of a unit: a multiple of kRing plus 1, so that its input rows
+// (2 kRadius more) are whole turns of the ring.  The lowest units of at most
+// kTargetUnits: three waves on each of the 1024 SIMDs (what the registers
+// allow) are resident at once then, so every unit runs in the same pass over
+// the GPU.  Low units give a small image more waves (3 x 547 x 979: units of 12
+// rows 20 us, of 23 rows 22, of 45 rows 30); once the SIMDs are full the halo
+// rows decide, and a second pass with few waves costs most (2 x 3 x 1063 x 1599:
+// 2850 units of 56 rows 58 us, 3600 of 45 rows 64, 6900 of 23 rows 75;
+// 3 x 720 x 1280: 1920 units of 23 rows 24 us, 3600 of 12 rows 28).
+int unit_rows(int64_t strips, int32_t height) {
+    const int64_t per_strip = strips < kTargetUnits ? kTargetUnits / strips : 1;
+    const int64_t rows = (height + per_strip - 1) / per_strip;
+    const int64_t turns = (rows - 1 + kRing - 1) / kRing;
+    return (int)(turns < 1 ? 1 : turns < kMaxTurns ? turns : kMaxTurns) * kRing + 1;
 }
 
 // Workgroups: one per kUnitWaves units, at most kMaxBlocks (their waves then
 // take several units each).  The count depends on the image geometry alone, so
 // the per-workgroup partial sums, and so the mean, do not depend on the device.
-constexpr int kMaxBlocks = 1024;
-
-struct Geometry {
-    int tiles_x, tiles_y, tiles;
-    int blocks;
-};
-
-// Units of kRows output rows.
-template <int kRows>
 bool geometry(int32_t batch, int32_t channels, int32_t height, int32_t width, Geometry &g) {
     if (batch <= 0 || channels <= 0 || height <= 0 || width <= 0) return false;
     const int64_t planes = (int64_t)batch * channels;
     if (planes > 65535) return false;
     g.tiles_x = ceil_div(width, kTileX);
-    g.tiles_y = ceil_div(height, kRows);
-    const int64_t tiles = planes * g.tiles_x * g.tiles_y;
+    const int64_t strips = planes * g.tiles_x;
+    g.rows = unit_rows(strips, height);
+    g.tiles_y = ceil_div(height, g.rows);
+    const int64_t tiles = strips * g.tiles_y;
     if (tiles > 0x7fffffffLL) return false;
     g.tiles = (int)tiles;
     const int per = ceil_div(g.tiles, kUnitWaves);
@@ -677,6 +731,8 @@ int fill_planes(Planes &p, const Geometry &g, const float *img1, const int64_t *
     p.tiles_x = g.tiles_x;
     p.tiles_y = g.tiles_y;
     p.tiles = g.tiles;
+    p.rows = g.rows;
+    p.walk = ceil_div(g.rows + 2 * kRadius, kRing) * kRing;
     p.valid = valid ? 1 : 0;
     p.inv_count = 0.0f;
     p.inv1 = 1.0f;
@@ -699,7 +755,7 @@ using namespace gs;
 extern "C" int gs_ssim_workspace_size(int32_t batch, int32_t channels, int32_t height,
                                       int32_t width, size_t *bytes) {
     Geometry g;
-    if (!bytes || !geometry<FwdShape::rows>(batch, channels, height, width, g))
+    if (!bytes || !geometry(batch, channels, height, width, g))
         return GS_ERR_INVALID_ARGUMENT;
     *bytes = (size_t)g.blocks * sizeof(double);
     return GS_OK;
@@ -718,7 +774,7 @@ int ssim_forward_impl(const float *img1, const int64_t *strides1, const float *i
                       size_t capacity, hipStream_t stream) {
     Geometry g;
     Planes p;
-    if (!geometry<FwdShape::rows>(batch, channels, height, width, g) || !ssim_mean ||
+    if (!geometry(batch, channels, height, width, g) || !ssim_mean ||
         !(img1_divisor > 0.0f))
         return GS_ERR_INVALID_ARGUMENT;
     if (loss && !other_loss) return GS_ERR_INVALID_ARGUMENT;
@@ -737,7 +793,7 @@ int ssim_forward_impl(const float *img1, const int64_t *strides1, const float *i
     st = launch_status();
     if (st) return st;
     hipLaunchKernelGGL(ssim_mean_kernel, dim3(1), dim3(kThreads), 0, stream,
-                       (const double *)partials, (int64_t)g.blocks, count, ssim_mean, other_loss,
+                       (const double *)partials, g.blocks, count, ssim_mean, other_loss,
                        lambda, loss);
     return launch_status();
 }
@@ -804,7 +860,7 @@ extern "C" int gs_ssim_forward_noalloc(const float *img1, const int64_t *strides
                                        float *dm_dsigma12, const float *other_loss, float lambda,
                                        float *loss, hipStream_t stream) {
     Geometry g;
-    if (!geometry<FwdShape::rows>(batch, channels, height, width, g))
+    if (!geometry(batch, channels, height, width, g))
         return GS_ERR_INVALID_ARGUMENT;
     // the partials the launch needs must fit the static array (always true:
     // geometry() caps the workgroups at kMaxBlocks)
@@ -827,7 +883,7 @@ extern "C" int gs_ssim_backward(const float *grad_mean, const float *img1,
                                 const int64_t *grad_strides, hipStream_t stream) {
     Geometry g;
     Planes p;
-    if (!geometry<BwdShape::rows>(batch, channels, height, width, g) || !(img1_divisor > 0.0f))
+    if (!geometry(batch, channels, height, width, g) || !(img1_divisor > 0.0f))
         return GS_ERR_INVALID_ARGUMENT;
     int st = fill_planes(p, g, img1, strides1, img2, strides2, channels, height, width, 0);
     if (st) return st;

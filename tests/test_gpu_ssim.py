@@ -57,6 +57,22 @@ def test_ssim_matches_oracle(gpu, shape, padding):
     check_against_oracle(a, b, padding, val, grad, grad_out=0.37)
 
 
+# Unit heights follow the geometry (12, 23, 34, ... rows; at most 3072 units of 64
+# columns where that can be): one unit exactly and one row more; 300 strips of 130
+# rows: 23-row units; 4000 strips: one unit of 34 rows each; 4300: more units than
+# the waves of 1024 workgroups, so some take two.
+@pytest.mark.parametrize("shape", [(1, 1, 12, 64), (1, 2, 13, 65), (100, 3, 130, 64),
+                                   (1000, 4, 25, 7), (2150, 2, 13, 6)])
+@pytest.mark.parametrize("padding", ["same", "valid"])
+def test_unit_heights(gpu, shape, padding):
+    a, b = images(shape, seed=sum(shape))
+    val, grad = run(a.to(gpu), b.to(gpu), padding, grad_out=0.37)
+    if padding == "valid" and (shape[2] <= 10 or shape[3] <= 10):
+        assert torch.isnan(val)  # no pixel at least 5 from the border
+        return
+    check_against_oracle(a, b, padding, val, grad, grad_out=0.37)
+
+
 def test_reference_call_layout_full_size(gpu):
     """(H, W, 3) images permuted to (1, 3, H, W) as the reference does, at
     1920x1080: same values as the contiguous call, gradient laid out like img1."""

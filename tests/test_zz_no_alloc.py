@@ -6,9 +6,8 @@ device array instead of a caller workspace, so its outputs -- the mean, the
 three derivative maps and the combined loss -- must equal gs_ssim_forward's bit
 for bit (the mean is reduced in a fixed order).  Checked on two calls in a row,
 each with a smaller input than the one before (the array then still holds
-the earlier call's partials past the later call's workgroup count; the first
-fills all 1024), in both orders of the two entry points, and its argument
-checks.
+the earlier call's partials past the later call's workgroup count), in both
+orders of the two entry points, and its argument checks.
 """
 
 from __future__ import annotations
@@ -66,12 +65,11 @@ def _inputs(shape_hwc, seed, permuted, gpu):
             y.permute(2, 0, 1).contiguous().unsqueeze(0).to(gpu))
 
 
-# Units of 64 columns x 34 output rows per plane, 4 per workgroup, at most 1024
-# workgroups (the static array's size).  2160x3840x3: 60 x 64 x 3 = 11520 units,
-# 2880 workgroups capped at 1024, so the array is filled to capacity; then
-# 720x1280x3: 20 x 22 x 3 = 1320 units, 330 workgroups; then 32x96x3: 2 x 1 x 3 =
-# 6 units, 2 workgroups (every partial past the second still holds an earlier
-# call's value)
+# Units of 64 columns per plane, 4 per workgroup, at most 1024 workgroups (the
+# static array's size).  2160x3840x3: 60 x 17 x 3 = 3060 units of 133 output rows,
+# 765 workgroups; then 720x1280x3: 20 x 32 x 3 = 1920 units of 23 rows, 480
+# workgroups; then 32x96x3: 2 x 3 x 3 = 18 units of 12 rows, 5 workgroups (every
+# partial past the fifth still holds an earlier call's value)
 CALLS = [((2160, 3840, 3), 4, True, 0, 255.0), ((720, 1280, 3), 1, True, 1, 255.0),
          ((32, 96, 3), 2, False, 0, 255.0)]
 
