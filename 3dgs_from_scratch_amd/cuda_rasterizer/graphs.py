@@ -27,9 +27,37 @@ kernels), and none waits on the host once the capacities are set.
 
 from __future__ import annotations
 
+import contextlib
+import gc
+import threading
+
 import torch
 
 import cuda_rasterizer as _cr
+
+_hold_lock = threading.Lock()
+_holds = [0, False]  # captures in progress; whether the collector was on before the first
+
+
+@contextlib.contextmanager
+def _collector_held():
+    """Keeps the cyclic garbage collector from running during a capture (of any
+    thread).  A step that a cycle of references holds -- its function refers to
+    the object that owns it -- is freed by the collector; if that happens while
+    another step records, the dead graph's destructor makes a HIP call that a
+    capture forbids, and the process ends."""
+    with _hold_lock:
+        if _holds[0] == 0:
+            _holds[1] = gc.isenabled()
+            gc.disable()
+        _holds[0] += 1
+    try:
+        yield
+    finally:
+        with _hold_lock:
+            _holds[0] -= 1
+            if _holds[0] == 0 and _holds[1]:
+                gc.enable()
 
 
 class CapturedStep:
@@ -62,7 +90,7 @@ class CapturedStep:
         self.graph = None  # release the previous graph's pool before capturing again
         self.output = None
         graph = torch.cuda.CUDAGraph()
-        with _cr.CapturedChecks() as sink:
+        with _collector_held(), _cr.CapturedChecks() as sink:
             with torch.cuda.graph(graph):
                 out = self._fn()
         self.graph, self.output, self.checks = graph, out, sink.checks

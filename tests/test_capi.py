@@ -238,3 +238,25 @@ def test_check_forward_order_rejects_broken_orders(n_tiles):
     for bad in (dup, across, out, neg):
         with pytest.raises(cuda_rasterizer.RasterizerError):
             cuda_rasterizer.check_forward_order(bad, n_tiles)
+
+
+def test_collector_held_during_captures():
+    """Off inside, also where captures overlap, and afterwards as it was."""
+    import gc
+
+    from cuda_rasterizer.graphs import _collector_held
+
+    was = gc.isenabled()
+    try:
+        for on in (True, False):
+            gc.enable() if on else gc.disable()
+            first, second = _collector_held(), _collector_held()
+            first.__enter__()
+            assert not gc.isenabled()
+            second.__enter__()
+            first.__exit__(None, None, None)
+            assert not gc.isenabled()
+            second.__exit__(None, None, None)
+            assert gc.isenabled() == on
+    finally:
+        gc.enable() if was else gc.disable()
