@@ -30,7 +30,7 @@ import time
 import torch
 
 from . import _lib
-from ._lib import RasterizerError
+from ._lib import RasterizerError, on_device as _on, stream_of as _stream
 from .ssim import fused_ssim
 
 __all__ = [
@@ -82,7 +82,7 @@ def _prep(t: torch.Tensor, name: str, dtype: torch.dtype, shape: tuple, device) 
         raise RuntimeError(f"{name}: expected dtype {dtype}, got {t.dtype}")
     if device is not None and t.device != device:
         raise RuntimeError(f"{name}: expected device {device}, got {t.device}")
-    if tuple(t.shape) != tuple(shape):
+    if t.shape != shape:
         raise RuntimeError(f"{name}: expected shape {tuple(shape)}, got {tuple(t.shape)}")
     return t.contiguous()
 
@@ -96,10 +96,6 @@ def _device_of(t: torch.Tensor) -> torch.device:
             "(there is no CPU fallback)"
         )
     return t.device
-
-
-def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
 
 
 def project_points(
@@ -137,7 +133,7 @@ def project_points(
     cov_inv_image = torch.empty((n, 3), dtype=f32, device=dev)
     radii = torch.empty((n, 2), dtype=f32, device=dev)
     mask = torch.empty((n,), dtype=torch.bool, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ev = _lib.timer.record("project_points", dev)
         _lib.check(
             _lib.load().gs_project_points(
@@ -187,7 +183,7 @@ def project_points_backward(
     g_means = torch.empty((n, 3), dtype=f32, device=dev)
     g_scales = torch.empty((n, 3), dtype=f32, device=dev)
     g_quats = torch.empty((n, 4), dtype=f32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ev = _lib.timer.record("project_points_backward", dev)
         _lib.check(
             _lib.load().gs_project_points_backward(
@@ -215,7 +211,7 @@ def evaluate_spherical_harmonics(
     sh_coeffs_rest = _prep(sh_coeffs_rest, "sh_coeffs_rest", f32, (n, 15, 3), dev)
     mask = _prep(mask, "mask", torch.bool, (n,), dev)
     colors = torch.empty((n, 3), dtype=f32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ev = _lib.timer.record("evaluate_sh", dev)
         _lib.check(
             _lib.load().gs_evaluate_sh(
@@ -255,7 +251,7 @@ def evaluate_spherical_harmonics_backward(
     g_means = torch.empty((n, 3), dtype=f32, device=dev)
     g_dc = torch.empty((n, 3), dtype=f32, device=dev)
     g_rest = torch.empty((n, 15, 3), dtype=f32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ev = _lib.timer.record("evaluate_sh_backward", dev)
         _lib.check(
             _lib.load().gs_evaluate_sh_backward(
@@ -335,7 +331,7 @@ def _tile_intersection(points_image, radii, depths, mask, width, height, tile_si
                            "which a graph capture cannot wait for (render through "
                            "render_l1 or render(), whose capped sort needs no host read)")
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _on(dev):
         stream = _stream(dev)
         sz = ctypes.c_size_t(0)
         _lib.check(lib.gs_bin_count_workspace_size(n, ctypes.byref(sz)), "workspace query")
@@ -563,7 +559,7 @@ def tile_intersection_capped(points_image, radii, depths, mask, width, height, t
     mask = _prep(mask, "mask", torch.bool, (n,), dev)
     lib = _lib.load()
     k_cap, m_cap = caps
-    with torch.cuda.device(dev):
+    with _on(dev):
         stream = _stream(dev)
         sz = ctypes.c_size_t(0)
         _lib.check(lib.gs_bin_count_workspace_size(n, ctypes.byref(sz)), "workspace query")
@@ -668,7 +664,7 @@ def rasterize(
         indexing_offset, gaussian_ids_sorted, points_image, cov_inv_image, opacities, colors)
     width, height = int(width), int(height)
     image = torch.empty((height, width, 3), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ev = _lib.timer.record("rasterize", dev)
         _lib.check(
             _lib.load().gs_rasterize(
@@ -715,7 +711,7 @@ def _backward_split(*args, **kw):
     and their copy costs a few microseconds: 72 MB moved at 1M Gaussians."""
     blend = args[3]
     dev, n = blend[0], blend[1]
-    with torch.cuda.device(dev):
+    with _on(dev):
         rows = torch.zeros((9 * n,), dtype=torch.float32, device=dev)
         _backward_rows(*args, rows=rows, **kw)
         out = _blend_grad_views(torch.empty_like(rows), n)
@@ -862,7 +858,7 @@ def rasterize_work(indexing_offset, gaussian_ids_sorted, points_image, cov_inv_i
     dev, n, off, ids, pts, conic, opac, _ = _blend_inputs(
         indexing_offset, gaussian_ids_sorted, points_image, cov_inv_image, opacities, colors)
     counters = torch.empty((2,), dtype=torch.int64, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.check(
             _lib.load().gs_rasterize_work(
                 _ptr(off), _ptr(ids), off.shape[0], ids.shape[0], _ptr(pts), _ptr(conic),
@@ -945,7 +941,7 @@ def evaluate_spherical_harmonics_render(world_to_camera, points_world, sh_coeffs
         colors = out
     if sh_cache is not None:
         _check_sh_cache(sh_cache, n, dev, "evaluate_spherical_harmonics_render")
-    with torch.cuda.device(dev):
+    with _on(dev):
         ev = _lib.timer.record("evaluate_sh_render", dev, stream)
         lib = _lib.load()
         launch = _stream(dev) if stream is None else stream.cuda_stream
@@ -989,7 +985,7 @@ def evaluate_spherical_harmonics_render_backward(grad_colors, world_to_camera, p
         g_means = torch.empty((n, 3), dtype=f32, device=dev)
     g_dc = torch.empty((n, 3), dtype=f32, device=dev)
     g_rest = torch.empty((n, 15, 3), dtype=f32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ev = _lib.timer.record("evaluate_sh_render_backward", dev)
         _lib.check(
             _lib.load().gs_evaluate_sh_render_backward(
@@ -1022,7 +1018,7 @@ def rasterize_display(indexing_offset, gaussian_ids_sorted, points_image, cov_in
     _check_order(forward_order, schedule, off.shape[0], dev, "rasterize_display")
     image = torch.empty((height, width, 3), dtype=torch.float32, device=dev)
     display = torch.empty((height, width, 3), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ev = _lib.timer.record("rasterize_display", dev)
         _lib.check(
             _lib.load().gs_rasterize_display(
@@ -1074,7 +1070,7 @@ def activate(log_scales, quats_raw, opacity_logits):
     scales = torch.empty((n, 3), dtype=f32, device=dev)
     quats = torch.empty((n, 4), dtype=f32, device=dev)
     opac = torch.empty((n,), dtype=f32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ev = _lib.timer.record("activate", dev)
         _lib.check(_lib.load().gs_activate(_ptr(log_scales), _ptr(quats_raw), _ptr(opacity_logits),
                                            n, _ptr(scales), _ptr(quats), _ptr(opac), _stream(dev)),
@@ -1097,7 +1093,7 @@ def activate_backward(grad_scales, grad_quats, grad_opacities, scales, quats_raw
     g_ls = torch.empty((n, 3), dtype=f32, device=dev)
     g_q = torch.empty((n, 4), dtype=f32, device=dev)
     g_l = torch.empty((n,), dtype=f32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ev = _lib.timer.record("activate_backward", dev)
         _lib.check(_lib.load().gs_activate_backward(
             _ptr(gs_), _ptr(gq), _ptr(go), _ptr(scales), _ptr(quats_raw), _ptr(opacities), n,
@@ -1138,7 +1134,7 @@ def preprocess_forward(means, log_scales, quats_raw, opacity_logits, sh_coeffs_d
            for shape in ((n, 2), (n,), (n, 3), (n, 3), (n, 2))]
     mask = torch.empty((n,), dtype=torch.bool, device=dev)
     opac = torch.empty((n,), dtype=f32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ev = _lib.timer.record("preprocess_forward" if with_colors else "preprocess_project", dev)
         _lib.check(_lib.load().gs_preprocess_forward(
             _ptr(means), _ptr(log_scales), _ptr(quats_raw), _ptr(opacity_logits), _ptr(dc),
@@ -1213,7 +1209,7 @@ def _preprocess_backward(entry, grads, means, log_scales, quats_raw, opacity_log
     intrinsic = _prep(intrinsic, "intrinsic", f32, (3, 3), dev)
     outs = [torch.empty(shape, dtype=f32, device=dev)
             for shape in ((n, 3), (n, 3), (n, 4), (n,), (n, 3), (n, 15, 3))]
-    with torch.cuda.device(dev):
+    with _on(dev):
         ev = _lib.timer.record("preprocess_backward", dev)
         _lib.check(getattr(_lib.load(), entry)(
             *(_ptr(g) for g in grads), _ptr(means), _ptr(log_scales), _ptr(quats_raw),
@@ -1251,7 +1247,7 @@ def render_preprocess_backward(grad_points_image, grad_cov_inv_image, grad_color
     intrinsic = _prep(intrinsic, "intrinsic", f32, (3, 3), dev)
     outs = [torch.empty(shape, dtype=f32, device=dev)
             for shape in ((n, 3), (n, 3), (n, 4), (n, 3), (n, 15, 3))]
-    with torch.cuda.device(dev):
+    with _on(dev):
         ev = _lib.timer.record("render_preprocess_backward", dev)
         _lib.check(_lib.load().gs_render_preprocess_backward(
             _ptr(g_pts), _ptr(g_conic), _ptr(g_col), _ptr(means), _ptr(scales),
@@ -1306,7 +1302,7 @@ def rasterize_display_l1(indexing_offset, gaussian_ids_sorted, points_image, cov
         _check_order(forward_order, schedule, n_tiles, dev, "rasterize_display_l1")
         fwd_order = forward_order
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _on(dev):
         ev = _lib.timer.record("rasterize_display_l1", dev)
         _lib.check(lib.gs_rasterize_display_l1(
             _ptr(off), _ptr(ids), n_tiles, ids.shape[0], _ptr(pts), _ptr(conic), _ptr(opac),
@@ -1368,7 +1364,7 @@ def rasterize_l1_backward(target, grad_loss, indexing_offset, gaussian_ids_sorte
                                extra=extra, schedule=schedule)
     _check_accumulators(accumulators, n, dev, "rasterize_l1_backward")
     g_pts, g_conic, g_opac, g_col = _blend_grad_views(accumulators, n)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ev = _lib.timer.record("rasterize_l1_backward", dev)
         _lib.check(_lib.load().gs_rasterize_l1_backward(
             _ptr(target), _ptr(gl), _ptr(img), _ptr(off), _ptr(ids), off.shape[0], ids.shape[0],
@@ -1396,7 +1392,7 @@ def rasterize_l1_backward_rows(target, grad_loss, indexing_offset, gaussian_ids_
     if accumulators is None:
         accumulators = torch.zeros((9 * n,), dtype=torch.float32, device=dev)
     _check_accumulators(accumulators, n, dev, "rasterize_l1_backward_rows")
-    with torch.cuda.device(dev):
+    with _on(dev):
         _backward_rows("rasterize_l1_backward", _SEED_L1, target, blend, int(width), int(height),
                        16, alpha_threshold, transmittance_threshold, chi_squared_threshold, img,
                        rows=accumulators, grad_loss=gl, loss_scale=loss_scale, extra=extra,

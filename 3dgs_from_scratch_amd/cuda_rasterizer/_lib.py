@@ -2,8 +2,11 @@
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
+
+import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libgsraster.so")
@@ -123,6 +126,21 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+def stream_of(device: torch.device) -> int:
+    """The current stream's handle (torch.cuda.current_stream(device).cuda_stream
+    without the Stream object: 0.2 instead of 2.5 us a call)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+_ENTERED = contextlib.nullcontext()
+
+
+def on_device(device: torch.device):
+    """torch.cuda.device(device), or nothing to enter where `device` is the current
+    one already: a step enters it nine times, at 2 to 3 us each."""
+    return _ENTERED if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
+
+
 class StageTimer:
     """Opt-in HIP-event timing of entry points on the stream they launch on.
 
@@ -145,8 +163,6 @@ class StageTimer:
         self._used = 0
 
     def _event(self):
-        import torch
-
         if self._used == len(self._pool):
             self._pool.append(torch.cuda.Event(enable_timing=True))
         ev = self._pool[self._used]
@@ -154,8 +170,6 @@ class StageTimer:
         return ev
 
     def record(self, stage: str, device, stream=None):
-        import torch
-
         if not self.enabled or (self.only is not None and stage not in self.only):
             return None
         ev = (self._event(), self._event())
@@ -164,14 +178,10 @@ class StageTimer:
         return ev
 
     def stop(self, ev, device, stream=None):
-        import torch
-
         if ev is not None:
             ev[1].record(stream if stream is not None else torch.cuda.current_stream(device))
 
     def summary(self) -> dict:
-        import torch
-
         torch.cuda.synchronize()
         return {k: (len(v), sum(a.elapsed_time(b) for a, b in v)) for k, v in self.events.items()}
 

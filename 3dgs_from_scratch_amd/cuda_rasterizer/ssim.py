@@ -74,7 +74,7 @@ def ssim_forward(img1: torch.Tensor, img2: torch.Tensor, padding: str = "same",
     maps = (tuple(torch.empty((b * c, h, w), dtype=torch.float32, device=dev) for _ in range(3))
             if with_maps else (None, None, None))
     s1, s2 = _strides(img1), _strides(img2)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         ev = _lib.timer.record("ssim_forward", dev)
         _lib.check(lib.gs_ssim_forward(
             img1.data_ptr(), _sp(s1), img2.data_ptr(), _sp(s2), b, c, h, w,
@@ -82,7 +82,7 @@ def ssim_forward(img1: torch.Tensor, img2: torch.Tensor, padding: str = "same",
             *(None if m is None else m.data_ptr() for m in maps),
             None if other_loss is None else other_loss.data_ptr(), float(lam),
             None if loss is None else loss.data_ptr(), ws.data_ptr(), int(sz.value),
-            torch.cuda.current_stream(dev).cuda_stream), "ssim_forward")
+            _lib.stream_of(dev)), "ssim_forward")
         _lib.timer.stop(ev, dev)
     if other_loss is not None:
         return mean, maps, loss
@@ -100,12 +100,12 @@ def ssim_backward(grad_mean: torch.Tensor, img1: torch.Tensor, img2: torch.Tenso
     g = grad_mean.reshape(1).to(device=dev, dtype=torch.float32).contiguous()
     grad = torch.empty_like(img1)
     s1, s2, sg = _strides(img1), _strides(img2), _strides(grad)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         ev = _lib.timer.record("ssim_backward", dev)
         _lib.check(_lib.load().gs_ssim_backward(
             g.data_ptr(), img1.data_ptr(), _sp(s1), img2.data_ptr(), _sp(s2), b, c, h, w,
             float(img1_divisor), *(m.data_ptr() for m in maps), float(grad_scale),
-            grad.data_ptr(), _sp(sg), torch.cuda.current_stream(dev).cuda_stream),
+            grad.data_ptr(), _sp(sg), _lib.stream_of(dev)),
             "ssim_backward")
         _lib.timer.stop(ev, dev)
     return grad

@@ -42,7 +42,7 @@ def _ptr(t):
 
 
 def _stream(t):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return _lib.stream_of(t.device)
 
 
 class FusedAdam:
@@ -78,7 +78,7 @@ class FusedAdam:
         if specs:
             arr = (GsAdamTensor * len(specs))(*specs)
             dev = next(iter(self.params.values()))
-            with torch.no_grad(), torch.cuda.device(dev.device):
+            with torch.no_grad(), _lib.on_device(dev.device):
                 _lib.check(_lib.load().gs_adam_step(arr, len(specs), self.beta1, self.beta2,
                                                     self.eps, _stream(dev)), "adam_step")
         if "means" in self.lr:
@@ -115,7 +115,7 @@ class Densifier:
             g = g.contiguous()
         stride = g.stride(0) if g.dim() == 2 else 2
         r = radii.detach().contiguous()
-        with torch.cuda.device(g.device):
+        with _lib.on_device(g.device):
             _lib.check(_lib.load().gs_accumulate_grad2d_strided(
                 _ptr(g), stride, _ptr(r), n, int(width), int(height), _ptr(self.grads),
                 _ptr(self.count), _stream(g)), "accumulate_grad2d")
@@ -148,7 +148,7 @@ class Densifier:
                     specs.append(GsGatherTensor(_ptr(store[k]), _ptr(s_dst), None, width, 1))
                     keep.append((store, k, s_dst))
         arr = (GsGatherTensor * len(specs))(*specs)
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             _lib.check(_lib.load().gs_gather_rows(n_out, _ptr(src_rows), _ptr(fresh), arr,
                                                   len(specs), _stream(src_rows)), "gather_rows")
         for item in keep:
