@@ -702,22 +702,38 @@ int radix_pass(const KeyT *kin, const uint32_t *vin, KeyT *kout, uint32_t *vout,
 // followed by segment_sort_kernel: each workgroup takes the buckets that begin
 // in its nominal range of kSegChunk positions and sorts them by the full key,
 // stably, so that the result is ordered by (key, index) as a full 32-bit
-// stable sort is.  A chunk of at most kSegMax keys is sorted in LDS (LSD
-// passes of at most 8 bits over the bits below its highest differing bit); a
-// larger one (a bucket of more than about kSegMax - kSegChunk keys: exact ties,
-// or depths packed far more densely than elsewhere) is sorted by the same
-// workgroup through global memory.
+// stable sort is.  Three ways, by how crowded the chunk's buckets are:
+//  - a scene's depths: the chunk's key range cut into kSegSubs even sub-buckets,
+//    about one key each.  A counter's atomic places a key in its sub-bucket, in any
+//    order; its rank there is the keys (and, among equal keys, the positions) below
+//    it.  One pass whatever the range, and the rectangles' gather runs under it.
+//  - more than kSegSubMax keys in a sub-bucket (ties), up to kSegMax keys: LSD passes
+//    in LDS, of at most 8 bits, over the bits below the highest differing bit.
+//  - a larger one (exact ties, or depths packed far more densely than
+//    elsewhere): the same passes through global memory.
 constexpr int kSegThreads = 256;
 constexpr int kSegWaves = kSegThreads / kWave;
 constexpr int kSegItems = 4;
 constexpr int kSegMax = kSegThreads * kSegItems;  // keys of a chunk sorted in LDS
 constexpr int kSegChunk = 512;                    // nominal positions per workgroup
+// Positions a workgroup loads to find its chunk: kSegChunk and a third item per
+// thread, for the bucket that runs over the range's end.  One that runs further is
+// searched for in global memory.
+constexpr int kSegWindowItems = 3;
+constexpr int kSegWindow = kSegThreads * kSegWindowItems;
+static_assert(kSegWindow > kSegChunk && kSegWindow <= kSegMax, "window within the LDS chunk");
 static_assert(kSegMax < 65536, "window counts are packed in 16 bits");
+constexpr int kSegSubBits = 10;
+constexpr int kSegSubs = 1 << kSegSubBits;
+static_assert(kSegSubs == 4 * kSegThreads && kSegSubs == kSegWaves * kRadixMax,
+              "four counters a thread, in wave_count's words");
+// A sub-bucket's largest count: its keys are compared pairwise.
+constexpr uint32_t kSegSubMax = 48;
 
 struct SegLds {
     uint32_t keys[2][kSegMax];
     uint32_t vals[2][kSegMax];
-    uint32_t wave_count[kSegWaves][kRadixMax];
+    alignas(16) uint32_t wave_count[kSegWaves][kRadixMax];
     uint32_t digit_start[kRadixMax];
     uint32_t running[kRadixMax];
     uint32_t scan_tmp[kSegThreads / kWave + 1];
@@ -889,12 +905,13 @@ __device__ __forceinline__ void for_each_supertile(uint2 r, int super_x, F f) {
 }
 
 // The LDS path's level-1 counts: the chunk [start, start + size) meets at most
-// three kL1Threads-position blocks (size <= kSegMax); each is counted per
+// three kL1Threads-position blocks (size <= kSegMax; item it of this thread is
+// position pos[it] of the chunk); each is counted per
 // supertile in the now free key buffer and its non-zero counts added to the
 // table.  Every thread of the workgroup calls it (it contains barriers).
 __device__ void seg_l1_counts(const SegArgs &a, uint32_t start, uint32_t size,
                               const uint2 (&r)[kSegItems], const bool (&valid)[kSegItems],
-                              int ipw, SegLds &s) {
+                              const uint32_t (&pos)[kSegItems], SegLds &s) {
     uint32_t *cnt = s.keys[0];  // 3 x kRadixMax counters
     const uint32_t b0 = start / kL1Threads;
     const uint32_t nb = (start + size - 1) / kL1Threads - b0 + 1;  // 1..3
@@ -904,7 +921,7 @@ __device__ void seg_l1_counts(const SegArgs &a, uint32_t start, uint32_t size,
 #pragma unroll
     for (int it = 0; it < kSegItems; ++it) {
         if (!valid[it]) continue;
-        const uint32_t row = (start + (uint32_t)seg_slot(it, ipw)) / kL1Threads - b0;
+        const uint32_t row = (start + pos[it]) / kL1Threads - b0;
         for_each_supertile(r[it], a.super_x,
                            [&](int st) { atomicAdd(&cnt[row * kRadixMax + st], 1u); });
     }
@@ -1012,6 +1029,12 @@ __device__ void seg_sort_global(const SegArgs &a, uint32_t start, uint32_t end, 
     }
 }
 
+// Bound by the latency of its chain (live count, transform, window, rectangles) on
+// small scenes and by the rectangles' gather (8 bytes of a memory line a key) on
+// large ones, not by its 40 bytes a key.  Comparing a key with its whole depth
+// bucket instead of a sub-bucket was slower where buckets hold over 100 keys (bin at
+// 1M Gaussians 162 us); LDS passes on every chunk took 27.8 (1M Gaussians,
+// 2560x1440) and 62.7 us (3M, 1920x1080), this takes 23.7 and 56.1.
 __global__ __launch_bounds__(kSegThreads) void segment_sort_kernel(SegArgs a) {
     __shared__ SegLds s;
     const int64_t live64 = *a.n_live;
@@ -1031,17 +1054,18 @@ __global__ __launch_bounds__(kSegThreads) void segment_sort_kernel(SegArgs a) {
     // here, which also holds the chunk's keys unless its last bucket runs past
     // the window; the buckets <= that of position lo - 1 (resp. hi - 1) form a
     // prefix of the window.
-    const uint32_t wlen = min((uint32_t)kSegMax, live - lo);
-    const int wipw = seg_items(wlen);
+    const uint32_t wlen = min((uint32_t)kSegWindow, live - lo);
     const uint32_t b_lo = lo > 0 ? bf(a.keys[lo - 1]) : 0u;
     const bool end_in = hi < live;  // else end = live
     const uint32_t b_hi = end_in ? bf(a.keys[hi - 1]) : 0u;
-    uint32_t wk[kSegItems], wv[kSegItems];
+    // item it of this thread is position it * kSegThreads + threadIdx.x of the window,
+    // so that all waves share a chunk of kSegChunk keys
+    uint32_t wk[kSegWindowItems], wv[kSegWindowItems];
     uint32_t c_lo = 0, c_hi = 0;
 #pragma unroll
-    for (int it = 0; it < kSegItems; ++it) {
-        const uint32_t j = (uint32_t)seg_slot(it, wipw);
-        const bool in = it < wipw && j < wlen;
+    for (int it = 0; it < kSegWindowItems; ++it) {
+        const uint32_t j = (uint32_t)(it * kSegThreads) + threadIdx.x;
+        const bool in = j < wlen;
         wk[it] = in ? a.keys[lo + j] : 0u;
         wv[it] = in ? a.vals[lo + j] : 0u;
         c_lo += (in && lo > 0 && bf(wk[it]) <= b_lo) ? 1u : 0u;
@@ -1065,18 +1089,82 @@ __global__ __launch_bounds__(kSegThreads) void segment_sort_kernel(SegArgs a) {
         seg_sort_global(a, start, end, s);
         return;
     }
-    // LDS path: the chunk in buffer 0 (from the window, or loaded again when its
-    // last bucket runs past the window), then LSD passes between the buffers
-    if (end <= lo + wlen) {
+    // LDS paths: the chunk in buffer 0, from the window, or loaded again when its
+    // last bucket runs past the window
+    uint32_t pos[kSegItems];
+    uint2 r[kSegItems];
+    bool valid[kSegItems];
+    if (end <= lo + wlen) {  // uniform
         const uint32_t off = start - lo;
 #pragma unroll
         for (int it = 0; it < kSegItems; ++it) {
-            const uint32_t j = (uint32_t)seg_slot(it, wipw);
-            if (it < wipw && j >= off && j < off + size) {
-                s.keys[0][j - off] = wk[it];
-                s.vals[0][j - off] = wv[it];
-            }
+            pos[it] = (uint32_t)(it * kSegThreads) + threadIdx.x - off;  // unsorted, wraps before start
+            valid[it] = it < kSegWindowItems && pos[it] < size;
         }
+#pragma unroll
+        for (int it = 0; it < kSegWindowItems; ++it) {
+            if (valid[it]) s.keys[0][pos[it]] = wk[it];
+            r[it] = rect_or_empty(a.rects, valid[it] ? wv[it] : 0xFFFFFFFFu, a.n);
+        }
+        uint32_t *cnt = &s.wave_count[0][0];
+        reinterpret_cast<uint4 *>(cnt)[threadIdx.x] = make_uint4(0u, 0u, 0u, 0u);
+        __syncthreads();
+        // the range from the first bucket's lower end to the last one's upper end; keys
+        // that BucketFn clamped lie outside it and go to the end sub-buckets (still monotone)
+        const uint32_t b0 = bf(s.keys[0][0]), nb1 = bf(s.keys[0][size - 1]) - b0;  // buckets - 1
+        const uint32_t low = bf.kmin + (b0 << bf.shift);
+        const int sub_shift = max(bf.shift + (nb1 ? 32 - __clz(nb1) : 0) - kSegSubBits, 0);
+        uint32_t sub[kSegWindowItems], slot[kSegWindowItems];
+        int crowded = 0;
+#pragma unroll
+        for (int it = 0; it < kSegWindowItems; ++it) {
+            const uint32_t rel = wk[it] > low ? (wk[it] - low) >> sub_shift : 0u;
+            sub[it] = min(rel, (uint32_t)kSegSubs - 1u);
+            slot[it] = valid[it] ? atomicAdd(&cnt[sub[it]], 1u) : 0u;
+            crowded |= slot[it] >= kSegSubMax ? 1 : 0;
+        }
+        if (!__syncthreads_or(crowded)) {  // uniform
+            uint4 c = reinterpret_cast<const uint4 *>(cnt)[threadIdx.x];
+            uint32_t all;
+            const uint32_t before = block_exclusive_scan<uint32_t, kSegThreads>(
+                c.x + c.y + c.z + c.w, s.scan_tmp, all);
+            reinterpret_cast<uint4 *>(cnt)[threadIdx.x] =
+                make_uint4(before, before + c.x, before + c.x + c.y, before + c.x + c.y + c.z);
+            __syncthreads();
+            uint32_t first[kSegWindowItems], last[kSegWindowItems];
+#pragma unroll
+            for (int it = 0; it < kSegWindowItems; ++it) {
+                first[it] = cnt[sub[it]];
+                last[it] = sub[it] + 1u < (uint32_t)kSegSubs ? cnt[sub[it] + 1u] : size;
+                if (valid[it] && first[it] + slot[it] < (uint32_t)kSegMax) {
+                    s.keys[1][first[it] + slot[it]] = wk[it];
+                    s.vals[1][first[it] + slot[it]] = pos[it];
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int it = 0; it < kSegWindowItems; ++it) {
+                if (!valid[it]) continue;
+                uint32_t rank = first[it];
+                for (uint32_t e = first[it]; e < last[it]; ++e) {
+                    const uint32_t k2 = s.keys[1][e], q2 = s.vals[1][e];
+                    rank += (k2 < wk[it] || (k2 == wk[it] && q2 < pos[it])) ? 1u : 0u;
+                }
+                pos[it] = rank;
+                if (rank >= size) valid[it] = false;  // never: guards the stores
+            }
+#pragma unroll
+            for (int it = 0; it < kSegWindowItems; ++it) {
+                if (!valid[it]) continue;
+                a.vals[start + pos[it]] = wv[it];
+                seg_store(a, start + pos[it], r[it]);
+            }
+            if (a.l1_hist) seg_l1_counts(a, start, size, r, valid, pos, s);  // uniform
+            return;
+        }
+#pragma unroll
+        for (int it = 0; it < kSegWindowItems; ++it)
+            if (valid[it]) s.vals[0][pos[it]] = wv[it];
     } else {
         for (uint32_t q = threadIdx.x; q < size; q += kSegThreads) {
             s.keys[0][q] = a.keys[start + q];
@@ -1086,7 +1174,6 @@ __global__ __launch_bounds__(kSegThreads) void segment_sort_kernel(SegArgs a) {
     __syncthreads();
     const int ipw = seg_items(size);
     uint32_t k[kSegItems], v[kSegItems];
-    bool valid[kSegItems];
     uint32_t diff = 0;
     const uint32_t k0 = s.keys[0][0];
 #pragma unroll
@@ -1100,7 +1187,7 @@ __global__ __launch_bounds__(kSegThreads) void segment_sort_kernel(SegArgs a) {
     const SegPlan plan = seg_plan(seg_reduce<false>(diff, s));
     for (int p = 0; p < plan.passes; ++p) {
         const int sh = p * plan.width;
-        uint32_t pos[kSegItems], total;
+        uint32_t total;
         seg_rank(k, valid, ipw, sh, min(plan.width, plan.bits - sh), pos, s, total);
         uint32_t *dk = s.keys[(p + 1) & 1], *dv = s.vals[(p + 1) & 1];
 #pragma unroll
@@ -1122,18 +1209,18 @@ __global__ __launch_bounds__(kSegThreads) void segment_sort_kernel(SegArgs a) {
     }
     // sorted: item it of this thread is position seg_slot(it, ipw) of the chunk;
     // every rectangle is loaded before the first store, so the loads overlap
-    uint2 r[kSegItems];
 #pragma unroll
-    for (int it = 0; it < kSegItems; ++it)
+    for (int it = 0; it < kSegItems; ++it) {
+        pos[it] = (uint32_t)seg_slot(it, ipw);
         r[it] = rect_or_empty(a.rects, valid[it] ? v[it] : 0xFFFFFFFFu, a.n);
+    }
 #pragma unroll
     for (int it = 0; it < kSegItems; ++it) {
         if (!valid[it]) continue;
-        const uint32_t p = start + (uint32_t)seg_slot(it, ipw);
-        a.vals[p] = v[it];
-        seg_store(a, p, r[it]);
+        a.vals[start + pos[it]] = v[it];
+        seg_store(a, start + pos[it], r[it]);
     }
-    if (a.l1_hist) seg_l1_counts(a, start, size, r, valid, ipw, s);  // uniform
+    if (a.l1_hist) seg_l1_counts(a, start, size, r, valid, pos, s);  // uniform
 }
 
 // ------------------------------------------------------------- binning

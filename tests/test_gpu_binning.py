@@ -334,3 +334,21 @@ def test_capped_sort_overflow_leaves_empty_lists(gpu, monkeypatch):
     assert out[3] is not None and out[3].ok()
     shift = out[1].numel() - k
     assert shift > 0 and torch.equal(out[1][shift:], ids) and torch.equal(out[0] - shift, off)
+
+
+@pytest.mark.parametrize("keys,ulps", [
+    (2, 60), (47, 1), (48, 1), (49, 1), (50, 2), (300, 60), (700, 1), (1100, 60),
+])
+@pytest.mark.parametrize("width,height,tile", [(256, 256, 16), (2560, 1600, 8)])
+def test_segment_sort_crowding_bitexact(gpu, keys, ulps, width, height, tile):
+    """Groups of `keys` depths within `ulps` units of each other, about the limits of the
+    segment sort's three ways: one pass over sub-buckets (up to 48 keys in one), LDS passes
+    (a chunk of up to 1024 keys) and global memory (both level-1 forms)."""
+    n = 12_000
+    pts, radii, _, _ = _random_splats(n, width, height, seed=keys, rmax=12.0)
+    g = np.random.default_rng(keys)
+    group = (g.permutation(n) // keys).astype(np.uint32)
+    step = np.uint32((1 << 23) // (n // keys + 1))
+    depths = (np.float32(2.0).view(np.uint32) + group * step
+              + g.integers(0, ulps, n).astype(np.uint32)).view(np.float32)
+    assert _check(gpu, pts, radii, depths, np.ones(n, dtype=bool), width, height, tile) > 0
