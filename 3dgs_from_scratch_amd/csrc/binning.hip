@@ -1468,13 +1468,12 @@ __global__ __launch_bounds__(256) void tiles_from_rects_kernel(int64_t n,
 // Within a tile the entries therefore keep the depth order of the lists.
 struct L2Args {
     const int32_t *super_off;     // n_super: first list position of each supertile
-    const int32_t *super_ids;     // m: Gaussian ids per supertile, depth order
+    const uint2 *super_entries;   // m: entries per supertile, depth order (super_entry)
     const uint32_t *chunk_start;  // n_super + 1: first level-2 block of each supertile
     const uint4 *block_map;       // per level-2 workgroup w: (supertile, first and end list
                                   // position, logical block xcd_block(w, chunks)), laid out
                                   // so that each XCD takes a contiguous range of the
                                   // chunks; supertile kNoBlock past the last chunk
-    const uint2 *super_rects;     // m: packed tile rectangle of each list entry
     int64_t n, m, k;
     int n_super, super_x, tiles_x, tiles_y, width, height, tile_size;
     int64_t nblocks;              // level-2 blocks the grid covers (a bound on the chunks)
@@ -1544,34 +1543,10 @@ struct L2Block {
     uint32_t b;
     uint32_t trow;  // table[b * kSuperLocal + thread] for the first kSuperLocal threads
     int32_t g;
-    uint64_t mask;
-    int lx0, lx1, ly0, ly1;  // the mask as a rectangle of local tiles (empty: lx0 > lx1)
+    uint32_t cover;  // local rows and columns covered (super_entry; 0: none)
 };
 
-// Bit j (= ly * kSuper + lx) set for every tile of supertile s that Gaussian
-// g (list entry e, whose tile rectangle is super_rects[e]) covers; the covered
-// local rectangle goes to x.
-__device__ __forceinline__ uint64_t local_mask(const L2Args &a, int32_t g, uint2 packed, int s,
-                                               L2Block &x) {
-    x.lx0 = x.ly0 = 1;
-    x.lx1 = x.ly1 = 0;
-    if (g < 0 || (int64_t)g >= a.n) return 0;
-    const TileRect r = unpack_rect(packed);  // Gaussians in the lists have tiles
-    const int ox = (s % a.super_x) * kSuper, oy = (s / a.super_x) * kSuper;
-    const int x0 = max(r.tx0 - ox, 0), x1 = min(r.tx1 - ox, kSuper - 1);
-    const int y0 = max(r.ty0 - oy, 0), y1 = min(r.ty1 - oy, kSuper - 1);
-    if (x0 > x1 || y0 > y1) return 0;
-    x.lx0 = x0;
-    x.lx1 = x1;
-    x.ly0 = y0;
-    x.ly1 = y1;
-    const uint64_t row = ((1ull << (x1 - x0 + 1)) - 1ull) << x0;
-    uint64_t m = 0;
-    for (int y = y0; y <= y1; ++y) m |= row << (y * kSuper);
-    return m;
-}
-
-// Block -> supertile, this lane's Gaussian and mask.  Returns false (uniformly)
+// Block -> supertile, this lane's Gaussian and the tiles it covers.  Returns false (uniformly)
 // for the blocks past the last chunk (the grid is sized by an upper bound).
 // Workgroup w handles block w - skip (the first `skip` workgroups, a multiple of
 // kBinXcds, do other work).
@@ -1593,10 +1568,9 @@ __device__ __forceinline__ bool l2_block(const L2Args &a, L2Block &x, uint32_t s
     // compiler wait for all memory operations, stores included, before each of the
     // scatter's stores of x.g
     const int64_t ec = e < end ? e : end - 1;
-    const int32_t g = a.super_ids[ec];
-    const uint2 packed = a.super_rects[ec];
-    x.g = e < end ? g : -1;
-    x.mask = local_mask(a, x.g, packed, x.s, x);
+    const uint2 entry = a.super_entries[ec];
+    x.g = e < end ? (int32_t)entry.x : -1;
+    x.cover = x.g >= 0 && (int64_t)x.g < a.n ? entry.y : 0u;
     return true;
 }
 
@@ -1610,8 +1584,8 @@ __device__ __forceinline__ uint32_t wave_masks(const L2Block &x, uint64_t (&rows
     uint64_t mine_row = 0, mine_col = 0;
 #pragma unroll
     for (int q = 0; q < kSuper; ++q) {
-        rows[q] = __ballot(x.ly0 <= q && q <= x.ly1);
-        cols[q] = __ballot(x.lx0 <= q && q <= x.lx1);
+        rows[q] = __ballot((x.cover & (1u << q)) != 0u);
+        cols[q] = __ballot((x.cover & (1u << (kSuper + q))) != 0u);
         mine_row = lane / kSuper == q ? rows[q] : mine_row;
         mine_col = lane % kSuper == q ? cols[q] : mine_col;
     }
@@ -1863,6 +1837,19 @@ __global__ __launch_bounds__(kL2Threads) void l2_scatter_kernel(L2Args a,
         scatter_runs<k32, true>(rows, cols, my_base, k_lo, a.k, x.g, ids_out);
 }
 
+// Level-1 entry of Gaussian g with tile rectangle t in supertile (sx, sy), which it
+// meets: {g, the local rows it covers in bits 0..7 and the local columns in bits
+// 8..15}.  Eight bytes, so that an entry is one store into its list and one load
+// in each level-2 kernel.
+static_assert(kSuper == 8, "one byte of rows, one of columns");
+__device__ __forceinline__ uint2 super_entry(uint32_t g, const TileRect &t, int sx, int sy) {
+    const int x0 = max(t.tx0 - sx * kSuper, 0), x1 = min(t.tx1 - sx * kSuper, kSuper - 1);
+    const int y0 = max(t.ty0 - sy * kSuper, 0), y1 = min(t.ty1 - sy * kSuper, kSuper - 1);
+    const uint32_t cols = (0xffu << x0) & (0xffu >> (kSuper - 1 - x1));
+    const uint32_t rows = (0xffu << y0) & (0xffu >> (kSuper - 1 - y1));
+    return make_uint2(g, rows | (cols << kSuper));
+}
+
 // Level-1 entries: for the Gaussian at depth-order position r, one entry per
 // supertile of its rectangle (row-major), at offsets[r].. (thread per position).
 template <typename KeyT>
@@ -1870,7 +1857,7 @@ __global__ __launch_bounds__(256) void emit_super_kernel(
     int64_t n, int64_t m, const uint32_t *__restrict__ order,
     const uint64_t *__restrict__ offsets, const uint2 *__restrict__ rects, int super_x,
     KeyT *__restrict__ keys_out, uint32_t *__restrict__ vals_out,
-    uint2 *__restrict__ rects_out) {
+    uint2 *__restrict__ entries_out) {
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= n) return;
     const uint32_t g = order[r];
@@ -1884,7 +1871,7 @@ __global__ __launch_bounds__(256) void emit_super_kernel(
             if (o >= m) return;
             keys_out[o] = (KeyT)(y * super_x + x);
             vals_out[o] = g;
-            rects_out[o] = packed;
+            entries_out[o] = super_entry(g, t, x, y);
         }
 }
 
@@ -1898,7 +1885,7 @@ __global__ __launch_bounds__(256) void emit_super_kernel(
 // rank among the block's entries of s is the popcount of the lanes before it.
 // The segment sort adds each block's counts to a digit-major table as it emits
 // the depth order (seg_l1_counts), digit_scan_kernel turns them into positions,
-// and l1_scatter_kernel writes every entry's id and packed tile rectangle at
+// and l1_scatter_kernel writes every entry (super_entry) at
 // its position in the supertile-sorted list, which is stable: (supertile, depth
 // order).
 
@@ -1924,42 +1911,7 @@ __device__ __forceinline__ int64_t l1_live_blocks(const L1Args &a) {
     return (*a.n_live + kL1Threads - 1) / kL1Threads;
 }
 
-// This thread's Gaussian and the supertile range its tile rectangle meets
-// (false: none).
-__device__ __forceinline__ bool l1_gaussian(const L1Args &a, int64_t blk, uint32_t &g,
-                                            uint2 &packed, TileRect &sr) {
-    const int64_t r = blk * kL1Threads + threadIdx.x;
-    if (r >= a.n) return false;
-    g = a.order[r];
-    packed = a.rects_depth[r];
-    const TileRect t = unpack_rect(packed);
-    if (g >= (uint64_t)a.n || t.tx0 > t.tx1) return false;
-    sr.tx0 = t.tx0 / kSuper;
-    sr.tx1 = t.tx1 / kSuper;
-    sr.ty0 = t.ty0 / kSuper;
-    sr.ty1 = t.ty1 / kSuper;
-    return true;
-}
-
-// lanes[w][s] for the block (zeroed here); returns whether this lane has entries.
-__device__ __forceinline__ bool l1_lane_masks(const L1Args &a, int64_t blk,
-                                              uint64_t (*lanes)[kRadixMax], uint32_t &g,
-                                              uint2 &packed, TileRect &sr) {
-    for (int i = threadIdx.x; i < kL1Waves * kRadixMax; i += kL1Threads) lanes[0][i] = 0ull;
-    __syncthreads();
-    const int wave = threadIdx.x / kWave;
-    const uint64_t bit = 1ull << (threadIdx.x % kWave);
-    const bool has = l1_gaussian(a, blk, g, packed, sr);
-    if (has)
-        for (int y = sr.ty0; y <= sr.ty1; ++y)
-            for (int x = sr.tx0; x <= sr.tx1; ++x)
-                atomicOr(reinterpret_cast<unsigned long long *>(&lanes[wave][y * a.super_x + x]),
-                         (unsigned long long)bit);
-    __syncthreads();
-    return has;
-}
-
-// The level-2 block plan, from block 0 of l1_scatter_kernel (thread d holds
+// The level-2 block plan, from workgroup 0 of l1_scatter_kernel (thread d holds
 // supertile d's entry count `tot` and first list position `first`): chunks of
 // kL2Threads list positions per supertile, their exclusive scan chunk_start
 // (chunk_start[n_super] = all chunks) and the block map: entry w = (supertile,
@@ -2005,12 +1957,18 @@ __device__ __forceinline__ void l1_block_plan(int n_super, uint32_t tot, uint32_
 
 // `hist` holds, after digit_scan_kernel, the first position of (s, block)
 // among the entries of s and `totals` the entries of each s.  Writes
-// super_ids / super_rects, zeroes the per-tile entry counters of level 2 and,
-// from block 0, super_off[s] = entries with a smaller supertile and the
-// level-2 block plan (l1_block_plan).
+// super_entries, zeroes the per-tile entry counters of level 2 and,
+// from workgroup 0, super_off[s] = entries with a smaller supertile and the
+// level-2 block plan (l1_block_plan).  The grid is one workgroup more than the
+// blocks: the plan starts first and runs beside the scatter.  Every load of a
+// block is issued before its first barrier.  Bound by its stores, runs of about
+// five entries that fill a part of a line each: 21.0 us at 1M Gaussians and
+// 2560x1440 with an id and a packed rectangle per entry in two arrays, 15.2 with
+// one 8-byte entry (39.4 and 28.0 at 3M, 1920x1080; l2_scatter_kernel, which reads
+// them, 70.4 and 58.5).
 __global__ __launch_bounds__(kL1Threads) void l1_scatter_kernel(
     L1Args a, const uint32_t *__restrict__ hist, const uint32_t *__restrict__ totals,
-    int n_super, int32_t *__restrict__ super_ids, uint2 *__restrict__ super_rects,
+    int n_super, uint2 *__restrict__ super_entries,
     int32_t *__restrict__ super_off, uint32_t *__restrict__ chunk_start,
     uint4 *__restrict__ block_map, int64_t l2_nblocks, int n_tiles,
     uint32_t *__restrict__ tile_counts) {
@@ -2021,24 +1979,41 @@ __global__ __launch_bounds__(kL1Threads) void l1_scatter_kernel(
          t += (int64_t)gridDim.x * kL1Threads)
         tile_counts[t] = 0u;
     if (a.cap_totals && a.cap_totals[1] > a.m) return;  // past the entry capacity: no output
-    const int64_t blk = blockIdx.x;  // (round robin over the XCDs measured faster here)
-    if (blk != 0 && !l1_live_block(a, blk)) return;  // no entries (block 0 writes the plan)
-    uint32_t g = 0;
-    uint2 packed = make_uint2(0u, 0u);
-    TileRect sr{0, -1, 0, -1};
-    const bool has = l1_lane_masks(a, blk, lanes, g, packed, sr);
     const int d = threadIdx.x;
-    const uint32_t tot = d < n_super ? totals[d] : 0u;
     uint32_t all;
-    const uint32_t smaller = block_exclusive_scan<uint32_t, kL1Threads>(tot, scan_tmp, all);
-    if (blk == 0) {  // uniform per workgroup; wave_pos serves as staging
+    if (blockIdx.x == 0) {  // uniform per workgroup; wave_pos serves as staging
+        const uint32_t tot = d < n_super ? totals[d] : 0u;
+        const uint32_t smaller = block_exclusive_scan<uint32_t, kL1Threads>(tot, scan_tmp, all);
         if (d < n_super) super_off[d] = (int32_t)smaller;
         l1_block_plan(n_super, tot, smaller, scan_tmp, wave_pos[0], wave_pos[1], wave_pos[2],
                       chunk_start, block_map, l2_nblocks);
-        __syncthreads();
+        return;
     }
+    const int64_t blk = (int64_t)blockIdx.x - 1;  // (round robin over the XCDs measured faster here)
+    if (!l1_live_block(a, blk)) return;           // no entries
+    const int64_t r = blk * kL1Threads + d;
+    const int64_t rc = r < a.n ? r : a.n - 1;
+    const uint32_t g = a.order[rc];
+    const uint2 packed = a.rects_depth[rc];
+    const uint32_t tot = d < n_super ? totals[d] : 0u;
+    const uint32_t earlier = d < n_super ? hist[hist_index(d, (int)blk, a.nblocks)] : 0u;
+    for (int i = d; i < kL1Waves * kRadixMax; i += kL1Threads) lanes[0][i] = 0ull;
+    const uint32_t smaller = block_exclusive_scan<uint32_t, kL1Threads>(tot, scan_tmp, all);
+    // (the scan's barriers also order the zeroing)  The supertiles this Gaussian meets:
+    const TileRect t = unpack_rect(packed);
+    const bool has = r < a.n && g < (uint64_t)a.n && t.tx0 <= t.tx1;
+    const TileRect sr{t.tx0 / kSuper, t.tx1 / kSuper, t.ty0 / kSuper, t.ty1 / kSuper};
+    if (has) {
+        const uint64_t bit = 1ull << (d % kWave);
+        for (int y = sr.ty0; y <= sr.ty1; ++y)
+            for (int x = sr.tx0; x <= sr.tx1; ++x)
+                atomicOr(reinterpret_cast<unsigned long long *>(
+                             &lanes[d / kWave][y * a.super_x + x]),
+                         (unsigned long long)bit);
+    }
+    __syncthreads();
     if (d < kRadixMax) {
-        uint32_t pos = smaller + (d < n_super ? hist[hist_index(d, (int)blk, a.nblocks)] : 0u);
+        uint32_t pos = smaller + earlier;
 #pragma unroll
         for (int w = 0; w < kL1Waves; ++w) {
             wave_pos[w][d] = pos;
@@ -2053,10 +2028,8 @@ __global__ __launch_bounds__(kL1Threads) void l1_scatter_kernel(
             for (int x = sr.tx0; x <= sr.tx1; ++x) {
                 const int s = y * a.super_x + x;
                 const uint32_t p = wave_pos[wave][s] + (uint32_t)__popcll(lanes[wave][s] & below);
-                if ((int64_t)p < a.m) {  // always true for consistent counts; guards the store
-                    super_ids[p] = (int32_t)g;
-                    super_rects[p] = packed;
-                }
+                if ((int64_t)p < a.m)  // always true for consistent counts; guards the store
+                    super_entries[p] = super_entry(g, t, x, y);
             }
     }
 }
@@ -2166,8 +2139,8 @@ inline bool use_u16_keys(int tile_bits) { return tile_bits <= 16; }
 // Level 1: the (supertile, Gaussian) entries and their sort by supertile.
 struct SortWs {
     void *keys_a, *keys_b;  // supertile keys (u16 or u32)
-    uint32_t *vals_tmp;
-    uint2 *rects_tmp;       // packed tile rectangle of each entry (payload of the sort)
+    uint32_t *vals_a, *vals_b;
+    uint2 *entries_tmp;     // the entries (payload of the sort)
     void *pass_ws;  // histogram table + digit totals of each pass
     size_t bytes;
 };
@@ -2177,8 +2150,9 @@ inline SortWs carve_sort(Carve &c, int64_t m, int super_bits) {
     const int64_t kb = use_u16_keys(super_bits) ? 2 : 4;
     w.keys_a = c.take<char>(m * kb);
     w.keys_b = c.take<char>(m * kb);
-    w.vals_tmp = c.take<uint32_t>(m);
-    w.rects_tmp = c.take<uint2>(m);
+    w.vals_a = c.take<uint32_t>(m);
+    w.vals_b = c.take<uint32_t>(m);
+    w.entries_tmp = c.take<uint2>(m);
     w.pass_ws = c.take<char>((int64_t)radix_workspace_bytes<kTileItems>(m));
     w.bytes = 0;
     return w;
@@ -2214,8 +2188,7 @@ inline int64_t l2_blocks_bound(int64_t m, int n_super) {
 struct BinWs {
     SortWs lvl1;            // general level 1 (more than kRadixMax supertiles)
     int32_t *super_off;     // n_super (+1 spare)
-    int32_t *super_ids;     // m
-    uint2 *super_rects;     // m: packed tile rectangle of each super_ids entry
+    uint2 *super_entries;   // m: the entries by supertile (super_entry)
     uint32_t *chunk_start;  // n_super + 1: first level-2 block of each supertile
     uint4 *block_map;       // level-2 block -> (supertile, first and end list position, 0)
     uint32_t *table;        // level-2 blocks x 64 local tiles
@@ -2230,8 +2203,7 @@ inline BinWs carve_bins(void *base, int64_t n, int64_t m, const Grid &g) {
     (void)n;
     if (g.n_super > kRadixMax) w.lvl1 = carve_sort(c, m, g.super_bits);
     w.super_off = c.take<int32_t>((int64_t)g.n_super + 1);
-    w.super_ids = c.take<int32_t>(m);
-    w.super_rects = c.take<uint2>(m);
+    w.super_entries = c.take<uint2>(m);
     w.chunk_start = c.take<uint32_t>((int64_t)g.n_super + 1);
     w.block_map = c.take<uint4>(l2_blocks_bound(m, g.n_super));
     w.table = c.take<uint32_t>(l2_blocks_bound(m, g.n_super) * kSuperLocal);
@@ -2248,30 +2220,27 @@ inline int bits_for(int64_t max_value) {
 }
 
 // Level 1: the (supertile, Gaussian) entries in depth order, stably sorted by
-// supertile id; writes the per-supertile list starts and the sorted ids.
+// supertile id; writes the per-supertile list starts and the sorted entries.
 template <typename KeyT>
 int super_sort(const EmitArgs &a, const SortWs &w, int super_bits, int n_super,
-               int32_t *super_off, int32_t *super_ids, uint2 *super_rects, hipStream_t stream) {
+               int32_t *super_off, uint2 *super_entries, hipStream_t stream) {
     const SortPlan plan = plan_sort(super_bits);
     const int P = plan.passes;
     KeyT *ka = reinterpret_cast<KeyT *>(w.keys_a), *kb = reinterpret_cast<KeyT *>(w.keys_b);
-    uint32_t *out = reinterpret_cast<uint32_t *>(super_ids);
-    // pass p writes (kb, out, super_rects) when P-1-p is even, (ka, vals_tmp,
-    // rects_tmp) otherwise; the entries (pass -1) go to the other set than pass 0.
-    // Each entry carries its Gaussian's packed tile rectangle, so that level 2
-    // reads it in list order.
+    // pass p writes (kb, vals_b, super_entries) when P-1-p is even, (ka, vals_a,
+    // entries_tmp) otherwise; the entries (pass -1) go to the other set than pass 0.
     auto keys_for = [&](int p) { return ((P - 1 - p) % 2 == 0) ? kb : ka; };
-    auto vals_for = [&](int p) { return ((P - 1 - p) % 2 == 0) ? out : w.vals_tmp; };
-    auto rects_for = [&](int p) { return ((P - 1 - p) % 2 == 0) ? super_rects : w.rects_tmp; };
+    auto vals_for = [&](int p) { return ((P - 1 - p) % 2 == 0) ? w.vals_b : w.vals_a; };
+    auto entries_for = [&](int p) { return ((P - 1 - p) % 2 == 0) ? super_entries : w.entries_tmp; };
     hipLaunchKernelGGL(emit_super_kernel<KeyT>, dim3(ceil_div(a.n, 256)), dim3(256), 0, stream,
                        a.n, a.k, a.order, a.offsets, a.rects, a.tiles_x, keys_for(-1),
-                       vals_for(-1), rects_for(-1));
+                       vals_for(-1), entries_for(-1));
     int st = launch_status();
     if (st) return st;
     for (int p = 0; p < P; ++p) {
         PassExtras x;
-        x.pin = rects_for(p - 1);
-        x.pout = rects_for(p);
+        x.pin = entries_for(p - 1);
+        x.pout = entries_for(p);
         st = radix_pass<KeyT, kTileItems, true>(keys_for(p - 1), vals_for(p - 1), keys_for(p),
                                                 vals_for(p), a.k, p * plan.bits_per_pass,
                                                 pass_bits(plan, super_bits, p), true, w.pass_ws,
@@ -2566,9 +2535,9 @@ int bin_sort(const float *points_image, const float *radii, const float *depths,
     if (g.n_super <= kRadixMax) {  // counts and positions came from gs_bin_count
         L1Args la = l1_args(cw, n, m, g.super_x);
         la.cap_totals = capped ? cw.dev_totals : nullptr;
-        hipLaunchKernelGGL(l1_scatter_kernel, dim3(la.nblocks), dim3(kL1Threads), 0, stream, la,
+        hipLaunchKernelGGL(l1_scatter_kernel, dim3(la.nblocks + 1), dim3(kL1Threads), 0, stream, la,
                            (const uint32_t *)cw.l1_hist, (const uint32_t *)cw.l1_totals,
-                           g.n_super, w.super_ids, w.super_rects, w.super_off, w.chunk_start,
+                           g.n_super, w.super_entries, w.super_off, w.chunk_start,
                            w.block_map, nb2, g.n_tiles, w.tile_counts);
         st = launch_status();
     } else {  // emitted entries sorted by supertile over several radix passes
@@ -2581,9 +2550,9 @@ int bin_sort(const float *points_image, const float *radii, const float *depths,
         a.tiles_x = g.super_x;
         st = use_u16_keys(g.super_bits)
                  ? super_sort<uint16_t>(a, w.lvl1, g.super_bits, g.n_super, w.super_off,
-                                        w.super_ids, w.super_rects, stream)
+                                        w.super_entries, stream)
                  : super_sort<uint32_t>(a, w.lvl1, g.super_bits, g.n_super, w.super_off,
-                                        w.super_ids, w.super_rects, stream);
+                                        w.super_entries, stream);
         if (st) return st;
         // level-2 block plan (the one-pass level 1 writes it itself)
         hipLaunchKernelGGL(l2_plan_kernel, dim3(1), dim3(kPlanThreads), 0, stream, g.n_super, m,
@@ -2596,10 +2565,9 @@ int bin_sort(const float *points_image, const float *radii, const float *depths,
     // level 2: per-tile counts, tile offsets and block prefixes, scatter
     L2Args l2;
     l2.super_off = w.super_off;
-    l2.super_ids = w.super_ids;
+    l2.super_entries = w.super_entries;
     l2.chunk_start = w.chunk_start;
     l2.block_map = w.block_map;
-    l2.super_rects = w.super_rects;
     l2.n = n;
     l2.m = m;
     l2.k = k;
