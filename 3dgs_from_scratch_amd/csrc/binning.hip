@@ -306,6 +306,16 @@ __device__ __forceinline__ int64_t hist_index(int d, int b, int nblocks) {
     return (int64_t)d * nblocks + b;
 }
 
+// The one-pass level 1's counts, which atomics fill: the counts of 16 consecutive
+// supertiles of a block share a 64-byte line, so that the lanes of one atomic
+// instruction meet four lines instead of 64: segment_sort_kernel, which issues them,
+// 23.5 -> 17.6 us at 1M Gaussians and 2560x1440 (54.8 -> 48.4 at 3M, 1920x1080),
+// against 4.3 -> 5.5 (9.1 -> 12.1) for the scan that reads the groups.
+constexpr int kL1Group = 16;
+__device__ __forceinline__ int64_t l1_count_index(int s, int b, int nblocks) {
+    return ((int64_t)(s / kL1Group) * nblocks + b) * kL1Group + s % kL1Group;
+}
+
 // Per-block sums of count_tiles (tiles, supertile entries, Gaussians with
 // tiles; three per block) reduced by one workgroup of kScanThreads to
 // sums_out[0] = K, sums_out[1] = M and *live_out (K and M also to sums_dev, a
@@ -373,8 +383,10 @@ __device__ __forceinline__ void reduce_block_sums(const unsigned long long *__re
 // block_minmax when it is set).
 constexpr int kDigitScanItems = 8;  // column entries per thread held in registers
 
+// With l1_counts, the counts come from there (l1_count_index).
 __global__ __launch_bounds__(kScanThreads) void digit_scan_kernel(
-    uint32_t *__restrict__ table, int nblocks, uint32_t *__restrict__ totals,
+    uint32_t *__restrict__ table, const uint32_t *__restrict__ l1_counts, int nblocks,
+    uint32_t *__restrict__ totals,
     const unsigned long long *__restrict__ block_sums, const uint32_t *__restrict__ block_minmax,
     int nsum_blocks, int64_t *__restrict__ sums_out, int64_t *__restrict__ live_out,
     int64_t *__restrict__ sums_dev) {
@@ -395,7 +407,9 @@ __global__ __launch_bounds__(kScanThreads) void digit_scan_kernel(
         uint32_t mine = 0;
 #pragma unroll
         for (int it = 0; it < kDigitScanItems; ++it) {
-            c[it] = first + it < nblocks ? col[first + it] : 0u;
+            const int b = first + it;
+            c[it] = b < nblocks ? (l1_counts ? l1_counts[l1_count_index(d, b, nblocks)] : col[b])
+                                : 0u;
             mine += c[it];
         }
         uint32_t chunk;
@@ -665,7 +679,7 @@ int radix_pass(const KeyT *kin, const uint32_t *vin, KeyT *kout, uint32_t *vout,
     }
     const int sums_block = x.block_sums ? 1 : 0;
     hipLaunchKernelGGL(digit_scan_kernel, dim3((1 << nbits) + sums_block), dim3(kScanThreads), 0,
-                       stream, hist, nblocks, totals, x.block_sums, x.block_minmax, nblocks,
+                       stream, hist, nullptr, nblocks, totals, x.block_sums, x.block_minmax, nblocks,
                        x.sums_out, x.live_out, x.sums_dev);
     st = launch_status();
     if (st) return st;
@@ -876,8 +890,8 @@ struct SegArgs {
     uint64_t *counts_out;           // general level 1: supertile count per depth position
     uint2 *rects_out;               // one-pass level 1: rectangle per depth position
     // one-pass level 1: its (supertile, block) entry counts, added here per emitted
-    // position (hist_index(s, p / kL1Threads, l1_nblocks), zeroed by count_tiles_kernel)
-    uint32_t *l1_hist;
+    // position (l1_count_index, block p / kL1Threads; zeroed by count_tiles_kernel)
+    uint32_t *l1_counts;
     int super_x, l1_nblocks;
 };
 
@@ -929,8 +943,8 @@ __device__ void seg_l1_counts(const SegArgs &a, uint32_t start, uint32_t size,
     for (uint32_t i = threadIdx.x; i < nb * kRadixMax; i += kSegThreads) {
         const uint32_t c = cnt[i];
         if (c)
-            atomicAdd(&a.l1_hist[hist_index((int)(i % kRadixMax), (int)(b0 + i / kRadixMax),
-                                            a.l1_nblocks)],
+            atomicAdd(&a.l1_counts[l1_count_index((int)(i % kRadixMax), (int)(b0 + i / kRadixMax),
+                                                  a.l1_nblocks)],
                       c);
     }
 }
@@ -1022,9 +1036,10 @@ __device__ void seg_sort_global(const SegArgs &a, uint32_t start, uint32_t end, 
         const uint32_t p = start + t;
         const uint2 r = rect_or_empty(a.rects, a.vals[p], a.n);
         seg_store(a, p, r);
-        if (a.l1_hist)  // a rare path: one table atomic per (position, supertile)
+        if (a.l1_counts)  // a rare path: one table atomic per (position, supertile)
             for_each_supertile(r, a.super_x, [&](int st) {
-                atomicAdd(&a.l1_hist[hist_index(st, (int)(p / kL1Threads), a.l1_nblocks)], 1u);
+                atomicAdd(
+                    &a.l1_counts[l1_count_index(st, (int)(p / kL1Threads), a.l1_nblocks)], 1u);
             });
     }
 }
@@ -1033,8 +1048,9 @@ __device__ void seg_sort_global(const SegArgs &a, uint32_t start, uint32_t end, 
 // small scenes and by the rectangles' gather (8 bytes of a memory line a key) on
 // large ones, not by its 40 bytes a key.  Comparing a key with its whole depth
 // bucket instead of a sub-bucket was slower where buckets hold over 100 keys (bin at
-// 1M Gaussians 162 us); LDS passes on every chunk took 27.8 (1M Gaussians,
-// 2560x1440) and 62.7 us (3M, 1920x1080), this takes 23.7 and 56.1.
+// 1M Gaussians 162 us instead of 152).  LDS passes on every chunk took 27.8 us (1M
+// Gaussians, 2560x1440) and 62.7 us (3M, 1920x1080), this took 23.7 and 56.1, and
+// with l1_count_index's order it takes 17.6 and 48.4.
 __global__ __launch_bounds__(kSegThreads) void segment_sort_kernel(SegArgs a) {
     __shared__ SegLds s;
     const int64_t live64 = *a.n_live;
@@ -1159,7 +1175,7 @@ __global__ __launch_bounds__(kSegThreads) void segment_sort_kernel(SegArgs a) {
                 a.vals[start + pos[it]] = wv[it];
                 seg_store(a, start + pos[it], r[it]);
             }
-            if (a.l1_hist) seg_l1_counts(a, start, size, r, valid, pos, s);  // uniform
+            if (a.l1_counts) seg_l1_counts(a, start, size, r, valid, pos, s);  // uniform
             return;
         }
 #pragma unroll
@@ -1220,7 +1236,7 @@ __global__ __launch_bounds__(kSegThreads) void segment_sort_kernel(SegArgs a) {
         a.vals[start + pos[it]] = v[it];
         seg_store(a, start + pos[it], r[it]);
     }
-    if (a.l1_hist) seg_l1_counts(a, start, size, r, valid, pos, s);  // uniform
+    if (a.l1_counts) seg_l1_counts(a, start, size, r, valid, pos, s);  // uniform
 }
 
 // ------------------------------------------------------------- binning
@@ -2082,7 +2098,8 @@ struct CountWs {
     int64_t *n_live;                 // Gaussians with tiles (keys of depth passes 1..)
     int64_t *dev_totals;             // K and M in device memory (read by gs_bin_sort_capped)
     uint64_t *m_scan;                // the general level 1's entry total (equals M)
-    uint32_t *l1_hist;               // one-pass level 1: kRadixMax x l1_blocks(n) table
+    uint32_t *l1_counts;             // one-pass level 1: its counts (l1_count_index) and
+    uint32_t *l1_hist;               //   positions, kRadixMax x l1_blocks(n) each
     uint32_t *l1_totals;             // one-pass level 1: entries per supertile
     void *sort_ws, *scan_ws;
     size_t bytes;
@@ -2106,6 +2123,7 @@ inline CountWs carve_count(void *base, int64_t n) {
     w.dev_totals = c.take<int64_t>(2);
     w.n_live = c.take<int64_t>(1);
     w.m_scan = c.take<uint64_t>(1);
+    w.l1_counts = c.take<uint32_t>(kRadixMax * l1_blocks(n));
     w.l1_hist = c.take<uint32_t>(kRadixMax * l1_blocks(n));
     w.l1_totals = c.take<uint32_t>(kRadixMax);
     w.sort_ws = c.take<char>((int64_t)radix_workspace_bytes<kDepthItems>(n));
@@ -2358,8 +2376,10 @@ int bin_count_begin(const CountCall &c, hipStream_t stream) {
                        stream, c.n, c.points_image, c.radii, c.depths, c.mask, c.width, c.height,
                        c.tile_size, w.rects, w.dkeys_a, w.block_sums, w.block_minmax,
                        c.hint_kmin, hinted ? c.hint_shift : 0, hinted ? hist : nullptr, w.xform,
-                       one_pass_l1 ? w.l1_hist : nullptr,
-                       one_pass_l1 ? (int64_t)grid.n_super * l1_blocks(c.n) : (int64_t)0);
+                       one_pass_l1 ? w.l1_counts : nullptr,
+                       one_pass_l1 ? (int64_t)ceil_div(grid.n_super, kL1Group) * kL1Group *
+                                         l1_blocks(c.n)
+                                   : (int64_t)0);
     st = launch_status();
     if (st) return st;
     if (!hinted) {
@@ -2397,7 +2417,7 @@ int bin_count_finish(const CountCall &c, hipStream_t stream) {
     sa.rects_out = one_pass_l1 ? w.rects_depth : nullptr;
     // the one-pass level 1's (supertile, block) counts, added as the positions are
     // emitted into the table count_tiles_kernel zeroed
-    sa.l1_hist = one_pass_l1 ? w.l1_hist : nullptr;
+    sa.l1_counts = one_pass_l1 ? w.l1_counts : nullptr;
     sa.super_x = grid.super_x;
     sa.l1_nblocks = (int)l1_blocks(c.n);
     hipLaunchKernelGGL(segment_sort_kernel, dim3(ceil_div(c.n, kSegChunk)), dim3(kSegThreads), 0,
@@ -2407,8 +2427,8 @@ int bin_count_finish(const CountCall &c, hipStream_t stream) {
     if (one_pass_l1) {
         const L1Args la = l1_args(w, c.n, 0, grid.super_x);
         hipLaunchKernelGGL(digit_scan_kernel, dim3(grid.n_super), dim3(kScanThreads), 0, stream,
-                           w.l1_hist, la.nblocks, w.l1_totals, nullptr, nullptr, 0, nullptr,
-                           nullptr, nullptr);
+                           w.l1_hist, w.l1_counts, la.nblocks, w.l1_totals, nullptr, nullptr, 0,
+                           nullptr, nullptr, nullptr);
         return launch_status();
     }
     // supertile entry offsets in depth order (the total equals count_tiles' M; it
