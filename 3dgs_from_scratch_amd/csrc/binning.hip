@@ -381,9 +381,9 @@ __device__ __forceinline__ void reduce_block_sums(const unsigned long long *__re
 // the column total to totals[d].  The downsweep adds the keys of smaller digits.
 // With block_sums, one more block (the last) runs reduce_block_sums (with
 // block_minmax when it is set).
+// With l1_counts, the counts come from there (l1_count_index).
 constexpr int kDigitScanItems = 8;  // column entries per thread held in registers
 
-// With l1_counts, the counts come from there (l1_count_index).
 __global__ __launch_bounds__(kScanThreads) void digit_scan_kernel(
     uint32_t *__restrict__ table, const uint32_t *__restrict__ l1_counts, int nblocks,
     uint32_t *__restrict__ totals,
@@ -1899,8 +1899,8 @@ __global__ __launch_bounds__(256) void emit_super_kernel(
 // lanes[w][s] has bit L set when lane L of wave w meets supertile s; the
 // block's count of s is the sum of popcounts over its waves, and an entry's
 // rank among the block's entries of s is the popcount of the lanes before it.
-// The segment sort adds each block's counts to a digit-major table as it emits
-// the depth order (seg_l1_counts), digit_scan_kernel turns them into positions,
+// The segment sort adds each block's counts to a table (l1_count_index) as it
+// emits the depth order (seg_l1_counts), digit_scan_kernel turns them into positions,
 // and l1_scatter_kernel writes every entry (super_entry) at
 // its position in the supertile-sorted list, which is stable: (supertile, depth
 // order).
@@ -2222,6 +2222,7 @@ inline BinWs carve_bins(void *base, int64_t n, int64_t m, const Grid &g) {
     if (g.n_super > kRadixMax) w.lvl1 = carve_sort(c, m, g.super_bits);
     w.super_off = c.take<int32_t>((int64_t)g.n_super + 1);
     w.super_entries = c.take<uint2>(m);
+    c.take<uint32_t>(m);  // unused: the size stays at 12 bytes an entry and more, as queried before
     w.chunk_start = c.take<uint32_t>((int64_t)g.n_super + 1);
     w.block_map = c.take<uint4>(l2_blocks_bound(m, g.n_super));
     w.table = c.take<uint32_t>(l2_blocks_bound(m, g.n_super) * kSuperLocal);
