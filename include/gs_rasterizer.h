@@ -231,9 +231,9 @@ int gs_bin_sort_capped(const float *points_image, const float *radii, const floa
 
 /*
  * Waves per 16x16 tile of the blend kernels (every gs_rasterize* entry with
- * tile_size 16): 0, the default, picks by the tile count (4 waves for grids of
- * at most 1024 tiles; above that 1, except the forward entries, which take 2
- * up to 6144 tiles); 1, 2 or 4 force that count.  With
+ * tile_size 16): 0, the default, picks by the tile count (forward: 4 waves
+ * up to 6144 tiles, 2 up to 16384, 1 above; backward: 4 up to 1024 tiles, 1
+ * above); 1, 2 or 4 force that count.  With
  * W waves, wave w composites strips w * 4/W .. of the tile's four 16x4 strips
  * and the waves share each staged batch.  Images are bit-equal for every
  * setting; gradients and the per-tile loss sums differ only in float summation
