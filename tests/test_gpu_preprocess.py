@@ -7,6 +7,8 @@ bound is 1e-3).
 
 from __future__ import annotations
 
+import math
+
 import pytest
 import torch
 
@@ -95,6 +97,50 @@ def test_project_points_backward(gpu, name):
     for nm, a, b in zip(["means", "scales", "quats"], got, ref):
         assert helpers.rel_l2(a, b) <= 1e-4, nm
         assert float(a[~p["keep"].to(gpu)].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("ratio", [1.0, 30.0, 1000.0, 6000.0])
+def test_projection_backward_of_thin_splats(gpu, ratio, fused):
+    """Splats whose image covariance has about the given eigenvalue ratio, at all angles: the
+    conic's gradient is a loss's at 64 pixels drawn about the splat, whose terms cancel by
+    the ratio's square on the way to the scales.  Against the same in 64 bits: covariance,
+    conic gradient and covariance gradient are rounded to float and the ratio amplifies each
+    of these roundings once, so 3 ratio 2^-24 of the gradients (0.4 to 1.2 in an emulation;
+    with the terms summed in float 9 at a ratio of 1000 and 23 at 6000)."""
+    n, f, z, W, H = 2000, 800.0, 4.0, 979, 547
+    g = torch.Generator().manual_seed(int(ratio))
+    means = torch.cat([torch.rand(n, 2, generator=g) - 0.5, torch.full((n, 1), z)], dim=1)
+    minor = 0.05 / (f / z)  # with the low-pass filter's 0.3: an eigenvalue of about 0.3
+    major = max((0.3 * ratio) ** 0.5 / (f / z), minor)
+    scales = torch.tensor([[major, minor, minor]]) * (1 + 0.1 * torch.rand(n, 3, generator=g))
+    half = torch.rand(n, generator=g) * math.pi / 2
+    quats = torch.stack([0 * half, 0 * half, torch.sin(half), torch.cos(half)], dim=1)
+    opac, w2c, K = torch.full((n,), 0.5), torch.eye(4), helpers.intrinsic(f, W, H)
+    leaves = [t.double().requires_grad_(True) for t in (means, scales, quats)]
+    p = preprocess.project(*leaves, opac.double(), w2c, K, W, H, NEAR, FAR, MIN_O, MIN_R, 200.0)
+    assert bool(p["keep"].all())
+    cov = torch.stack([p["a"], p["b"], p["b"], p["c"]], dim=1).detach().reshape(n, 2, 2)
+    d = torch.linalg.cholesky(cov) @ torch.randn(n, 2, 64, generator=g, dtype=torch.float64)
+    h = torch.randn(n, 1, 64, generator=g, dtype=torch.float64)
+    up = (h * torch.stack([-0.5 * d[:, 0] ** 2, -d[:, 0] * d[:, 1], -0.5 * d[:, 1] ** 2], 1)).sum(2)
+    up = up.float()
+    conic = torch.stack([p["A"], p["B"], p["C"]], dim=1)
+    (conic * up.double()).sum().backward()
+    ref = torch.cat([leaves[1].grad * scales, leaves[2].grad], dim=1)
+
+    dev = [t.to(gpu) for t in (means, scales, quats, opac, w2c, K)]
+    fwd = cr.project_points(*dev, NEAR, FAR, MIN_O, MIN_R, 200.0, W, H)
+    zero = torch.zeros(n, 3, device=gpu)
+    if fused:
+        got = cr.render_preprocess_backward(zero[:, :2], up.to(gpu), zero, *dev[:3], zero,
+                                            torch.zeros(n, 15, 3, device=gpu), fwd[2], fwd[5],
+                                            dev[4], dev[5], W, H)
+    else:
+        got = cr.project_points_backward(zero[:, :2], up.to(gpu), *dev, W, H, fwd[2], fwd[5])
+    got = torch.cat([got[1].cpu() * scales, got[2].cpu()], dim=1)
+    eig = torch.linalg.eigvalsh(cov)
+    assert helpers.rel_l2(got, ref) <= 3 * 2.0**-24 * float((eig[:, 1] / eig[:, 0]).median())
 
 
 @pytest.mark.parametrize("sh_sigmoid", [False, True])
