@@ -586,7 +586,8 @@ __device__ __forceinline__ void blend_entry(const BatchLds<W> &s, int slot,
         if (inc[q] == 0) continue;
         work += kCostStrip;
         const float alpha = alpha_of(E[q], aux.z);
-        const float w = (__builtin_amdgcn_inverse_ballot_w64(inc[q]) ? alpha : 0.0f) * L.T[q];
+        const float aT = alpha * L.T[q];
+        const float w = __builtin_amdgcn_inverse_ballot_w64(inc[q]) ? aT : 0.0f;
         L.cr[q] = fmaf(w, aux.w, L.cr[q]);
         L.cg[q] = fmaf(w, gb.x, L.cg[q]);
         L.cb[q] = fmaf(w, gb.y, L.cb[q]);
@@ -639,10 +640,12 @@ constexpr int kGroup = 4;
 // The next entries of a wave's list that reach its strips (bits of `m`, past its end
 // the slot that composites nothing), kGroup at a time.  Their records are loaded and
 // their alphas formed together, without branches, over all the wave's strips: only T
-// runs from entry to entry (a product, a difference and a select, which keeps a
-// finished pixel's T at 0).  A walk's length is its instructions' latencies where few
-// waves share a SIMD: entry by entry, 20k Gaussians at 251x183 (192 tiles) spent about
-// 380 cycles on each, 118 us in all, in groups 45 us.
+// runs from entry to entry (a product, a select by the pixel's active bit and a
+// difference).  The select is on the weight: a finished pixel's T is what the entry
+// that finished it left, below the threshold but not 0, and alpha may be infinite (a
+// conic that is not positive definite).  A walk's length is its instructions'
+// latencies where few waves share a SIMD: entry by entry, 20k Gaussians at 251x183
+// (192 tiles) spent about 380 cycles on each, 118 us in all, in groups 45 us.
 template <int W>
 __device__ __forceinline__ void blend_group(const BatchLds<W> &s, int base, uint64_t &m,
                                             const LanePixels<kStrips / W> &pix, float T_thr,
@@ -677,13 +680,13 @@ __device__ __forceinline__ void blend_group(const BatchLds<W> &s, int base, uint
     for (int i = 0; i < kGroup; ++i) {
 #pragma unroll
         for (int q = 0; q < S; ++q) {
-            const float w = alpha[i][q] * L.T[q];
+            const float aT = alpha[i][q] * L.T[q];
+            const float w = __builtin_amdgcn_inverse_ballot_w64(act[q]) ? aT : 0.0f;
             L.cr[q] = fmaf(w, aux[i].w, L.cr[q]);
             L.cg[q] = fmaf(w, gb[i].x, L.cg[q]);
             L.cb[q] = fmaf(w, gb[i].y, L.cb[q]);
-            const float T = L.T[q] - w;
-            act[q] = __ballot(!(T < T_thr));
-            L.T[q] = __builtin_amdgcn_inverse_ballot_w64(act[q]) ? T : 0.0f;
+            L.T[q] = L.T[q] - w;
+            act[q] = __ballot(!(L.T[q] < T_thr));
         }
     }
 }
@@ -817,8 +820,7 @@ __device__ __forceinline__ void blend_accumulate(
     const float T_thr = effective_T_thr(T_thr_in);
 #pragma unroll
     for (int q = 0; q < S; ++q) {
-        // outside the image: 0 where blend_group multiplies it by alpha
-        L.T[q] = pix.inside[q] ? 1.0f : 0.0f;
+        L.T[q] = pix.inside[q] ? 1.0f : kInactiveT;
         L.cr[q] = L.cg[q] = L.cb[q] = 0.0f;
     }
     if (n_ck) *n_ck = 0;

@@ -300,3 +300,67 @@ def test_backward_pending_entries(gpu, waves, count, opaque, t_thr):
     rows = cr.rasterize_l1_backward_rows(*l1)
     for nm, a, b in zip(INPUTS, want, (rows[:, :2], rows[:, 2:5], rows[:, 5], rows[:, 6:])):
         assert helpers.rel_l2(b, a) <= 1e-5, nm
+
+
+def _one_tile_images(gpu, pts, conic, opac, col, t_thr):
+    """One 16x16 tile with every entry in index order, composited by 1, 2 and 4 waves."""
+    n = pts.shape[0]
+    d = [t.to(gpu) for t in (pts, conic, opac, col)]
+    off = torch.zeros(1, dtype=torch.int32, device=gpu)
+    ids = torch.arange(n, dtype=torch.int32, device=gpu)
+    out = []
+    for w in (1, 2, 4):
+        cr.set_blend_waves(w)
+        out.append(cr.rasterize(off, ids, *d, 16, 16, 16, 1e-4, t_thr, 9.21).cpu())
+    cr.set_blend_waves(0)
+    return out
+
+
+@pytest.mark.parametrize("bad", ["colour", "opacity"])
+def test_batches_after_a_special_one(gpu, bad):
+    """A batch with a non-finite colour or opacity is composited with selects and leaves
+    finished pixels with 0 < T < the threshold; the ordinary batches that follow (lists of
+    three batches of the widest form, whose first two leave the right columns open) add
+    nothing to them.  Equal bits for every wave count, and the oracle's image beyond the
+    special splat's reach (1e-5: about 20 products of rounded factors)."""
+    n, g = 768, torch.Generator().manual_seed(5)
+    pts = torch.rand(n, 2, generator=g) * 16
+    pts[:512, 0] *= 6 / 16
+    conic = torch.tensor([[0.2, 0.0, 0.2]]).repeat(n, 1)  # a reach of 6.8 pixels
+    opac = torch.rand(n, generator=g) * 0.2 + 0.1
+    col = torch.rand(n, 3, generator=g)
+    pts[3], conic[3] = torch.tensor([2.0, 2.0]), torch.tensor([4.0, 0.0, 4.0])  # 1.5 pixels
+    plain = [pts, conic, opac.clone(), col.clone()]
+    if bad == "colour":
+        col[3, 1] = float("nan")
+    else:
+        opac[3] = float("nan")
+    images = _one_tile_images(gpu, pts, conic, opac, col, 0.5)
+    for image in images[1:]:
+        assert helpers.same(image, images[0])
+    plain[2][3] = 0.0
+    ref = blend.rasterize(torch.zeros(1, dtype=torch.int32), torch.arange(n, dtype=torch.int32),
+                          *plain, 16, 16, 16, 1e-4, 0.5, 9.21)
+    far = torch.ones(16, 16, dtype=torch.bool)
+    far[:5, :5] = False
+    assert helpers.max_abs(images[0][far], ref[far]) <= 1e-5
+
+
+def test_finished_pixels_and_an_unbounded_alpha(gpu):
+    """A conic that is not positive definite gives alpha = exp2(900): infinite where it is
+    composited, and nothing to the pixels that opaque splats finished before."""
+    n = 40
+    pts = torch.tensor([[2.0, 8.0]]).repeat(n, 1)
+    conic = torch.tensor([[0.05, 0.0, 0.001]]).repeat(n, 1)  # columns 0..15, E = 8.5 at the last
+    opac, col = torch.full((n,), 0.99), torch.rand(n, 3, generator=torch.Generator().manual_seed(6))
+    conic[6:, 0] = 1.0  # six reach the whole tile and finish its columns 0..4
+    pts[20], conic[20] = torch.tensor([60.0, 8.0]), torch.tensor([-1.0, 0.0, 1.0])
+    images = _one_tile_images(gpu, pts, conic, opac, col, 1e-4)
+    for image in images[1:]:
+        assert helpers.same(image, images[0])
+    keep = torch.arange(n) != 20
+    ref = blend.rasterize(torch.zeros(1, dtype=torch.int32),
+                          torch.arange(n - 1, dtype=torch.int32), pts[keep], conic[keep],
+                          opac[keep], col[keep], 16, 16, 16, 1e-4, 1e-4, 9.21)
+    assert helpers.max_abs(images[0][:, :5], ref[:, :5]) <= 1e-5
+    assert not torch.isfinite(images[0][:, 15]).any()  # composited there
