@@ -364,3 +364,25 @@ def test_finished_pixels_and_an_unbounded_alpha(gpu):
                           opac[keep], col[keep], 16, 16, 16, 1e-4, 1e-4, 9.21)
     assert helpers.max_abs(images[0][:, :5], ref[:, :5]) <= 1e-5
     assert not torch.isfinite(images[0][:, 15]).any()  # composited there
+
+
+@pytest.mark.parametrize("t_thr", [1e-30, 1e-10, 0.0])
+def test_backward_small_thresholds(gpu, waves, t_thr):
+    """Pixels composited down to T of 1e-29 with gradients of 1e18: what the sums leave of
+    1e18 by rounding (1e11) over T would be infinite, and infinity times a weight of 0 NaN.
+    Relative 1e-4: the sums' roundings, sqrt(256) of 6e-8 on terms of either sign."""
+    n, g = 70, torch.Generator().manual_seed(7)
+    pts = torch.rand(n, 2, generator=g) * 4 + 6
+    conic = torch.tensor([[0.05, 0.0, 0.05]]).repeat(n, 1)
+    opac, col = torch.full((n,), 0.9), torch.rand(n, 3, generator=g)
+    off, ids = torch.zeros(1, dtype=torch.int32), torch.arange(n, dtype=torch.int32)
+    args = (16, 16, 16, 1e-4, t_thr, 9.21)
+    ins = [t.clone().requires_grad_(True) for t in (pts, conic, opac, col)]
+    up = torch.randn(16, 16, 3, generator=g)
+    (blend.rasterize(off, ids, *ins, *args) * up).sum().backward()
+    d = [t.to(gpu) for t in (pts, conic, opac, col)]
+    off, ids = off.to(gpu), ids.to(gpu)
+    image = cr.rasterize(off, ids, *d, *args)
+    got = cr.rasterize_backward(1e18 * up.to(gpu), off, ids, *d, *args, rendered_image=image)
+    for nm, a, t in zip(INPUTS, got, ins):
+        assert helpers.rel_l2(a / 1e18, t.grad) <= 1e-4, nm
