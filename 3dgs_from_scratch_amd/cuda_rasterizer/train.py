@@ -111,9 +111,12 @@ class Densifier:
         as the fused step's, are read in place)."""
         n = self.grads.shape[0]
         g = grad_points_image.detach()
-        if g.dim() != 2 or g.stride(1) != 1 or not 2 <= g.stride(0) < 2**31:
+        rows = g.dim() == 2 and g.shape[1] >= 2
+        if rows and g.stride(1) == 1 and 2 <= g.stride(0) < 2**31:
+            stride = g.stride(0)
+        else:  # (a single row may report any stride, also after contiguous())
             g = g.contiguous()
-        stride = g.stride(0) if g.dim() == 2 else 2
+            stride = g.shape[1] if rows else 2
         r = radii.detach().contiguous()
         with _lib.on_device(g.device):
             _lib.check(_lib.load().gs_accumulate_grad2d_strided(

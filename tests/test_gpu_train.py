@@ -72,6 +72,26 @@ def test_accumulate_grad2d_matches_oracle(gpu):
     assert torch.equal(d.count.cpu(), count)
 
 
+@pytest.mark.parametrize("n", [1, 5])
+@pytest.mark.parametrize("form", ["rows", "transposed", "one_column", "expanded", "nine"])
+def test_accumulate_grad2d_layouts(gpu, n, form):
+    """Gradients of any layout: the first two columns of wider rows, transposed (a single
+    row then reports a row stride of 1, also once contiguous), 2N values in one column."""
+    g = torch.Generator().manual_seed(n)
+    wide = torch.randn(n, 9, generator=g).to(gpu)
+    gp = {"rows": wide[:, :2], "transposed": torch.empty(2, n, device=gpu).copy_(wide[:, :2].t()).t(),
+          "one_column": wide[:, :2].reshape(2 * n, 1), "expanded": wide[:1, :2].expand(n, 2),
+          "nine": wide}[form]
+    want = gp.reshape(n, -1)[:, :2].cpu()
+    radii = torch.ones(n, 2, device=gpu)
+    d = Densifier(n, gpu)
+    d.update(gp, radii, 640, 480)
+    grads, count = otrain.accumulate_grad2d(torch.zeros(n), torch.zeros(n), want, radii.cpu(), 640,
+                                            480)
+    assert helpers.rel_l2(d.grads, grads) <= 1e-6
+    assert torch.equal(d.count.cpu(), count)
+
+
 def _opt_with_state(params, gen, dev):
     opt = FusedAdam(params)
     for k in params:
