@@ -2222,7 +2222,6 @@ inline BinWs carve_bins(void *base, int64_t n, int64_t m, const Grid &g) {
     if (g.n_super > kRadixMax) w.lvl1 = carve_sort(c, m, g.super_bits);
     w.super_off = c.take<int32_t>((int64_t)g.n_super + 1);
     w.super_entries = c.take<uint2>(m);
-    c.take<uint32_t>(m);  // unused: the size stays at 12 bytes an entry and more, as queried before
     w.chunk_start = c.take<uint32_t>((int64_t)g.n_super + 1);
     w.block_map = c.take<uint4>(l2_blocks_bound(m, g.n_super));
     w.table = c.take<uint32_t>(l2_blocks_bound(m, g.n_super) * kSuperLocal);
