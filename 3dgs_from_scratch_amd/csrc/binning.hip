@@ -262,14 +262,14 @@ __device__ __forceinline__ uint32_t rect_supertiles(uint2 packed) {
 // Depth key of a Gaussian without tiles: the first depth pass drops these keys.
 constexpr uint32_t kNoTilesKey = 0xFFFFFFFFu;
 
-// kPayload: each value carries an 8-byte payload (a packed tile rectangle).
+// kPayload: 8-byte values (level-1 entries) in place of the 4-byte ones.
 template <int ITEMS, bool kPayload = false>
 struct SortLds {
     uint32_t wave_count[kSortWaves][kRadixMax];
     uint32_t global_start[kRadixMax];
     uint32_t local_start[kRadixMax];
     uint32_t skeys[kSortThreads * ITEMS];
-    uint32_t svals[kSortThreads * ITEMS];
+    uint32_t svals[kPayload ? 1 : kSortThreads * ITEMS];
     uint2 spay[kPayload ? kSortThreads * ITEMS : 1];
     uint32_t scan_tmp[kSortThreads / kWave + 1];
 };
@@ -425,8 +425,8 @@ __global__ __launch_bounds__(kScanThreads) void digit_scan_kernel(
 }
 
 // Stable rank of the block's keys (registers) by digit, staged through LDS in
-// digit order and written to keys_out/vals_out (and, with kPayload, the
-// payloads to pay_out).  `table` holds the position of each (digit, block)
+// digit order and written to keys_out/vals_out (with kPayload, keys_out and
+// pay_out alone).  `table` holds the position of each (digit, block)
 // among the keys of its digit, `totals` the keys per digit.  When counts_out
 // is set, counts_out[dst] = rect_supertiles(rects[value]) is written as well,
 // and when rects_out is set, rects_out[dst] = rects[value].
@@ -492,8 +492,10 @@ __device__ __forceinline__ void block_scatter(const uint32_t (&k)[ITEMS],
             const uint32_t d = digit_of(bf(k[it]), shift, dmask);
             const uint32_t p = s.local_start[d] + s.wave_count[wave][d] + rank[it];
             s.skeys[p] = k[it];
-            s.svals[p] = v[it];
-            if (kPayload) s.spay[p] = pay[it];
+            if constexpr (kPayload)
+                s.spay[p] = pay[it];
+            else
+                s.svals[p] = v[it];
         }
     }
     __syncthreads();
@@ -502,14 +504,17 @@ __device__ __forceinline__ void block_scatter(const uint32_t (&k)[ITEMS],
         const uint32_t d = digit_of(bf(key), shift, dmask);
         const uint32_t dst = s.global_start[d] + (p - s.local_start[d]);
         if (dst < (uint64_t)n) {  // always true for a consistent histogram; guards the store
-            const uint32_t val = s.svals[p];
             if (write_keys) keys_out[dst] = (KeyT)key;
-            vals_out[dst] = val;
-            if (kPayload) pay_out[dst] = s.spay[p];
-            if (counts_out || rects_out) {
-                const uint2 r = rect_or_empty(rects, val, n);
-                if (counts_out) counts_out[dst] = rect_supertiles(r);
-                if (rects_out) rects_out[dst] = r;
+            if constexpr (kPayload) {
+                pay_out[dst] = s.spay[p];
+            } else {
+                const uint32_t val = s.svals[p];
+                vals_out[dst] = val;
+                if (counts_out || rects_out) {
+                    const uint2 r = rect_or_empty(rects, val, n);
+                    if (counts_out) counts_out[dst] = rect_supertiles(r);
+                    if (rects_out) rects_out[dst] = r;
+                }
             }
         }
     }
@@ -547,7 +552,7 @@ struct PassExtras {
     bool hist_ready = false;            // the caller wrote this pass's histogram table
     bool drop_no_tiles = false;         // keys equal to kNoTilesKey are not sorted
     const int64_t *n_live = nullptr;    // device: sort only the first *n_live keys
-    const uint2 *pin = nullptr;         // kPayload: 8-byte payload per key
+    const uint2 *pin = nullptr;         // kPayload: the values (vin and vout are unused)
     uint2 *pout = nullptr;
     const uint2 *rects = nullptr;       // gathered by value (last pass):
     uint64_t *counts_out = nullptr;     //   rect_supertiles(rects[value])
@@ -600,7 +605,7 @@ __global__ __launch_bounds__(kSortThreads) void radix_downsweep_kernel(DownArgs<
         const int64_t i = base + slot_index<ITEMS>(it);
         const bool in = i < live;
         k[it] = in ? (uint32_t)a.keys_in[i] : 0u;
-        v[it] = in ? (a.vals_in ? a.vals_in[i] : (uint32_t)i) : 0u;
+        v[it] = !kPayload && in ? (a.vals_in ? a.vals_in[i] : (uint32_t)i) : 0u;
         pay[it] = (kPayload && in) ? a.pay_in[i] : make_uint2(0u, 0u);
         valid[it] = in && !(a.drop_no_tiles && k[it] == kNoTilesKey);
         k[it] = valid[it] ? k[it] : 0u;
@@ -609,7 +614,7 @@ __global__ __launch_bounds__(kSortThreads) void radix_downsweep_kernel(DownArgs<
                                          a.keys_out, a.vals_out, a.pay_out, a.n,
                                          a.write_keys != 0, s, a.totals, a.counts_out, a.rects,
                                          a.rects_out, blk, bf);
-    if (a.n_live && !a.write_keys) {
+    if (!kPayload && a.n_live && !a.write_keys) {
         for (int t = threadIdx.x; t < kSortThreads * ITEMS; t += kSortThreads) {
             const int64_t j = base + t;
             if (j < live || j >= a.n) continue;
@@ -1872,8 +1877,7 @@ template <typename KeyT>
 __global__ __launch_bounds__(256) void emit_super_kernel(
     int64_t n, int64_t m, const uint32_t *__restrict__ order,
     const uint64_t *__restrict__ offsets, const uint2 *__restrict__ rects, int super_x,
-    KeyT *__restrict__ keys_out, uint32_t *__restrict__ vals_out,
-    uint2 *__restrict__ entries_out) {
+    KeyT *__restrict__ keys_out, uint2 *__restrict__ entries_out) {
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= n) return;
     const uint32_t g = order[r];
@@ -1886,7 +1890,6 @@ __global__ __launch_bounds__(256) void emit_super_kernel(
         for (int x = t.tx0 / kSuper; x <= t.tx1 / kSuper; ++x, ++o) {
             if (o >= m) return;
             keys_out[o] = (KeyT)(y * super_x + x);
-            vals_out[o] = g;
             entries_out[o] = super_entry(g, t, x, y);
         }
 }
@@ -2157,8 +2160,7 @@ inline bool use_u16_keys(int tile_bits) { return tile_bits <= 16; }
 // Level 1: the (supertile, Gaussian) entries and their sort by supertile.
 struct SortWs {
     void *keys_a, *keys_b;  // supertile keys (u16 or u32)
-    uint32_t *vals_a, *vals_b;
-    uint2 *entries_tmp;     // the entries (payload of the sort)
+    uint2 *entries_tmp;     // the entries (the values of the sort)
     void *pass_ws;  // histogram table + digit totals of each pass
     size_t bytes;
 };
@@ -2168,8 +2170,6 @@ inline SortWs carve_sort(Carve &c, int64_t m, int super_bits) {
     const int64_t kb = use_u16_keys(super_bits) ? 2 : 4;
     w.keys_a = c.take<char>(m * kb);
     w.keys_b = c.take<char>(m * kb);
-    w.vals_a = c.take<uint32_t>(m);
-    w.vals_b = c.take<uint32_t>(m);
     w.entries_tmp = c.take<uint2>(m);
     w.pass_ws = c.take<char>((int64_t)radix_workspace_bytes<kTileItems>(m));
     w.bytes = 0;
@@ -2245,22 +2245,21 @@ int super_sort(const EmitArgs &a, const SortWs &w, int super_bits, int n_super,
     const SortPlan plan = plan_sort(super_bits);
     const int P = plan.passes;
     KeyT *ka = reinterpret_cast<KeyT *>(w.keys_a), *kb = reinterpret_cast<KeyT *>(w.keys_b);
-    // pass p writes (kb, vals_b, super_entries) when P-1-p is even, (ka, vals_a,
-    // entries_tmp) otherwise; the entries (pass -1) go to the other set than pass 0.
+    // pass p writes (kb, super_entries) when P-1-p is even, (ka, entries_tmp)
+    // otherwise; the entries (pass -1) go to the other set than pass 0.
     auto keys_for = [&](int p) { return ((P - 1 - p) % 2 == 0) ? kb : ka; };
-    auto vals_for = [&](int p) { return ((P - 1 - p) % 2 == 0) ? w.vals_b : w.vals_a; };
     auto entries_for = [&](int p) { return ((P - 1 - p) % 2 == 0) ? super_entries : w.entries_tmp; };
     hipLaunchKernelGGL(emit_super_kernel<KeyT>, dim3(ceil_div(a.n, 256)), dim3(256), 0, stream,
                        a.n, a.k, a.order, a.offsets, a.rects, a.tiles_x, keys_for(-1),
-                       vals_for(-1), entries_for(-1));
+                       entries_for(-1));
     int st = launch_status();
     if (st) return st;
     for (int p = 0; p < P; ++p) {
         PassExtras x;
         x.pin = entries_for(p - 1);
         x.pout = entries_for(p);
-        st = radix_pass<KeyT, kTileItems, true>(keys_for(p - 1), vals_for(p - 1), keys_for(p),
-                                                vals_for(p), a.k, p * plan.bits_per_pass,
+        st = radix_pass<KeyT, kTileItems, true>(keys_for(p - 1), nullptr, keys_for(p), nullptr,
+                                                a.k, p * plan.bits_per_pass,
                                                 pass_bits(plan, super_bits, p), true, w.pass_ws,
                                                 stream, x);
         if (st) return st;

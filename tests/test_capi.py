@@ -71,6 +71,11 @@ def test_workspace_queries(lib):
     assert lib.gs_bin_sort_workspace_size(1000, 20_000_000, 1_000_000, 1920, 1080, 16,
                                           ctypes.byref(sz)) == 0
     assert 1_000_000 * 8.5 <= sz.value < 1_000_000 * 8.7
+    # more than 256 supertiles: a sort's two 16-bit key buffers, a second buffer of entries
+    # and 256 counters per 1024 entries on top, and no ids of their own
+    assert lib.gs_bin_sort_workspace_size(1000, 20_000_000, 1_000_000, 3840, 2160, 16,
+                                          ctypes.byref(sz)) == 0
+    assert 1_000_000 * 21.5 <= sz.value < 1_000_000 * 22
     assert lib.gs_bin_sort_workspace_size(1000, 20_000_000, 1_000_000, 1920, 0, 16,
                                           ctypes.byref(sz)) == -1
     assert lib.gs_bin_count_workspace_size(-1, ctypes.byref(sz)) == -1
