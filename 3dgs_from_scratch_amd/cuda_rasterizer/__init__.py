@@ -705,18 +705,45 @@ def _backward_rows(stage, seed, grad, blend, width, height, tile_size, alpha_thr
     _lib.timer.stop(ev, dev)
 
 
-def _backward_split(*args, **kw):
-    """_backward_rows into zeroed rows, then the four gradients (N,2), (N,3), (N,), (N,3),
-    carved from one buffer.  The rows' atomics are much cheaper than the four arrays'
-    and their copy costs a few microseconds: 72 MB moved at 1M Gaussians."""
-    blend = args[3]
-    dev, n = blend[0], blend[1]
+# Lists of at most this many entries add their gradients straight into the four arrays:
+# up to about 100k entries the call is as long as its host work, and the rows' copy is a
+# launch and an allocation more (27 against 21 us at 184 to 39k entries, 35 against 30 at
+# 90k); above, the rows' cheaper atomics decide (68 against 80 us at 304k, 157 against 205
+# at 911k).
+_FOUR_ARRAYS_KEYS = 1 << 17
+
+
+def _backward_split(stage, seed, grad, blend, width, height, tile_size, alpha_threshold,
+                    transmittance_threshold, chi_squared_threshold, image, grad_loss=None,
+                    loss_scale=0.0, extra=None, schedule=None):
+    """The four gradients (N,2), (N,3), (N,), (N,3), carved from one buffer: the blend's
+    sums in it, or, for lists of more than _FOUR_ARRAYS_KEYS entries, in zeroed rows
+    (_backward_rows) that are then copied (72 MB moved at 1M Gaussians).  L1 only as rows."""
+    dev, n, off, ids, pts, conic, opac, col = blend
     with _on(dev):
-        rows = torch.zeros((9 * n,), dtype=torch.float32, device=dev)
-        _backward_rows(*args, rows=rows, **kw)
-        out = _blend_grad_views(torch.empty_like(rows), n)
-        _lib.check(_lib.load().gs_split_gradient_rows(_ptr(rows), n, *(_ptr(t) for t in out),
-                                                      _stream(dev)), args[0])
+        buf = torch.zeros((9 * n,), dtype=torch.float32, device=dev)
+        if seed != _SEED_L1 and ids.shape[0] <= _FOUR_ARRAYS_KEYS:
+            out = _blend_grad_views(buf, n)
+            args = (_ptr(grad), _ptr(image), _ptr(off), _ptr(ids), off.shape[0], ids.shape[0],
+                    _ptr(pts), _ptr(conic), _ptr(opac), _ptr(col), n, width, height,
+                    int(tile_size), float(alpha_threshold), float(transmittance_threshold),
+                    float(chi_squared_threshold), *(_ptr(t) for t in out), 1)
+            lib = _lib.load()
+            ev = _lib.timer.record(stage, dev)
+            if seed == _SEED_IMAGE:
+                st = lib.gs_rasterize_backward(*args, _stream(dev))
+            else:
+                st = lib.gs_rasterize_display_backward(*args, _ptr(schedule), _stream(dev))
+            _lib.check(st, stage)
+            _lib.timer.stop(ev, dev)
+            return out
+        _backward_rows(stage, seed, grad, blend, width, height, tile_size, alpha_threshold,
+                       transmittance_threshold, chi_squared_threshold, image, buf,
+                       grad_loss=grad_loss, loss_scale=loss_scale, extra=extra,
+                       schedule=schedule)
+        out = _blend_grad_views(torch.empty_like(buf), n)
+        _lib.check(_lib.load().gs_split_gradient_rows(_ptr(buf), n, *(_ptr(t) for t in out),
+                                                      _stream(dev)), stage)
     return out
 
 
@@ -1357,6 +1384,8 @@ def rasterize_l1_backward(target, grad_loss, indexing_offset, gaussian_ids_sorte
         opacities, colors, width, height, rendered_image, grad_display01, schedule)
     dev, n, off, ids, pts, conic, opac, col = blend
     width, height = int(width), int(height)
+    if accumulators is None and ids.shape[0] <= _FOUR_ARRAYS_KEYS:
+        accumulators = torch.zeros((9 * n,), dtype=torch.float32, device=dev)
     if accumulators is None:
         return _backward_split("rasterize_l1_backward", _SEED_L1, target, blend, width, height,
                                16, alpha_threshold, transmittance_threshold,

@@ -82,6 +82,38 @@ SCENES = {
 }
 
 
+@pytest.fixture(params=[0, 1 << 62])
+def four_arrays(request, monkeypatch):
+    """The gradients summed in rows and copied, or in the four arrays, whatever the lists."""
+    monkeypatch.setattr(cr, "_FOUR_ARRAYS_KEYS", request.param)
+
+
+@pytest.mark.parametrize("name", list(SCENES))
+def test_gradient_routes(gpu, name, four_arrays):
+    """Every seed of the backward by either route: the oracle's gradients (as
+    test_rasterize_shared_inputs), and for display and L1 the sums of the other entries."""
+    leaves, off, ids, cam, target = _shared_inputs(SCENES[name]())
+    W, H = cam["width"], cam["height"]
+    args = (W, H, 16, 1e-4, 1e-4, 9.21)
+    ins = [leaves[k].clone().requires_grad_(True) for k in INPUTS]
+    ref = blend.rasterize(off, ids, *ins, *args)
+    up = torch.randn(H, W, 3, generator=torch.Generator().manual_seed(9))
+    (ref.clamp(0, 1) * 255 * up).sum().backward()
+    d = [off.to(gpu), ids.to(gpu)] + [leaves[k].to(gpu) for k in INPUTS]
+    image = cr.rasterize(*d, *args)
+    inner = ((image >= 0) & (image <= 1)).float() * 255  # the clamp's gradient
+    up = up.to(gpu)
+    for got in (cr.rasterize_backward(up * inner, *d, *args, rendered_image=image),
+                cr.rasterize_display_backward(up, *d, *args, rendered_image=image)):
+        for nm, a, t in zip(INPUTS, got, ins):
+            assert a.is_contiguous() and helpers.rel_l2(a, t.grad) <= 1e-3, nm
+    one = torch.ones(1, device=gpu)
+    l1 = cr.rasterize_l1_backward(target.to(gpu), one, *d, W, H, image, 1e-4, 1e-4, 9.21)
+    rows = cr.rasterize_l1_backward_rows(target.to(gpu), one, *d, W, H, image, 1e-4, 1e-4, 9.21)
+    for nm, a, b in zip(INPUTS, l1, (rows[:, :2], rows[:, 2:5], rows[:, 5], rows[:, 6:])):
+        assert a.is_contiguous() and helpers.rel_l2(a, b) <= 1e-5, nm
+
+
 @pytest.mark.parametrize("name", list(SCENES))
 def test_rasterize_shared_inputs(gpu, name, waves):
     leaves, off, ids, cam, target = _shared_inputs(SCENES[name]())
