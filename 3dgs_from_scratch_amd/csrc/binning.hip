@@ -684,8 +684,8 @@ int radix_pass(const KeyT *kin, const uint32_t *vin, KeyT *kout, uint32_t *vout,
     }
     const int sums_block = x.block_sums ? 1 : 0;
     hipLaunchKernelGGL(digit_scan_kernel, dim3((1 << nbits) + sums_block), dim3(kScanThreads), 0,
-                       stream, hist, nullptr, nblocks, totals, x.block_sums, x.block_minmax, nblocks,
-                       x.sums_out, x.live_out, x.sums_dev);
+                       stream, hist, nullptr, nblocks, totals, x.block_sums, x.block_minmax,
+                       nblocks, x.sums_out, x.live_out, x.sums_dev);
     st = launch_status();
     if (st) return st;
     DownArgs<KeyT> a;

@@ -906,7 +906,7 @@ __device__ __forceinline__ float wave_sum(float x) {
 // Sums of nine per-lane values over each row of 16 lanes, by transposition: the
 // first two steps fold lane l with l + 8 and the halves of 8 lanes, each keeping
 // one field in the low and another in the high lanes (the masked DPP adds write
-// only their banks of 4 lanes); two butterflies within the quads finish.  22 DPP
+// only their banks of 4 lanes); two butterflies within the quads finish.  20 DPP
 // adds for nine sums in four rows at once.  Bank b of q0 holds field (0, 2, 1, 3)[b],
 // of q1 field (4, 6, 5, 7)[b], every lane of q2 field 8.  All lanes must be active.
 // One asm block: every DPP source is written at least two instructions before it
@@ -1370,7 +1370,8 @@ enum { kSeedImage = 0, kSeedDisplay = 1, kSeedL1 = 2 };
         int64_t k, int64_t n, const float *__restrict__ points,                               \
         const float *__restrict__ conics, const float *__restrict__ opac,                     \
         const float *__restrict__ colors, int tiles_x, int width, int height, float alpha_thr, \
-        float T_thr_in, float chi, GradOut out, const float *__restrict__ grad_loss, float inv_count, const float *__restrict__ extra
+        float T_thr_in, float chi, GradOut out, const float *__restrict__ grad_loss,          \
+        float inv_count, const float *__restrict__ extra
 
 // The backward walk of `tile`'s list, or (seg >= 0) of its segment seg: from the
 // start to checkpoint 0, between checkpoints seg - 1 and seg, or from the last
@@ -1711,7 +1712,9 @@ static int check_blend_args(const int32_t *indexing_offset, const int32_t *ids, 
 // Forward, us, 1 / 2 / 4 waves (entry by entry with one wave, in groups with more):
 //   192 tiles (20k Gaussians) 176 / 70 / 45, 256 tiles 99 / 43 / 29, 2170 tiles
 //   155 / 96 / 77, 3600 tiles 147 / 102 / 87, 6700 tiles 120 / 107 / 109, 8160 tiles
-//   138 / 122 / 127 (3M Gaussians 149 / 121 / 126), 32400 tiles 355 / 380 / 440.
+//   138 / 122 / 127 (3M Gaussians 149 / 121 / 126), 12750 tiles 178 / 169 / 183,
+//   16320 tiles 208 / 205 / 225, 18360 tiles 225 / 225 / 250, 22600 tiles
+//   260 / 263 / 296, 32400 tiles 345 / 364 / 416 (2M Gaussians: within 3% of these).
 // So 4 up to kCheckpointMaxTiles tiles, 2 up to kTwoWaveTiles and 1 above, where the
 // chip is full and only the instructions count.  Backward, us, 1 / 2 / 4 waves, from
 // the same checkpoints: 192 tiles 109 / 67 / 46, 256 tiles 54 / 39 / 30, 2170 tiles

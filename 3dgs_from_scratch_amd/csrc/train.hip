@@ -51,7 +51,8 @@ __global__ __launch_bounds__(kTrainBlock) void adam_kernel(AdamBatch batch, floa
 //   grads += |(du * W/2, dv * H/2)|, count += 1.
 __global__ __launch_bounds__(kTrainBlock) void accumulate_grad2d_kernel(
     int64_t n, const float *__restrict__ grad_points, int stride,
-    const float *__restrict__ radii, float half_w, float half_h, float *__restrict__ grads, float *__restrict__ count) {
+    const float *__restrict__ radii, float half_w, float half_h, float *__restrict__ grads,
+    float *__restrict__ count) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     if (!(radii[2 * i] > 0.0f && radii[2 * i + 1] > 0.0f)) return;

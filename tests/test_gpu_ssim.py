@@ -62,14 +62,11 @@ def test_ssim_matches_oracle(gpu, shape, padding):
 # rows: 23-row units; 4000 strips: one unit of 34 rows each; 4300: more units than
 # the waves of 1024 workgroups, so some take two.
 @pytest.mark.parametrize("shape", [(1, 1, 12, 64), (1, 2, 13, 65), (100, 3, 130, 64),
-                                   (1000, 4, 25, 7), (2150, 2, 13, 6)])
+                                   (1000, 4, 25, 11), (2150, 2, 13, 11)])
 @pytest.mark.parametrize("padding", ["same", "valid"])
 def test_unit_heights(gpu, shape, padding):
     a, b = images(shape, seed=sum(shape))
     val, grad = run(a.to(gpu), b.to(gpu), padding, grad_out=0.37)
-    if padding == "valid" and (shape[2] <= 10 or shape[3] <= 10):
-        assert torch.isnan(val)  # no pixel at least 5 from the border
-        return
     check_against_oracle(a, b, padding, val, grad, grad_out=0.37)
 
 

@@ -4,10 +4,10 @@ the C ABI.
 It runs gs_ssim_forward's kernels with the per-workgroup partials in a static
 device array instead of a caller workspace, so its outputs -- the mean, the
 three derivative maps and the combined loss -- must equal gs_ssim_forward's bit
-for bit (the mean is reduced in a fixed order).  Checked on two calls in a row,
-each with a smaller input than the one before (the array then still holds
-the earlier call's partials past the later call's workgroup count), in both
-orders of the two entry points, and its argument checks.
+for bit (the mean is reduced in a fixed order).  Checked on calls in a row,
+each with fewer workgroups than the one before (the array then still holds
+the earlier call's partials past the later call's count; the first fills all
+1024), in both orders of the two entry points, and its argument checks.
 """
 
 from __future__ import annotations
@@ -65,13 +65,14 @@ def _inputs(shape_hwc, seed, permuted, gpu):
             y.permute(2, 0, 1).contiguous().unsqueeze(0).to(gpu))
 
 
-# Units of 64 columns per plane, 4 per workgroup, at most 1024 workgroups (the
-# static array's size).  2160x3840x3: 60 x 17 x 3 = 3060 units of 133 output rows,
-# 765 workgroups; then 720x1280x3: 20 x 32 x 3 = 1920 units of 23 rows, 480
-# workgroups; then 32x96x3: 2 x 3 x 3 = 18 units of 12 rows, 5 workgroups (every
+# Units of 64 columns per plane, 4 per workgroup, at most 1024 workgroups (the static
+# array's size).  13x11x4300: 4300 units of 23 output rows, 1075 workgroups capped at 1024,
+# so the array is filled to capacity (and some waves take two units); then 2160x3840x3:
+# 60 x 17 x 3 = 3060 units of 133 rows, 765 workgroups; 720x1280x3: 20 x 32 x 3 = 1920 units
+# of 23 rows, 480 workgroups; 32x96x3: 2 x 3 x 3 = 18 units of 12 rows, 5 workgroups (every
 # partial past the fifth still holds an earlier call's value)
-CALLS = [((2160, 3840, 3), 4, True, 0, 255.0), ((720, 1280, 3), 1, True, 1, 255.0),
-         ((32, 96, 3), 2, False, 0, 255.0)]
+CALLS = [((13, 11, 4300), 5, False, 0, 255.0), ((2160, 3840, 3), 4, True, 0, 255.0),
+         ((720, 1280, 3), 1, True, 1, 255.0), ((32, 96, 3), 2, False, 0, 255.0)]
 
 
 @pytest.mark.parametrize("noalloc_first", [True, False])
