@@ -26,7 +26,7 @@
 // backward, which filters them back the same way.  The mean is reduced
 // deterministically: per-workgroup double partials, then one workgroup.
 //
-// What bounds it: the issue of vector instructions (the forward 140 a row and
+// What bounds it: the issue of vector instructions (the forward 130 a row and
 // wave, 88 of them FMAs by a tap) together with the LDS (11 reads of 16 bytes),
 // at 3 waves a SIMD; the backward of a large image the memory (2 x 3 x 1063 x
 // 1599: 246 MB in 65 us, 3.8 TB/s).  Measured in us, forward / backward, with
@@ -289,7 +289,7 @@ __device__ __forceinline__ void taps_ready(f4v (&v)[kTaps]) {
 
 // The window's taps in vector registers (they are symmetric: 6 of them).  An
 // FMA that reads a scalar register takes 4.3 cycles of a SIMD on gfx950, one
-// that reads only vector registers 2.5; of the forward's 140 vector
+// that reads only vector registers 2.5; of the forward's 130 vector
 // instructions a row 88 multiply by a tap.
 __device__ __forceinline__ void taps_to_vector(Window &win) {
 #pragma unroll
