@@ -45,7 +45,10 @@ def _collector_held():
     thread).  A step that a cycle of references holds -- its function refers to
     the object that owns it -- is freed by the collector; if that happens while
     another step records, the dead graph's destructor makes a HIP call that a
-    capture forbids, and the process ends."""
+    capture forbids, and the process ends; so does a pending CappedCheck, which
+    waits for an event.  The collector's state is the process's: a gc.disable()
+    that another thread calls during a capture (some milliseconds) is undone when
+    the last capture ends."""
     with _hold_lock:
         if _holds[0] == 0:
             _holds[1] = gc.isenabled()
